@@ -68,12 +68,14 @@ const void* grid_batch(stp_ctx* ctx, const std::vector<BatchGridItem>& items, co
 // context stream; grid_batch_tiles launches the tile and total kernels on the
 // context stream, which must by then be ordered after the binning.
 struct BatchPlan {
-    static constexpr int CLASSES = 6;  // kernel width (8 or 16 taps) x tile width (16, 32, 64)
+    static constexpr int CLASSES = 6;  // tile width (16, 32, 64); two-float: x kernel width (8 or 16 taps)
     const void* d_tab = nullptr;       // device tables (snapshot records first)
     const void* d_extra = nullptr;     // the caller's tables
     int items = 0;
     bool twofloat = false;
     size_t pre_t_off = 0;              // byte offset of the tile-class prefixes in d_tab
+    size_t pre_m_off = 0;              // byte offset of the merge prefix in d_tab
+    size_t merges = 0;                 // merge workgroups of split tiles
     size_t tiles[CLASSES] = {};
     size_t tile_lds[CLASSES] = {};
 };

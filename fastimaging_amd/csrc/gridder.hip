@@ -1,5 +1,5 @@
 // Convolutional gridding for gfx950: the scatter-add of convolve_to_grid
-// (src/stp/gridder/gridder.h:240-997) as a tile-binned, LDS-accumulated gather.
+// (src/stp/gridder/gridder.h:240-997) as a tile-binned gather.
 //
 //  1. grid_count   : per visibility, the reference's pre-processing (half-plane
 //                    conversion gridder.cpp:11-37, rint centre/fraction
@@ -9,9 +9,9 @@
 //                    sums the good weights in the canonical order.
 //  2. tile_scan    : exclusive scan of the per-tile counts.
 //  3. grid_scatter : writes one 40-byte entry per (pass, tile) pair, binned by tile.
-//  4. grid_tiles   : one workgroup per TILE_R x TILE_C tile accumulates every
-//                    entry's taps that fall inside it in LDS (ds_add_f64), then
-//                    writes the whole tile once: no global atomics, no memset.
+//  4. grid_tiles   : one workgroup per TILE_R x TILE_C tile sums every entry's
+//                    taps that fall inside it on the FP64 matrix cores, then
+//                    writes the whole tile once: no atomics, no memset.
 // Per tap the arithmetic is the reference's: kval = K * w, grid += vis * kval,
 // beam += kval (gridder.h:854-858); the oversampled kernel is the separable
 // product ky[row] * kx[col] of normalised 1-D kernels (gridder.h:84-102).
@@ -340,25 +340,6 @@ __global__ __launch_bounds__(GWG) void grid_count_kernel(GridGeom g, const doubl
     }
 }
 
-__global__ __launch_bounds__(GWG) void grid_scatter_kernel(GridGeom g, const double* uv, const double* vis,
-    const double* wts, uint32_t* cursor, Entry* entries, uint32_t cap)
-{
-    const long long i = (long long)blockIdx.x * GWG + threadIdx.x;
-    if (i >= g.n)
-        return;
-    const Prep p = prep_vis(g, uv, vis, wts, i);
-    if (!p.good)
-        return;
-    for (int pass = 0; pass <= p.dup; pass++) {
-        const Entry e = make_entry(g, p, pass, i);
-        visit_tiles(g, e.gx, e.gy, [&](int ct, int rt) {
-            const uint32_t slot = atomicAdd(&cursor[ct * g.tiles_r + rt], 1u);
-            if (slot < cap)
-                entries[slot] = e;
-        });
-    }
-}
-
 // Kernel functors on the device (exact gridding only; conv_func.cpp:10-202).
 // Spheroidal function of the PSWF functor (conv_func.cpp:112-182): F. Schwab's
 // rational approximation (Indirect Imaging, 1984), M = 6, alpha = 1; the same
@@ -372,12 +353,16 @@ __device__ double dev_spheroidal(double nu)
     nu = fabs(nu);
     const bool part = nu >= 0.75 && nu <= 1.0;
     const double nuend = (nu >= 0.0 && nu < 0.75) ? 0.75 : ((nu <= 1.0) ? 1.0 : 0.0);
-    const double d = pow(nu, 2.0) - pow(nuend, 2.0);
+    const double d = nu * nu - nuend * nuend;
     double top = part ? p1[0] : p0[0], bot = part ? q1[0] : q0[0];
-    for (int k = 1; k < 5; k++)
-        top += (part ? p1[k] : p0[k]) * pow(d, double(k));
-    for (int k = 1; k < 3; k++)
-        bot += (part ? q1[k] : q0[k]) * pow(d, double(k));
+    double dk = d; // powers by products: a library pow() per term cost most of the exact path
+#pragma unroll
+    for (int k = 1; k < 5; k++) {
+        top += (part ? p1[k] : p0[k]) * dk;
+        if (k < 3)
+            bot += (part ? q1[k] : q0[k]) * dk;
+        dk *= d;
+    }
     return bot > 0.0 ? top / bot : 0.0;
 }
 
@@ -401,7 +386,7 @@ __device__ double dev_kernel(const GridGeom& g, double r)
         break;
     case STP_KERNEL_PSWF: { // conv_func.cpp:185-196
         const double nu = r / g.kparam;
-        v = dev_spheroidal(nu) * (1.0 - pow(nu, 2.0));
+        v = dev_spheroidal(nu) * (1.0 - nu * nu);
         break;
     }
     default: { // GaussianSinc
@@ -417,21 +402,22 @@ __device__ double dev_kernel(const GridGeom& g, double r)
     return v;
 }
 
-// Last canonical level of the (good weights, good count) block pairs: the sampling
-// grid total 2 * sum(weights) and the good count.
-// Also copies the number of gridding entries (the end of the last tile's range).
-__global__ __launch_bounds__(CANON_LANES) void grid_total_kernel(const double* part, unsigned m, double* total,
-    unsigned long long* ngood, const uint32_t* entries_end, unsigned long long* nentries)
+__global__ __launch_bounds__(GWG) void grid_scatter_kernel(GridGeom g, const double* uv, const double* vis,
+    const double* wts, uint32_t* cursor, Entry* entries, uint32_t cap)
 {
-    __shared__ double lds[2 * CANON_LANES];
-    double a, b;
-    canon_last_level(part, m, a, b, lds);
-    if (threadIdx.x == 0) {
-        total[0] = a * 2.0;
-        if (ngood)
-            *ngood = (unsigned long long)b;
-        if (nentries)
-            *nentries = *entries_end;
+    const long long i = (long long)blockIdx.x * GWG + threadIdx.x;
+    if (i >= g.n)
+        return;
+    const Prep p = prep_vis(g, uv, vis, wts, i);
+    if (!p.good)
+        return;
+    for (int pass = 0; pass <= p.dup; pass++) {
+        const Entry e = make_entry(g, p, pass, i);
+        visit_tiles(g, e.gx, e.gy, [&](int ct, int rt) {
+            const uint32_t slot = atomicAdd(&cursor[ct * g.tiles_r + rt], 1u);
+            if (slot < cap)
+                entries[slot] = e;
+        });
     }
 }
 
@@ -610,11 +596,111 @@ __device__ uint32_t scan_tile_totals(const uint32_t* totals, int ntiles, uint32_
     return total;
 }
 
+// Splitting of heavy tiles.  Interferometers crowd the origin of the uv plane, so a
+// few tiles can hold most of the entries, and one workgroup per tile then leaves the
+// rest of the chip idle.  A tile of more than ch entries is summed in chunks of ch by
+// several workgroups: chunk 0 by the tile's own, chunks 1.. by extra workgroups.  Every
+// chunk of a split tile stores its FP64 sums in a slot, and merge workgroups add the
+// slots in chunk order.  ch = max(SPLIT_MIN, entries / ext_max), so at most ext_max
+// extra chunks, as many split tiles and 2 ext_max slots exist.  Below SPLIT_MIN entries
+// a tile's sums take less than a merge costs; SPLIT_EXTRA_MAX gives every CU two chunks.
+//
+// The plan and the slots lie in the unused end of the entry buffer, which is sized for
+// the most tiles that footprints can touch (eight entries for each visibility at 7 x 7
+// taps; 1.2 to 1.6 are used): every kernel derives the same view from the entry count,
+// and where the end is short there are fewer chunks or none.
+constexpr uint32_t SPLIT_MIN = 1024;
+constexpr size_t SPLIT_EXTRA_MAX = 512;
+constexpr size_t SPLIT_PLAN_BYTES = 16384;
+static_assert(256 + SPLIT_EXTRA_MAX * 20 <= SPLIT_PLAN_BYTES, "plan layout");
+struct Split {
+    uint32_t* hdr;     // extra chunks, split tiles, ch (null: no splitting)
+    uint32_t* ext;     // per extra chunk: tile, chunk
+    uint32_t* spl;     // per split tile (in tile order): tile, first slot, chunks
+    double* part;      // slots of 3 x tile columns x TILE_R sums
+    size_t room;       // bytes for slots
+};
+
+inline int split_extra_max(size_t n) { return int(std::min(SPLIT_EXTRA_MAX, n / SPLIT_MIN)); }
+// Merge workgroups (four tile columns each).
+inline size_t merge_blocks(int ext_host, int tc) { return size_t(ext_host) * (tc / 4); }
+
+__device__ __forceinline__ Split split_view(Entry* entries, uint32_t cap, uint32_t nent, int ext_host, int tc)
+{
+    Split sp{ nullptr, nullptr, nullptr, nullptr, 0 };
+    const size_t used = (size_t(nent) * sizeof(Entry) + 255) & ~size_t(255);
+    const size_t room = size_t(cap) * sizeof(Entry), slot = size_t(3) * tc * TILE_R * sizeof(double);
+    if (ext_host <= 0 || room < used + SPLIT_PLAN_BYTES + 2 * slot)
+        return sp;
+    sp.room = room - used - SPLIT_PLAN_BYTES;
+    uint8_t* base = reinterpret_cast<uint8_t*>(entries) + used;
+    sp.hdr = reinterpret_cast<uint32_t*>(base);
+    sp.ext = sp.hdr + 64;
+    sp.spl = sp.ext + 2 * SPLIT_EXTRA_MAX;
+    sp.part = reinterpret_cast<double*>(base + SPLIT_PLAN_BYTES);
+    return sp;
+}
+
+// The plan from the tile totals, by one workgroup of BWG threads.
+__device__ void split_plan(const Split& sp, const uint32_t* totals, int ntiles, uint32_t total, int ext_host, int tc,
+    uint32_t* wsum)
+{
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const size_t slot = size_t(3) * tc * TILE_R * sizeof(double);
+    const uint32_t ext_max = uint32_t(min(size_t(ext_host), sp.room / (2 * slot)));
+    const uint32_t ch = max(SPLIT_MIN, (total + ext_max - 1) / ext_max);
+    const int per = (ntiles + BWG - 1) / BWG;
+    const int i0 = min(ntiles, tid * per), i1 = min(ntiles, i0 + per);
+    uint32_t s = 0; // extra chunks | split tiles << 16
+    for (int t = i0; t < i1; t++) {
+        const uint32_t c = totals[t];
+        if (c > ch)
+            s += (c - 1) / ch + (1u << 16);
+    }
+    uint32_t x = s;
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t y = __shfl_up(x, off, 64);
+        if (lane >= off)
+            x += y;
+    }
+    __syncthreads();
+    if (lane == 63)
+        wsum[w] = x;
+    __syncthreads();
+    uint32_t sum = 0;
+    for (int k = 0; k < BWG / 64; k++) {
+        sum += wsum[k];
+        if (k < w)
+            x += wsum[k];
+    }
+    uint32_t e = (x - s) & 0xffffu, i = (x - s) >> 16;
+    for (int t = i0; t < i1; t++) {
+        const uint32_t c = totals[t];
+        if (c <= ch)
+            continue;
+        const uint32_t n = (c - 1) / ch + 1;
+        sp.spl[3 * i] = uint32_t(t);
+        sp.spl[3 * i + 1] = e + i;
+        sp.spl[3 * i + 2] = n;
+        for (uint32_t k = 1; k < n; k++, e++) {
+            sp.ext[2 * e] = uint32_t(t);
+            sp.ext[2 * e + 1] = k;
+        }
+        i++;
+    }
+    if (tid == 0) {
+        sp.hdr[0] = sum & 0xffffu;
+        sp.hdr[1] = sum >> 16;
+        sp.hdr[2] = ch;
+    }
+}
+
 // Block b's entries go to cursors tile offset + block offset; the tile offsets (the
 // scan of the tile totals) are computed by every block in LDS, and block 0 also
-// writes them to tile_off[0..ntiles] for the tile kernel.
+// writes them to tile_off[0..ntiles] for the tile kernel, and the split plan.
 __device__ __forceinline__ void bin_scatter_body(const GridGeom& g, const double* uv, const double* vis, const double* wts,
-    const uint32_t* totals, const uint32_t* block_off, Entry* entries, uint32_t cap, uint32_t* tile_off, int bid)
+    const uint32_t* totals, const uint32_t* block_off, Entry* entries, uint32_t cap, uint32_t* tile_off, int ext_host,
+    int bid)
 {
     extern __shared__ uint32_t cur[];
     __shared__ uint32_t wsum[BWG / 64];
@@ -646,7 +732,7 @@ __device__ __forceinline__ void bin_scatter_body(const GridGeom& g, const double
         const Prep p = prep_in(g, in[j]);
         if (!p.good)
             continue;
-        for (int pass = 0; pass <= p.dup; pass++) {
+            for (int pass = 0; pass <= p.dup; pass++) {
             const Entry e = make_entry(g, p, pass, i);
             visit_tiles(g, e.gx, e.gy, [&](int ct, int rt) {
                 const uint32_t slot = atomicAdd(&cur[ct * g.tiles_r + rt], 1u);
@@ -655,52 +741,490 @@ __device__ __forceinline__ void bin_scatter_body(const GridGeom& g, const double
             });
         }
     }
+    if (bid == 0 && ext_host > 0) {
+        const Split sp = split_view(entries, cap, total, ext_host, g.tc);
+        if (sp.hdr)
+            split_plan(sp, totals, ntiles, total, ext_host, g.tc, wsum);
+    }
 }
 
 __global__ __launch_bounds__(BWG) void grid_bin_scatter_kernel(GridGeom g, const double* uv, const double* vis,
-    const double* wts, const uint32_t* totals, const uint32_t* block_off, Entry* entries, uint32_t cap, uint32_t* tile_off)
+    const double* wts, const uint32_t* totals, const uint32_t* block_off, Entry* entries, uint32_t cap, uint32_t* tile_off,
+    int ext_host)
 {
-    bin_scatter_body(g, uv, vis, wts, totals, block_off, entries, cap, tile_off, int(blockIdx.x));
+    bin_scatter_body(g, uv, vis, wts, totals, block_off, entries, cap, tile_off, ext_host, int(blockIdx.x));
 }
 
 // ---------------------------------------------------------------------------
-// Tile accumulation: one workgroup per TILE_R x TILE_C tile accumulates the taps
-// of every entry binned to it in LDS, then writes the tile once (no global
-// atomics, no memset).  Lane mapping for supports up to 31: a wave takes
-// 64 / ks entries at a time, lane (entry e, kernel column j) walks the ks kernel
-// rows, so one load of kx[j] serves ks taps and the ks LDS atomics of a lane are
-// independent.  Wider kernels take one entry per wave, lanes striding columns.
+// Tile sums on the FP64 matrix cores.  The taps of an entry are the outer product of
+// its kernel row and column values, so the entries that touch a block of 16 x 16 cells
+// sum as a matrix product: v_mfma_f64_16x16x4 adds four entries at once, A = kx times
+// the entry's (vis w) re, (vis w) im or w over the block's columns, B = ky over its rows,
+// both zero outside the footprint.  A wave owns one block (three accumulators of four
+// doubles per lane) and a workgroup the tile's TC / 4 blocks.  The workgroup stages its
+// entries in LDS in batches, a thread for each, which queues the entry's index for the
+// blocks that it touches; each wave then takes its queue four at a time.
+// (Waves that each walked all entries spent more on the walk than on the products: 123 us
+// at 1 M visibilities, N = 4096.)
 //
-// FP64: ds_add_f64 per channel.  FP32 (compensated): each channel keeps an
-// unevaluated pair hi + lo.  The returning atomic add on hi yields the old value,
-// so the rounding error of the sum it stored is known exactly (Knuth's TwoSum on
-// old and x) and is itself added to lo.
+// Bound: FP64 matrix products and vector instructions share their issue (a wave's
+// products and another wave's integer instructions take the sum of their times), so the
+// time is the sum of both: a 7 x 7 footprint touches (22 / 16)^2 = 1.9 blocks, each 3 x 64
+// cycles per four entries plus 17 vector instructions, 57 us for 1 M visibilities at 2.1
+// GHz, and staging.  DPP broadcasts inside rows of 16 lanes hand the entries' values out,
+// since the LDS is nearly as busy with the kernel values.  Measured with N = 4096 and 1 M
+// visibilities: 99 us (uniform uv disk), 150 us (centrally condensed array, FP64) against
+// 144 and 554 us for LDS FP64 atomics, three per tap, the form before; exact PSWF
+// kernels, 300 k visibilities, N = 2048: 146 us against 3500.  The sums stay FP64 on the FP32
+// path too, whose kernel values are no longer rounded to FP32.
+//
+// Heavy tiles are summed in chunks (Split); the chunks of a split tile store their sums
+// in slots that grid_total's merge workgroups add in chunk order.
+typedef double double4v __attribute__((ext_vector_type(4)));
+
+// Where the kernel values come from: the oversampled table in LDS with 15 zeros on both
+// sides of each kernel, so that a block's 16 rows or columns read it without a range
+// check; the plain table, for oversampling factors whose padded table would take the LDS
+// of several workgroups; or exact kernels, evaluated into LDS for each batch.
+enum { KERNEL_PADDED = 0, KERNEL_TABLE = 1, KERNEL_EXACT = 2 };
+constexpr int KV_DOUBLES = 3584;          // kernel table, or exact kernel vectors of a batch (28 KB)
+constexpr int KPAD = 15;
+constexpr int PADDED_DOUBLES = 2560;      // largest padded table (20 KB: four workgroups per CU at 32 columns)
+constexpr int OUT_STRIDE = TILE_R + 4;
+
+inline int table_form(int cs, int ks) { return cs * (ks + 2 * KPAD) <= PADDED_DOUBLES ? KERNEL_PADDED : KERNEL_TABLE; }
+
+struct Staged {
+    double a, b, w;  // (vis w) re, im and w
+    int oy, ox;      // kernel row of the tile's first row and kernel column of its first column as padded
+                     // table indices; other forms: as 16-bit offsets | the kernel's table index << 16
+};
+
+__host__ __device__ constexpr int tile_threads(int tc) { return tc * 16; }
+// Waves per SIMD asked of the register allocator: six keep three 32-column workgroups on
+// a CU (eight spilled: 103 against 101 us at 1 M visibilities); exact kernels need the
+// registers.
+constexpr int tile_waves(int form) { return form == KERNEL_EXACT ? 2 : 6; }
+// Entries staged at a time: one per thread; exact kernels take two threads for each (its
+// row and its column values).
+__host__ __device__ constexpr int tile_batch(int tc, bool exact) { return exact ? tile_threads(tc) / 2 : tile_threads(tc); }
+
+// LDS of a tile workgroup: the kernel table, then the staged entries and the blocks'
+// queues or the tile's sums on their way to memory.
+inline size_t tiles_lds(int tc, int form, int cs, int ks)
+{
+    const size_t table = form == KERNEL_EXACT ? size_t(KV_DOUBLES)
+                                              : size_t(cs) * (form == KERNEL_PADDED ? ks + 2 * KPAD : ks);
+    const size_t batch = tile_batch(tc, form == KERNEL_EXACT);
+    const size_t stage = batch * sizeof(Staged) + batch * (tc / 4 + 1) * sizeof(uint16_t);
+    const size_t out = 2 * size_t(tc) * OUT_STRIDE * sizeof(double);
+    return ((table + 1) & ~size_t(1)) * sizeof(double) + std::max(stage, out);
+}
+
+// Lane R of each row of 16 lanes, to the whole row (DPP row_newbcast: no LDS traffic,
+// which the kernel-value reads need).
+template <int R>
+__device__ __forceinline__ int row_lane(int x)
+{
+    return __builtin_amdgcn_mov_dpp(x, 0x150 + R, 0xf, 0xf, true);
+}
+template <int R>
+__device__ __forceinline__ double row_lane(double x)
+{
+    const long long b = __double_as_longlong(x);
+    const int lo = row_lane<R>(int(b)), hi = row_lane<R>(int(b >> 32));
+    return __longlong_as_double((long long)((unsigned long long)(unsigned)hi << 32 | (unsigned)lo));
+}
+
+// f(integral_constant<int, R>) for R = 0 .. n - 1 (n <= 16, uniform)
+template <int R = 0, typename F>
+__device__ __forceinline__ void for_rows(int n, F f)
+{
+    if constexpr (R < 16) {
+        if (R < n) {
+            f(std::integral_constant<int, R>{});
+            for_rows<R + 1>(n, f);
+        }
+    }
+}
+
+template <typename T, int TC, int FORM>
+__device__ __forceinline__ void tiles_mfma_body(const GridGeom& g, Entry* entries, const uint32_t* offsets, uint32_t cap,
+    const double* ktab, const double* uv, cplx<T>* vgrid, cplx<T>* bgrid, int ext_host, int bid)
+{
+#pragma clang fp contract(off)
+    constexpr int NTH = tile_threads(TC), NB = TC / 4; // threads, blocks (one per wave)
+    constexpr int QCAP = tile_batch(TC, FORM == KERNEL_EXACT);
+    extern __shared__ __align__(16) double dyn[];
+    __shared__ int qcnt[NB];
+    __shared__ int oddcnt[2];
+    const int ks = g.ks, s = g.s, N = g.N;
+    const int cs = (g.os / 2) * 2 + 1;
+    const int ntiles = g.tiles_r * g.tiles_c;
+    const Split sp = split_view(entries, cap, offsets[ntiles], ext_host, TC);
+    uint32_t chunk = 0;
+    int t = bid - ext_host;
+    if (t < 0) {
+        // an extra chunk of a split tile
+        if (!sp.hdr || uint32_t(bid) >= sp.hdr[0])
+            return;
+        t = int(sp.ext[2 * bid]);
+        chunk = sp.ext[2 * bid + 1];
+    }
+    uint32_t eb = min(offsets[t], cap), ee = min(offsets[t + 1], cap);
+    const uint32_t ch = sp.hdr ? sp.hdr[2] : 0xffffffffu;
+    const bool split = ee - eb > ch;
+    if (split) {
+        const uint32_t e0 = eb + chunk * ch;
+        ee = min(ee, e0 + ch);
+        eb = e0;
+    }
+    const int rt = t % g.tiles_r, ct = t / g.tiles_r;
+    const int r0 = rt * TILE_R, c0 = ct * TC;
+    const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int pitch = FORM == KERNEL_PADDED ? ks + 2 * KPAD : ks;
+    double* kt = dyn;
+    double* area = dyn + (FORM == KERNEL_EXACT ? KV_DOUBLES : ((cs * pitch + 1) & ~1));
+    Staged* staged = reinterpret_cast<Staged*>(area);
+    uint16_t* queues = reinterpret_cast<uint16_t*>(staged + QCAP);
+    uint16_t* oddq = queues + NB * QCAP;
+    const int br = 16 * (wave & 3), bc = 16 * (wave >> 2); // the wave's block inside the tile
+    const int m = lane & 15, kk = lane >> 4;
+    double4v ar = { 0, 0, 0, 0 }, ai = { 0, 0, 0, 0 }, ab = { 0, 0, 0, 0 };
+
+    // kernel value i of an entry whose values start at kt[base], zero outside the kernel
+    auto checked = [&](int base, int i) -> double { return unsigned(i) < unsigned(ks) ? kt[base + i] : 0.0; };
+    // row (column) value m of the wave's block for staged entry q with offsets o
+    auto block_value = [&](int q, int o, int at, int axis) -> double {
+        if constexpr (FORM == KERNEL_PADDED)
+            return kt[o + at + m];
+        else
+            return checked(FORM == KERNEL_TABLE ? int(uint32_t(o) >> 16) : (q * 2 + axis) * ks, int(short(o & 0xffff)) + at + m);
+    };
+
+    if (eb < ee) {
+        if constexpr (FORM == KERNEL_PADDED) {
+            for (int k = threadIdx.x; k < cs * pitch; k += NTH) {
+                const int c = k / pitch, i = k - c * pitch - KPAD;
+                kt[k] = unsigned(i) < unsigned(ks) ? ktab[c * ks + i] : 0.0;
+            }
+        } else if constexpr (FORM == KERNEL_TABLE) {
+            for (int k = threadIdx.x; k < cs * ks; k += NTH)
+                kt[k] = ktab[k];
+        }
+        if (threadIdx.x < NB)
+            qcnt[threadIdx.x] = 0;
+        if (threadIdx.x < 2)
+            oddcnt[threadIdx.x] = 0;
+        const int batch = FORM == KERNEL_EXACT ? min(QCAP, KV_DOUBLES / (2 * ks)) : QCAP;
+        // exact kernels: thread k + QCAP evaluates the columns of thread k's entry
+        const int slot = FORM == KERNEL_EXACT ? int(threadIdx.x) % QCAP : int(threadIdx.x);
+        const bool lead = FORM != KERNEL_EXACT || int(threadIdx.x) < QCAP;
+        // the next batch's loads are in flight while this one is summed
+        int ngx, ngy, ncp, nidx;
+        double nvr, nvi, nw;
+        auto fetch = [&](uint32_t e) {
+            const Entry* p = entries + min(e + uint32_t(slot), ee - 1);
+            ngx = p->gx;
+            ngy = p->gy;
+            ncp = p->cp;
+            nidx = p->idx;
+            nvr = p->vr;
+            nvi = p->vi;
+            nw = p->w;
+        };
+        fetch(eb);
+        __syncthreads();
+        int round = 0;
+        for (uint32_t e0 = eb; e0 < ee; e0 += uint32_t(batch)) {
+            const int gx = ngx, gy = ngy, cp = ncp;
+            const double vr = nvr, vi = nvi;
+            double w = nw;
+            const bool valid = slot < batch && e0 + uint32_t(slot) < ee;
+            if constexpr (FORM == KERNEL_EXACT) {
+                // exact kernel of this visibility pass (make_kernel_array, conv_func.h:279-303),
+                // its tap sum folded into the weight
+                double sum = 0.0;
+                if (valid) {
+                    const long long k = nidx >> 1;
+                    double uu = uv[k] * g.scale;
+                    double vv = uv[g.n + k] * g.scale;
+                    if (g.halfplane && vv < 0.0) {
+                        uu = -uu;
+                        vv = -vv;
+                    }
+                    const double x = lead ? vv : uu;
+                    double f = x - int(rint(x));
+                    if (nidx & 1)
+                        f = -f;
+                    double* kv = kt + (slot * 2 + (lead ? 0 : 1)) * ks;
+                    for (int q = 0; q < ks; q++) {
+                        const double v = dev_kernel(g, double(q - s) - f);
+                        kv[q] = v;
+                        sum += v;
+                    }
+                    if (!lead)
+                        staged[slot].a = sum;
+                }
+                __syncthreads();
+                if (valid && lead)
+                    w = w / (sum * staged[slot].a);
+            }
+            fetch(e0 + uint32_t(batch));
+            const double a = vr * w, b = vi * w;
+            // the products multiply zeros outside the footprint: entries that are not
+            // finite are added tap by tap instead, so they touch their own taps only
+            const bool odd = !(fmax(fmax(fabs(a), fabs(b)), fabs(w)) < 1.0e290) || vr != vr || vi != vi || w != w;
+            // the footprint and its wrapped pieces that overlap the tile: raw rows at +N (rows
+            // past N wrap) and, for exact kernels, -N; raw columns at +-N.  One piece a round:
+            // a second one exists only on grids hardly wider than the tile.
+            const int iraw = r0 - (gy - s), jraw = c0 - (gx - s);
+            uint32_t pieces = 0;
+            if (valid && lead) {
+                uint32_t rp = 0, cpz = 0;
+                auto meets = [&](int o, int len) { return o < ks && o > -len; };
+                rp = (meets(iraw, TILE_R) ? 1u : 0u) | (meets(iraw + N, TILE_R) ? 2u : 0u) |
+                    (FORM == KERNEL_EXACT && meets(iraw - N, TILE_R) ? 4u : 0u);
+                cpz = (meets(jraw, TC) ? 1u : 0u) | (meets(jraw + N, TC) ? 2u : 0u) | (meets(jraw - N, TC) ? 4u : 0u);
+                pieces = ((rp & 1u) ? cpz : 0u) | ((rp & 2u) ? cpz << 3 : 0u) | ((rp & 4u) ? cpz << 6 : 0u);
+            }
+            bool more;
+            do {
+                uint32_t hits = 0; // blocks touched
+                if (pieces) {
+                    const int p = __builtin_ctz(pieces);
+                    pieces &= pieces - 1;
+                    const int pr = p / 3, pc = p % 3;
+                    const int i0 = iraw + (pr == 0 ? 0 : (pr == 1 ? N : -N)), j0 = jraw + (pc == 0 ? 0 : (pc == 1 ? N : -N));
+                    uint32_t rh = 0;
+#pragma unroll
+                    for (int k = 0; k < 4; k++)
+                        rh |= (i0 + 16 * k < ks && i0 + 16 * k > -16) ? 1u << k : 0u;
+#pragma unroll
+                    for (int k = 0; k < NB / 4; k++)
+                        hits |= (j0 + 16 * k < ks && j0 + 16 * k > -16) ? rh << (4 * k) : 0u;
+                    Staged st;
+                    st.a = odd ? vr : a;
+                    st.b = odd ? vi : b;
+                    st.w = w;
+                    const int by = FORM == KERNEL_EXACT ? 0 : (cp >> 16) * pitch + (FORM == KERNEL_PADDED ? KPAD : 0);
+                    const int bx = FORM == KERNEL_EXACT ? 0 : (cp & 0xffff) * pitch + (FORM == KERNEL_PADDED ? KPAD : 0);
+                    st.oy = FORM == KERNEL_PADDED && !odd ? by + i0 : (i0 & 0xffff) | by << 16;
+                    st.ox = FORM == KERNEL_PADDED && !odd ? bx + j0 : (j0 & 0xffff) | bx << 16;
+                    staged[slot] = st;
+                    if (odd) {
+                        oddq[atomicAdd(&oddcnt[round & 1], 1)] = uint16_t(slot);
+                        hits = 0;
+                    }
+                }
+                while (hits) {
+                    const int k = __builtin_ctz(hits);
+                    hits &= hits - 1;
+                    queues[k * QCAP + atomicAdd(&qcnt[k], 1)] = uint16_t(slot);
+                }
+                __syncthreads();
+                const int cnt = __builtin_amdgcn_readfirstlane(qcnt[wave]), nodd = __builtin_amdgcn_readfirstlane(oddcnt[round & 1]);
+                const uint16_t* queue = queues + wave * QCAP;
+                for (int q0 = 0; q0 < cnt; q0 += 64) {
+                    // 64 queued entries at once: lane (m, kk) holds entry kk of product m, and
+                    // product G takes lane G of each row of 16 lanes
+                    const int at = q0 + 4 * m + kk;
+                    const int q = queue[min(at, cnt - 1)];
+                    const Staged e = staged[q];
+                    const bool on = at < cnt;
+                    const double ea = on ? e.a : 0.0, eb4 = on ? e.b : 0.0, ew = on ? e.w : 0.0;
+                    const int groups = min(16, (cnt - q0 + 3) >> 2);
+                    for_rows(groups, [&](auto G) {
+                        constexpr int R = decltype(G)::value;
+                        const int qg = FORM == KERNEL_EXACT ? row_lane<R>(q) : 0;
+                        const double ky = block_value(qg, row_lane<R>(e.oy), br, 0);
+                        const double kx = block_value(qg, row_lane<R>(e.ox), bc, 1);
+                        ar = __builtin_amdgcn_mfma_f64_16x16x4f64(kx * row_lane<R>(ea), ky, ar, 0, 0, 0);
+                        ai = __builtin_amdgcn_mfma_f64_16x16x4f64(kx * row_lane<R>(eb4), ky, ai, 0, 0, 0);
+                        if (g.beam)
+                            ab = __builtin_amdgcn_mfma_f64_16x16x4f64(kx * row_lane<R>(ew), ky, ab, 0, 0, 0);
+                    });
+                }
+                for (int k = 0; k < nodd; k++) {
+                    const int q = oddq[k];
+                    const Staged e = staged[q];
+                    const int i = int(short(e.oy & 0xffff)) + br + m, j = int(short(e.ox & 0xffff)) + bc;
+                    const double ky = checked(FORM == KERNEL_EXACT ? q * 2 * ks : int(uint32_t(e.oy) >> 16), i);
+                    // lane m holds column value m
+                    const double kx = checked(FORM == KERNEL_EXACT ? (q * 2 + 1) * ks : int(uint32_t(e.ox) >> 16), j + m);
+#pragma unroll
+                    for (int v = 0; v < 4; v++) {
+                        const double kw = (ky * __shfl(kx, kk + 4 * v, 64)) * e.w;
+                        if (unsigned(i) < unsigned(ks) && unsigned(j + kk + 4 * v) < unsigned(ks)) {
+                            ar[v] += e.a * kw;
+                            ai[v] += e.b * kw;
+                            ab[v] += kw;
+                        }
+                    }
+                }
+                if (lane == 0)
+                    qcnt[wave] = 0;
+                if (threadIdx.x == 0)
+                    oddcnt[(round + 1) & 1] = 0;
+                round++;
+                more = __syncthreads_or(int(pieces != 0)) != 0;
+            } while (more);
+        }
+    }
+    // lane (m, kk) holds the block's row m, columns kk + 4 v
+    const int lr0 = br + m, lc0 = bc + kk;
+    if (split) {
+        uint32_t lo = 0, hi = sp.hdr[1] - 1; // the tile's record among the split tiles
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi) / 2;
+            if (sp.spl[3 * mid] < uint32_t(t))
+                lo = mid + 1;
+            else
+                hi = mid;
+        }
+        double* out = sp.part + size_t(sp.spl[3 * lo + 1] + chunk) * (3 * TC * TILE_R);
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            double* o = out + (lc0 + 4 * v) * TILE_R + lr0;
+            o[0] = ar[v];
+            o[TC * TILE_R] = ai[v];
+            if (g.beam)
+                o[2 * TC * TILE_R] = ab[v];
+        }
+        return;
+    }
+    // through LDS, so that a wave stores 64 consecutive rows of a column; the beam grid is
+    // complex (imaginary part 0) or, with g.bpack, packed real: cell (r, c) is component
+    // c & 1 of element (r, c / 2) of a rows x N/2 complex array
+    const bool some = eb < ee;
+    double* o0 = area;
+    double* o1 = area + TC * OUT_STRIDE;
+    if (some) {
+#pragma unroll
+        for (int v = 0; v < 4; v++) {
+            o0[(lc0 + 4 * v) * OUT_STRIDE + lr0] = ar[v];
+            o1[(lc0 + 4 * v) * OUT_STRIDE + lr0] = ai[v];
+        }
+        __syncthreads();
+    }
+    const int lr = threadIdx.x & 63, r = r0 + lr;
+    for (int lc = threadIdx.x >> 6; lc < TC; lc += NTH / 64) {
+        const int c = c0 + lc;
+        if (r < g.rows && c < N) {
+            cplx<T> v = { T(0), T(0) };
+            if (some)
+                v = { T(o0[lc * OUT_STRIDE + lr]), T(o1[lc * OUT_STRIDE + lr]) };
+            vgrid[size_t(r) + size_t(c) * g.rows] = v;
+        }
+    }
+    if (!g.beam)
+        return;
+    if (some) {
+        __syncthreads();
+#pragma unroll
+        for (int v = 0; v < 4; v++)
+            o0[(lc0 + 4 * v) * OUT_STRIDE + lr0] = ab[v];
+        __syncthreads();
+    }
+    for (int lc = threadIdx.x >> 6; lc < (g.bpack ? TC / 2 : TC); lc += NTH / 64) {
+        const int c = c0 + (g.bpack ? 2 * lc : lc);
+        if (r < g.rows && c < N) {
+            cplx<T> v = { T(0), T(0) };
+            if (some && g.bpack)
+                v = { T(o0[2 * lc * OUT_STRIDE + lr]), T(o0[(2 * lc + 1) * OUT_STRIDE + lr]) };
+            else if (some)
+                v = { T(o0[lc * OUT_STRIDE + lr]), T(0) };
+            bgrid[size_t(r) + size_t(g.bpack ? c / 2 : c) * g.rows] = v;
+        }
+    }
+}
+
+template <typename T, int TC, int FORM>
+__global__ __launch_bounds__(tile_threads(TC), tile_waves(FORM)) void grid_tiles_kernel(GridGeom g, Entry* entries, const uint32_t* offsets,
+    uint32_t cap, const double* ktab, const double* uv, cplx<T>* vgrid, cplx<T>* bgrid, int ext_host)
+{
+    tiles_mfma_body<T, TC, FORM>(g, entries, offsets, cap, ktab, uv, vgrid, bgrid, ext_host, int(blockIdx.x));
+}
+
+// Workgroup q of the merges: columns 4 (q % (tc / 4)) .. + 3 of split tile q / (tc / 4), the
+// sum of its chunks' slots in chunk order.  lds: 4 x TILE_R doubles.
+template <typename T>
+__device__ __forceinline__ void merge_body(const GridGeom& g, Entry* entries, uint32_t cap, uint32_t nent, int ext_host,
+    cplx<T>* vgrid, cplx<T>* bgrid, int q, double* lds)
+{
+    const Split sp = split_view(entries, cap, nent, ext_host, g.tc);
+    const int groups = g.tc / 4;
+    const uint32_t i = uint32_t(q / groups);
+    if (!sp.hdr || i >= sp.hdr[1])
+        return;
+    const int t = int(sp.spl[3 * i]);
+    const uint32_t slot = sp.spl[3 * i + 1], n = sp.spl[3 * i + 2];
+    const int lr = threadIdx.x & 63, lq = threadIdx.x >> 6, lc = 4 * (q % groups) + lq;
+    const size_t plane = size_t(g.tc) * TILE_R;
+    const double* p = sp.part + slot * 3 * plane + size_t(lc) * TILE_R + lr;
+    double a = 0.0, b = 0.0, w = 0.0;
+#pragma unroll 4
+    for (uint32_t k = 0; k < n; k++, p += 3 * plane) {
+        a += p[0];
+        b += p[plane];
+        if (g.beam)
+            w += p[2 * plane];
+    }
+    const int r = (t % g.tiles_r) * TILE_R + lr, c = (t / g.tiles_r) * g.tc + lc;
+    const bool cell = r < g.rows && c < g.N;
+    if (cell)
+        vgrid[size_t(r) + size_t(c) * g.rows] = { T(a), T(b) };
+    if (!g.beam)
+        return;
+    if (!g.bpack) {
+        if (cell)
+            bgrid[size_t(r) + size_t(c) * g.rows] = { T(w), T(0) };
+        return;
+    }
+    lds[threadIdx.x] = w;
+    __syncthreads();
+    if (cell && !(lq & 1))
+        bgrid[size_t(r) + size_t(c / 2) * g.rows] = { T(w), T(lds[threadIdx.x + 64]) };
+}
+
+// Workgroup 0: the last canonical level of the (good weights, good count) block pairs,
+// which gives the sampling grid total 2 * sum(weights) and the good count, and the number
+// of gridding entries (the end of the last tile's range).  The others merge split tiles.
+template <typename T>
+__global__ __launch_bounds__(CANON_LANES) void grid_total_kernel(const double* part, unsigned m, double* total,
+    unsigned long long* ngood, const uint32_t* entries_end, unsigned long long* nentries, GridGeom g, Entry* entries,
+    uint32_t cap, int ext_host, cplx<T>* vgrid, cplx<T>* bgrid)
+{
+    __shared__ double lds[2 * CANON_LANES];
+    if (blockIdx.x > 0) {
+        merge_body<T>(g, entries, cap, *entries_end, ext_host, vgrid, bgrid, int(blockIdx.x) - 1, lds);
+        return;
+    }
+    double a, b;
+    canon_last_level(part, m, a, b, lds);
+    if (threadIdx.x == 0) {
+        total[0] = a * 2.0;
+        if (ngood)
+            *ngood = (unsigned long long)b;
+        if (nentries)
+            *nentries = *entries_end;
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Two-float tile sums (STP_PRECISION_FP32_TWOFLOAT): one workgroup per tile
+// accumulates the taps of every entry binned to it in LDS, then writes the tile once.
+// Lane mapping for supports up to 31: a wave takes 64 / ks entries at a time, lane
+// (entry e, kernel column j) walks the ks kernel rows, so one load of kx[j] serves ks
+// taps and the ks LDS atomics of a lane are independent.  Wider kernels take one entry
+// per wave, lanes striding columns.  Each channel keeps an unevaluated pair hi + lo:
+// the returning atomic add on hi yields the old value, so the rounding error of the
+// sum it stored is known exactly (Knuth's TwoSum on old and x) and is added to lo.
 constexpr int TWG = 512;
 constexpr int TEB = 256;                  // entries staged per batch
-constexpr int KV_DOUBLES = 3584;          // exact mode: per-entry kernel vectors (28 KB)
 
 constexpr int RG = 4;                     // kernel rows per group of LDS atomics
 
-// FP64 accumulation (ds_add_f64) of FP64 or FP32 taps.
-struct AccF64 {
-    using S = double;
-    static constexpr int arrays = 3;      // re, im, beam
-    template <int R, typename T>
-    __device__ static void add_rows(double* base, int plane, const int* aa, const T* xr, const T* xi,
-        const T* xb, bool beam)
-    {
-#pragma unroll
-        for (int u = 0; u < R; u++) {
-            if (aa[u] < 0)
-                continue;
-            unsafeAtomicAdd(&base[aa[u]], double(xr[u]));
-            unsafeAtomicAdd(&base[plane + aa[u]], double(xi[u]));
-            if (beam)
-                unsafeAtomicAdd(&base[2 * plane + aa[u]], double(xb[u]));
-        }
-    }
-    __device__ static double value(const double* base, int plane, int ch, int a) { return base[ch * plane + a]; }
-};
 // Error of the rounded sum s = fl(old + x) (TwoSum).
 __device__ __forceinline__ float two_sum_err(float old, float x)
 {
@@ -781,7 +1305,7 @@ __device__ __forceinline__ void write_tile(const GridGeom& g, const typename Acc
 }
 
 template <typename T, typename Acc>
-__global__ __launch_bounds__(TWG) void grid_tiles_kernel(GridGeom g, const Entry* entries, const uint32_t* offsets, int ostride,
+__global__ __launch_bounds__(TWG) void grid_tiles_twofloat_kernel(GridGeom g, const Entry* entries, const uint32_t* offsets, int ostride,
     uint32_t cap, const double* ktab, const double* uv, cplx<T>* vgrid, cplx<T>* bgrid)
 {
 #pragma clang fp contract(off)
@@ -896,10 +1420,9 @@ __global__ __launch_bounds__(TWG) void grid_tiles_kernel(GridGeom g, const Entry
 }
 
 // Oversampled-kernel tiles with ks <= KSM taps per side (the common case): the
-// same lane mapping and tap arithmetic as grid_tiles_kernel, specialised so a
+// same lane mapping and tap arithmetic as grid_tiles_twofloat_kernel, specialised so a
 // lane preloads its entry's ks kernel-row values and computes row validity
-// without branches; taps that miss the tile issue no LDS atomic (the LDS FP64
-// atomic rate bounds this kernel).
+// without branches; taps that miss the tile issue no LDS atomic.
 template <typename T, typename Acc, int KSM>
 __device__ __forceinline__ void tiles_os_body(const GridGeom& g, const Entry* entries, const uint32_t* offsets, int ostride,
     uint32_t cap, const double* ktab, cplx<T>* vgrid, cplx<T>* bgrid, int t)
@@ -1850,6 +2373,7 @@ struct BItem {
     unsigned long long* ngood;
     uint32_t cap;
     int nblk;
+    int ext_host;              // extra chunk workgroups of split tiles
 };
 
 __device__ __forceinline__ int batch_item(const uint32_t* __restrict__ pre, int K, uint32_t b)
@@ -1886,33 +2410,54 @@ __global__ __launch_bounds__(BWG) void batch_scatter_kernel(const BItem* __restr
 {
     const int k = batch_item(pre, K, blockIdx.x);
     const BItem& it = items[k];
-    bin_scatter_body(it.g, it.uv, it.vis, it.wts, it.totals, it.counts, it.entries, it.cap, it.toffs,
+    bin_scatter_body(it.g, it.uv, it.vis, it.wts, it.totals, it.counts, it.entries, it.cap, it.toffs, it.ext_host,
         int(blockIdx.x - pre[k]));
 }
 
-template <typename T, typename Acc, int KSM>
-__global__ __launch_bounds__(TWG) void batch_tiles_kernel(const BItem* __restrict__ items, const uint32_t* __restrict__ pre,
+template <typename Acc, int KSM>
+__global__ __launch_bounds__(TWG) void batch_tiles_twofloat_kernel(const BItem* __restrict__ items,
+    const uint32_t* __restrict__ pre, int K)
+{
+    const int k = batch_item(pre, K, blockIdx.x);
+    const BItem& it = items[k];
+    tiles_os_body<float, Acc, KSM>(it.g, it.entries, it.toffs, 1, it.cap, it.ktab, (cplx<float>*)it.vgrid,
+        (cplx<float>*)it.bgrid, int(blockIdx.x - pre[k]));
+}
+
+template <typename T, int TC, int FORM>
+__global__ __launch_bounds__(tile_threads(TC), tile_waves(FORM)) void batch_tiles_kernel(const BItem* __restrict__ items, const uint32_t* __restrict__ pre,
     int K)
 {
     const int k = batch_item(pre, K, blockIdx.x);
     const BItem& it = items[k];
-    tiles_os_body<T, Acc, KSM>(it.g, it.entries, it.toffs, 1, it.cap, it.ktab, (cplx<T>*)it.vgrid, (cplx<T>*)it.bgrid,
-        int(blockIdx.x - pre[k]));
+    tiles_mfma_body<T, TC, FORM>(it.g, it.entries, it.toffs, it.cap, it.ktab, it.uv, (cplx<T>*)it.vgrid,
+        (cplx<T>*)it.bgrid, it.ext_host, int(blockIdx.x - pre[k]));
 }
 
-// One workgroup per snapshot: the last canonical level of its weight pairs (at
-// most CANON_BLOCK blocks), sample_grid_total and the good count.
-__global__ __launch_bounds__(CANON_LANES) void batch_total_kernel(const BItem* __restrict__ items)
+// Workgroups 0 .. K-1: the last canonical level of a snapshot's weight pairs (at most
+// CANON_BLOCK blocks), sample_grid_total and the good count; the others: the merges of
+// split tiles.
+template <typename T>
+__global__ __launch_bounds__(CANON_LANES) void batch_total_kernel(const BItem* __restrict__ items,
+    const uint32_t* __restrict__ pre, int K)
 {
     __shared__ double lds[2 * CANON_LANES];
-    const BItem& it = items[blockIdx.x];
-    double a, b;
-    canon_last_level(it.wpart, unsigned(it.nblk), a, b, lds);
-    if (threadIdx.x == 0) {
-        it.total[0] = a * 2.0;
-        if (it.ngood)
-            *it.ngood = (unsigned long long)b;
+    if (blockIdx.x < unsigned(K)) {
+        const BItem& it = items[blockIdx.x];
+        double a, b;
+        canon_last_level(it.wpart, unsigned(it.nblk), a, b, lds);
+        if (threadIdx.x == 0) {
+            it.total[0] = a * 2.0;
+            if (it.ngood)
+                *it.ngood = (unsigned long long)b;
+        }
+        return;
     }
+    const uint32_t q = blockIdx.x - unsigned(K);
+    const int k = batch_item(pre, K, q);
+    const BItem& it = items[k];
+    merge_body<T>(it.g, it.entries, it.cap, it.toffs[it.g.tiles_r * it.g.tiles_c], it.ext_host, (cplx<T>*)it.vgrid,
+        (cplx<T>*)it.bgrid, int(q - pre[k]), lds);
 }
 
 } // namespace
@@ -1969,6 +2514,35 @@ static GridGeom make_geom(const GridderArgs& a, size_t n, bool beam, KernelFn& k
     return g;
 }
 
+template <typename T, int FORM>
+static auto tiles_kernel_of(int tc)
+{
+    return tc == 16 ? grid_tiles_kernel<T, 16, FORM> : (tc == 32 ? grid_tiles_kernel<T, 32, FORM> : grid_tiles_kernel<T, 64, FORM>);
+}
+
+// The two-float tile sums of one call (ostride: stride of the tile offsets).
+static void twofloat_tiles(stp_ctx* ctx, const GridGeom& g, int cs, const Entry* entries, const uint32_t* offsets, int ostride,
+    uint32_t cap, const double* d_tab, const double* d_uv, cplx<float>* vgrid, cplx<float>* bgrid)
+{
+    const int ntiles = g.tiles_r * g.tiles_c;
+    const int S = TILE_R + (g.ks <= 15 ? g.ks : 1);
+    const size_t acc_bytes = ((6 * size_t(g.tc) * S * sizeof(float) + 7) / 8) * 8;
+    if (!g.exact && g.ks <= 16) {
+        // oversampled kernels up to 16 taps: the specialised tile kernel
+        const size_t bytes = acc_bytes + sizeof(double) * size_t(cs) * g.ks;
+        auto kern = g.ks <= 8 ? grid_tiles_os_kernel<float, AccTwoFloat, 8> : grid_tiles_os_kernel<float, AccTwoFloat, 16>;
+        HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)));
+        launch(ctx, "grid_tiles", kern, dim3(unsigned(ntiles)), dim3(TWG), bytes, g, entries, offsets, ostride, cap, d_tab, vgrid,
+            bgrid);
+    } else {
+        const size_t bytes = acc_bytes + (g.exact ? sizeof(double) * (KV_DOUBLES + TEB) : sizeof(double) * size_t(cs) * g.ks);
+        auto kern = grid_tiles_twofloat_kernel<float, AccTwoFloat>;
+        HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(bytes)));
+        launch(ctx, "grid_tiles", kern, dim3(unsigned(ntiles)), dim3(TWG), bytes, g, entries, offsets, ostride, cap, d_tab, d_uv,
+            vgrid, bgrid);
+    }
+}
+
 template <typename T>
 void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const double* d_uv, const double* d_vis,
     const double* d_w, cplx<T>* d_vis_grid, cplx<T>* d_sampling_grid, double* d_total, unsigned long long* d_ngood)
@@ -1991,6 +2565,9 @@ void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const doubl
         d_tab = dev_table(ctx, "k1d:none", std::vector<double>(1, 0.0));
     }
 
+    // FP64 tile sums (every path but two-float and W-projection) run on the matrix cores
+    const bool twofloat = std::is_same<T, float>::value && a.twofloat;
+    const bool mfma = !wproj && !twofloat;
     const size_t nblk = std::max<size_t>(1, (n + VPB - 1) / VPB);
     double* wpart = (double*)ws_get(ctx, "grid_wpart", sizeof(double) * (2 * nblk + 2));
     double* wscr = (double*)ws_get(ctx, "grid_wscr", sizeof(double) * canon_scratch_doubles(nblk));
@@ -2144,6 +2721,7 @@ void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const doubl
         }
     }
 
+    int ext_host = 0; // extra workgroups for split tiles
     const uint32_t* offsets;
     int ostride;
     const uint32_t* bcur = nullptr; // block cursors inside each tile (block binning only)
@@ -2156,12 +2734,13 @@ void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const doubl
         const size_t hist_bytes = sizeof(uint32_t) * size_t(ntiles);
         HIP_CHECK(hipFuncSetAttribute((const void*)grid_bin_count_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, int(hist_bytes)));
         HIP_CHECK(hipFuncSetAttribute((const void*)grid_bin_scatter_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, int(hist_bytes)));
+        ext_host = mfma ? split_extra_max(n) : 0;
         launch(ctx, "grid_count", grid_bin_count_kernel, dim3(unsigned(nblk)), dim3(BWG), hist_bytes, g, d_uv, d_vis, d_w, counts,
             wpart);
         launch(ctx, "grid_colscan", bin_colscan_kernel, dim3(div_up(ntiles, 64)), dim3(1024), 0, counts, int(nblk), int(ntiles),
             totals);
         launch(ctx, "grid_scatter", grid_bin_scatter_kernel, dim3(unsigned(nblk)), dim3(BWG), hist_bytes, g, d_uv, d_vis, d_w,
-            (const uint32_t*)totals, (const uint32_t*)counts, entries, cap, toffs);
+            (const uint32_t*)totals, (const uint32_t*)counts, entries, cap, toffs, ext_host);
         offsets = toffs;
         ostride = 1;
         bcur = counts;
@@ -2218,32 +2797,27 @@ void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const doubl
         }
     } else {
         STP_REQUIRE(a.kernel_exact || cs * g.ks <= KV_DOUBLES, "oversampled kernel table too large");
-        const bool twofloat = std::is_same<T, float>::value && a.twofloat;
-        const int S = TILE_R + (g.ks <= 15 ? g.ks : 1);
-        const size_t acc_bytes = twofloat ? 6 * size_t(g.tc) * S * sizeof(float) : 3 * size_t(g.tc) * S * sizeof(double);
-        const size_t kv_bytes = a.kernel_exact ? sizeof(double) * (KV_DOUBLES + TEB) : sizeof(double) * size_t(cs) * g.ks;
-        if (!a.kernel_exact && g.ks <= 16) {
-            // oversampled kernels up to 16 taps: the specialised tile kernel
-            const size_t os_acc = (twofloat ? 6 * sizeof(float) : 3 * sizeof(double)) * (size_t(g.tc) * S);
-            const size_t os_bytes = ((os_acc + 7) / 8) * 8 + kv_bytes;
-            auto kern = g.ks <= 8 ? (twofloat ? grid_tiles_os_kernel<T, AccTwoFloat, 8> : grid_tiles_os_kernel<T, AccF64, 8>)
-                                  : (twofloat ? grid_tiles_os_kernel<T, AccTwoFloat, 16> : grid_tiles_os_kernel<T, AccF64, 16>);
-            HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(os_bytes)));
-            launch(ctx, "grid_tiles", kern, dim3(ntiles), dim3(TWG), os_bytes, g, (const Entry*)entries, offsets, ostride, cap,
-                d_tab, d_vis_grid, d_sampling_grid);
-        } else {
-            const size_t dyn_bytes = ((acc_bytes + 7) / 8) * 8 + kv_bytes;
-            auto kern = twofloat ? grid_tiles_kernel<T, AccTwoFloat> : grid_tiles_kernel<T, AccF64>;
-            HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(dyn_bytes)));
-            launch(ctx, "grid_tiles", kern, dim3(ntiles), dim3(TWG), dyn_bytes, g, (const Entry*)entries, offsets, ostride, cap,
-                d_tab, d_uv, d_vis_grid, d_sampling_grid);
+        if constexpr (std::is_same<T, float>::value) {
+            if (twofloat)
+                twofloat_tiles(ctx, g, cs, entries, offsets, ostride, cap, d_tab, d_uv, d_vis_grid, d_sampling_grid);
+        }
+        if (mfma) {
+            const int form = a.kernel_exact ? KERNEL_EXACT : table_form(cs, g.ks);
+            auto kern = form == KERNEL_PADDED ? tiles_kernel_of<T, KERNEL_PADDED>(g.tc)
+                                              : (form == KERNEL_TABLE ? tiles_kernel_of<T, KERNEL_TABLE>(g.tc)
+                                                                      : tiles_kernel_of<T, KERNEL_EXACT>(g.tc));
+            const size_t lds = tiles_lds(g.tc, form, cs, g.ks);
+            HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(lds)));
+            launch(ctx, "grid_tiles", kern, dim3(unsigned(ntiles + ext_host)), dim3(unsigned(g.tc * 16)), lds, g, entries,
+                offsets, cap, d_tab, d_uv, d_vis_grid, d_sampling_grid, ext_host);
         }
     }
     // sample_grid_total = 2 * sum(good weights) (gridder.h:415-423); the good count
     size_t mfin = 0;
     const double* fin = canon_reduce_to_block(ctx, wpart, nblk, wscr, &mfin);
-    launch(ctx, "grid_total", grid_total_kernel, dim3(1), dim3(CANON_LANES), 0, fin, unsigned(mfin), d_total, d_ngood,
-        offsets + size_t(ntiles) * ostride, a.d_nentries);
+    launch(ctx, "grid_total", grid_total_kernel<T>, dim3(unsigned(1 + merge_blocks(ext_host, g.tc))), dim3(CANON_LANES), 0, fin,
+        unsigned(mfin), d_total, d_ngood, offsets + size_t(ntiles) * ostride, a.d_nentries, g, entries, cap, ext_host, d_vis_grid,
+        d_sampling_grid);
 }
 
 bool grid_batch_eligible(const GridderArgs& a, size_t n)
@@ -2276,8 +2850,8 @@ BatchPlan grid_batch_bin(stp_ctx* ctx, const std::vector<BatchGridItem>& items, 
     // tile launches per class: kernel width (up to 8 or 16 taps) x tile width (16, 32,
     // 64 columns), so each launch reserves the LDS its own tiles need
     constexpr int NCLS = BatchPlan::CLASSES;
-    std::vector<uint32_t> pre_b(K), pre_c(K), pre_t(size_t(NCLS) * K);
-    size_t nb = 0, nc = 0, nt[NCLS] = {}, pool = 0, hist_bytes = 4, tile_bytes[NCLS] = {};
+    std::vector<uint32_t> pre_b(K), pre_c(K), pre_t(size_t(NCLS) * K), pre_m(K);
+    size_t nb = 0, nc = 0, nm = 0, nt[NCLS] = {}, pool = 0, hist_bytes = 4, tile_bytes[NCLS] = {};
     for (int k = 0; k < K; k++) {
         const BatchGridItem& it = items[k];
         STP_REQUIRE(grid_batch_eligible(it.a, it.n), "snapshot not eligible for a fused batch");
@@ -2314,19 +2888,28 @@ BatchPlan grid_batch_bin(stp_ctx* ctx, const std::vector<BatchGridItem>& items, 
         pool = al(pool + sizeof(double) * (2 * nblk + 2));
         p.entries = pool;
         pool = al(pool + sizeof(Entry) * cap64);
+        b.ext_host = twofloat ? 0 : split_extra_max(it.n);
+        pre_m[k] = uint32_t(nm);
+        nm += merge_blocks(b.ext_host, g.tc);
         pre_b[k] = uint32_t(nb);
         nb += nblk;
         pre_c[k] = uint32_t(nc);
         nc += div_up(ntiles, 64);
-        const int cls = (g.ks <= 8 ? 0 : 3) + (g.tc == 16 ? 0 : (g.tc == 32 ? 1 : 2));
+        const int form = table_form((g.os / 2) * 2 + 1, g.ks);
+        const int cls = ((twofloat ? g.ks <= 8 : form == KERNEL_PADDED) ? 0 : 3) + (g.tc == 16 ? 0 : (g.tc == 32 ? 1 : 2));
         for (int c = 0; c < NCLS; c++)
             pre_t[size_t(c) * K + k] = uint32_t(nt[c]);
-        nt[cls] += ntiles;
+        nt[cls] += size_t(ntiles) + b.ext_host;
         hist_bytes = std::max(hist_bytes, sizeof(uint32_t) * size_t(ntiles));
-        const int S = TILE_R + (g.ks <= 15 ? g.ks : 1);
-        const size_t acc = (twofloat ? 6 * sizeof(float) : 3 * sizeof(double)) * (size_t(g.tc) * S);
         const int cs = (g.os / 2) * 2 + 1;
-        tile_bytes[cls] = std::max(tile_bytes[cls], ((acc + 7) / 8) * 8 + sizeof(double) * size_t(cs) * g.ks);
+        size_t lds;
+        if (twofloat) {
+            const int S = TILE_R + (g.ks <= 15 ? g.ks : 1);
+            lds = ((6 * sizeof(float) * (size_t(g.tc) * S) + 7) / 8) * 8 + sizeof(double) * size_t(cs) * g.ks;
+        } else {
+            lds = tiles_lds(g.tc, form, cs, g.ks);
+        }
+        tile_bytes[cls] = std::max(tile_bytes[cls], lds);
     }
     STP_REQUIRE(nb < (size_t(1) << 31) && *std::max_element(nt, nt + NCLS) < (size_t(1) << 31),
         "too many workgroups for one fused batch");
@@ -2341,7 +2924,7 @@ BatchPlan grid_batch_bin(stp_ctx* ctx, const std::vector<BatchGridItem>& items, 
     // tables: items, the stage prefixes, the caller's tables; one upload from the
     // page-locked stage once the previous batch's upload has left it
     const size_t o_items = 0, o_b = al(sizeof(BItem) * K), o_c = o_b + al(4 * K), o_t = o_c + al(4 * K);
-    const size_t o_x = o_t + al(4 * size_t(NCLS) * K), tab_bytes = o_x + std::max<size_t>(extra.size(), 1);
+    const size_t o_m = o_t + al(4 * size_t(NCLS) * K), o_x = o_m + al(4 * K), tab_bytes = o_x + std::max<size_t>(extra.size(), 1);
     hipEvent_t& up = ctx->batch_tab_events[ctx->ws_slot];
     if (!up)
         HIP_CHECK(hipEventCreateWithFlags(&up, hipEventDisableTiming));
@@ -2352,6 +2935,7 @@ BatchPlan grid_batch_bin(stp_ctx* ctx, const std::vector<BatchGridItem>& items, 
     memcpy(h + o_b, pre_b.data(), 4 * K);
     memcpy(h + o_c, pre_c.data(), 4 * K);
     memcpy(h + o_t, pre_t.data(), 4 * size_t(NCLS) * K);
+    memcpy(h + o_m, pre_m.data(), 4 * K);
     if (!extra.empty())
         memcpy(h + o_x, extra.data(), extra.size());
     HIP_CHECK(hipMemcpyAsync(d, h, tab_bytes, hipMemcpyHostToDevice, ctx->stream));
@@ -2369,6 +2953,8 @@ BatchPlan grid_batch_bin(stp_ctx* ctx, const std::vector<BatchGridItem>& items, 
     plan.items = K;
     plan.twofloat = twofloat;
     plan.pre_t_off = o_t;
+    plan.pre_m_off = o_m;
+    plan.merges = nm;
     for (int c = 0; c < NCLS; c++) {
         plan.tiles[c] = nt[c];
         plan.tile_lds[c] = tile_bytes[c];
@@ -2384,13 +2970,26 @@ void grid_batch_tiles(stp_ctx* ctx, const BatchPlan& plan)
     for (int c = 0; c < BatchPlan::CLASSES; c++) {
         if (plan.tiles[c] == 0)
             continue;
-        auto kern = c < 3 ? (plan.twofloat ? batch_tiles_kernel<T, AccTwoFloat, 8> : batch_tiles_kernel<T, AccF64, 8>)
-                           : (plan.twofloat ? batch_tiles_kernel<T, AccTwoFloat, 16> : batch_tiles_kernel<T, AccF64, 16>);
+        const uint32_t* pre = (const uint32_t*)((const uint8_t*)plan.d_tab + plan.pre_t_off) + size_t(c) * K;
+        if constexpr (std::is_same<T, float>::value) {
+            if (plan.twofloat) {
+                auto kern = c < 3 ? batch_tiles_twofloat_kernel<AccTwoFloat, 8> : batch_tiles_twofloat_kernel<AccTwoFloat, 16>;
+                HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(plan.tile_lds[c])));
+                launch(ctx, "batch_tiles", kern, dim3(unsigned(plan.tiles[c])), dim3(TWG), plan.tile_lds[c], d_items, pre, K);
+                continue;
+            }
+        }
+        const int w = c % 3;
+        auto kern = c < 3 ? (w == 0 ? batch_tiles_kernel<T, 16, KERNEL_PADDED>
+                                    : (w == 1 ? batch_tiles_kernel<T, 32, KERNEL_PADDED> : batch_tiles_kernel<T, 64, KERNEL_PADDED>))
+                          : (w == 0 ? batch_tiles_kernel<T, 16, KERNEL_TABLE>
+                                    : (w == 1 ? batch_tiles_kernel<T, 32, KERNEL_TABLE> : batch_tiles_kernel<T, 64, KERNEL_TABLE>));
         HIP_CHECK(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, int(plan.tile_lds[c])));
-        launch(ctx, "batch_tiles", kern, dim3(unsigned(plan.tiles[c])), dim3(TWG), plan.tile_lds[c], d_items,
-            (const uint32_t*)((const uint8_t*)plan.d_tab + plan.pre_t_off) + size_t(c) * K, K);
+        launch(ctx, "batch_tiles", kern, dim3(unsigned(plan.tiles[c])), dim3(256u << w),
+            plan.tile_lds[c], d_items, pre, K);
     }
-    launch(ctx, "batch_total", batch_total_kernel, dim3(unsigned(K)), dim3(CANON_LANES), 0, d_items);
+    launch(ctx, "batch_total", batch_total_kernel<T>, dim3(unsigned(K + plan.merges)), dim3(CANON_LANES), 0, d_items,
+        (const uint32_t*)((const uint8_t*)plan.d_tab + plan.pre_m_off), K);
 }
 
 template <typename T>

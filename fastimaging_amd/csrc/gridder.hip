@@ -32,6 +32,7 @@ namespace stp_hip {
 namespace {
 
 constexpr int TILE_R = 64;  // grid rows (v) per tile: 64 contiguous complex per column
+constexpr int W_TILE_C = 64; // with W-projection: its wide footprints touch fewer tiles
 constexpr int TILE_C = 32;  // default grid columns (u) per tile; GridderArgs::tile_cols overrides
 constexpr int GWG = 256;
 
@@ -49,12 +50,14 @@ struct GridGeom {
     int wproj = 0;
     const uint32_t* perm = nullptr;
     const uint16_t* plane = nullptr;
+    const int* psup = nullptr; // truncated support of each plane (null: s)
 };
 
 struct Entry {
     int gx, gy;   // kernel centre on the (shifted) grid for this pass
-    int cp;       // cp_x | cp_y << 16 (oversampled kernel indices); W-projection: bit 31 = conjugate kernel
-    int idx;      // visibility index << 1 | pass; W-projection: the W sub-kernel (plane, cp_y, cp_x)
+    int cp;       // cp_x | cp_y << 16 (oversampled kernel indices); W-projection: the support, bit 31 = conjugate
+                  // kernel, bits 30 and 29 = rows and columns of the sub-kernel mirrored
+    int idx;      // visibility index << 1 | pass; W-projection: the W sub-kernel (plane, |y| offset, |x| offset)
     double vr, vi, w; // W-projection: vr, vi are the visibility times w
 };
 static_assert(sizeof(Entry) == 40, "entry layout");
@@ -152,6 +155,9 @@ __device__ __forceinline__ void pass_geom(const GridGeom& g, const Prep& p, int 
     }
 }
 
+// Support of visibility position k's kernel.
+__device__ __forceinline__ int plane_support(const GridGeom& g, long long k) { return g.psup ? g.psup[g.plane[k]] : g.s; }
+
 // Entry of visibility position k, pass `pass`.  The conjugate pass conjugates the
 // visibility and negates w (gridder.h:794-805); a negative w selects the
 // conjugate W-kernel (gridder.h:826-843).
@@ -168,12 +174,13 @@ __device__ __forceinline__ Entry make_entry(const GridGeom& g, const Prep& p, in
     e.w = p.w;
     if (g.wproj) {
         const double wl = pass ? -p.wl : p.wl;
-        if (wl < 0.0)
-            e.cp |= int(0x80000000u);
-        // the W tile kernel takes the sub-kernel index (plane, cp_y, cp_x) and the
-        // visibility times its weight
-        const int cs = (g.os / 2) * 2 + 1;
-        e.idx = (int(g.plane[k]) * cs + cpy) * cs + cpx;
+        // the W tile kernel takes the sub-kernel index and the visibility times its weight;
+        // the plane's kernel is even, so the offset -y is offset y read backwards
+        const int op = g.os / 2;
+        const int y = min(cpy, 2 * op - cpy), x = min(cpx, 2 * op - cpx);
+        e.idx = (int(g.plane[k]) * (op + 1) + y) * (op + 1) + x;
+        e.cp = int(uint32_t(plane_support(g, k)) | (wl < 0.0 ? 0x80000000u : 0u) | (cpy > op ? 0x40000000u : 0u) |
+            (cpx > op ? 0x20000000u : 0u));
         e.vr = e.vr * p.w;
         e.vi = e.vi * p.w;
     } else {
@@ -250,12 +257,12 @@ __host__ __device__ __forceinline__ bool span_seen(const TileSpan& sp, int k, in
     return seen;
 }
 
-// Calls f(tile column, tile row) once for every distinct tile of the footprint.
+// Calls f(tile column, tile row) once for every distinct tile of a footprint of support s.
 template <typename F>
-__device__ __forceinline__ void visit_tiles(const GridGeom& g, int gx, int gy, F f)
+__device__ __forceinline__ void visit_tiles(const GridGeom& g, int gx, int gy, int s, F f)
 {
     TileSpan rs, cs;
-    footprint_spans(g.N, g.rows - 1, g.s, g.ks, g.exact, TILE_R, g.tc, gx, gy, rs, cs);
+    footprint_spans(g.N, g.rows - 1, s, 2 * s + 1, g.exact, TILE_R, g.tc, gx, gy, rs, cs);
 #pragma unroll
     for (int a = 0; a < 3; a++) {
         for (int ct = cs.lo[a]; ct <= cs.hi[a]; ct++) {
@@ -327,10 +334,11 @@ __global__ __launch_bounds__(GWG) void grid_count_kernel(GridGeom g, const doubl
             continue;
         wsum = wsum + p.w;
         nsum = nsum + 1.0;
+        const int sup = plane_support(g, i);
         for (int pass = 0; pass <= p.dup; pass++) {
             int gx, gy, cpx, cpy;
             pass_geom(g, p, pass, gx, gy, cpx, cpy);
-            visit_tiles(g, gx, gy, [&](int ct, int rt) { atomicAdd(&counts[ct * g.tiles_r + rt], 1u); });
+            visit_tiles(g, gx, gy, sup, [&](int ct, int rt) { atomicAdd(&counts[ct * g.tiles_r + rt], 1u); });
         }
     }
     canon_tree(wsum, nsum, lds);
@@ -411,9 +419,10 @@ __global__ __launch_bounds__(GWG) void grid_scatter_kernel(GridGeom g, const dou
     const Prep p = prep_vis(g, uv, vis, wts, i);
     if (!p.good)
         return;
+    const int sup = plane_support(g, i);
     for (int pass = 0; pass <= p.dup; pass++) {
         const Entry e = make_entry(g, p, pass, i);
-        visit_tiles(g, e.gx, e.gy, [&](int ct, int rt) {
+        visit_tiles(g, e.gx, e.gy, sup, [&](int ct, int rt) {
             const uint32_t slot = atomicAdd(&cursor[ct * g.tiles_r + rt], 1u);
             if (slot < cap)
                 entries[slot] = e;
@@ -461,10 +470,11 @@ __device__ __forceinline__ void bin_count_body(const GridGeom& g, const double* 
             if (p.good) {
                 wgood = p.w;
                 ng++;
+                const int sup = plane_support(g, i);
                 for (int pass = 0; pass <= p.dup; pass++) {
                     int gx, gy, cpx, cpy;
                     pass_geom(g, p, pass, gx, gy, cpx, cpy);
-                    visit_tiles(g, gx, gy, [&](int ct, int rt) { atomicAdd(&hist[ct * g.tiles_r + rt], 1u); });
+                    visit_tiles(g, gx, gy, sup, [&](int ct, int rt) { atomicAdd(&hist[ct * g.tiles_r + rt], 1u); });
                 }
             }
         }
@@ -610,6 +620,7 @@ __device__ uint32_t scan_tile_totals(const uint32_t* totals, int ntiles, uint32_
 // taps; 1.2 to 1.6 are used): every kernel derives the same view from the entry count,
 // and where the end is short there are fewer chunks or none.
 constexpr uint32_t SPLIT_MIN = 1024;
+constexpr uint32_t W_SPLIT_MIN = 256; // W-projection: an entry has up to 4096 taps in a tile
 constexpr size_t SPLIT_EXTRA_MAX = 512;
 constexpr size_t SPLIT_PLAN_BYTES = 16384;
 static_assert(256 + SPLIT_EXTRA_MAX * 20 <= SPLIT_PLAN_BYTES, "plan layout");
@@ -617,19 +628,19 @@ struct Split {
     uint32_t* hdr;     // extra chunks, split tiles, ch (null: no splitting)
     uint32_t* ext;     // per extra chunk: tile, chunk
     uint32_t* spl;     // per split tile (in tile order): tile, first slot, chunks
-    double* part;      // slots of 3 x tile columns x TILE_R sums
+    double* part;      // slots of chans x tile columns x TILE_R sums
     size_t room;       // bytes for slots
 };
 
-inline int split_extra_max(size_t n) { return int(std::min(SPLIT_EXTRA_MAX, n / SPLIT_MIN)); }
+inline int split_extra_max(size_t n, uint32_t least = SPLIT_MIN) { return int(std::min(SPLIT_EXTRA_MAX, n / least)); }
 // Merge workgroups (four tile columns each).
 inline size_t merge_blocks(int ext_host, int tc) { return size_t(ext_host) * (tc / 4); }
 
-__device__ __forceinline__ Split split_view(Entry* entries, uint32_t cap, uint32_t nent, int ext_host, int tc)
+__device__ __forceinline__ Split split_view(Entry* entries, uint32_t cap, uint32_t nent, int ext_host, int tc, int chans)
 {
     Split sp{ nullptr, nullptr, nullptr, nullptr, 0 };
     const size_t used = (size_t(nent) * sizeof(Entry) + 255) & ~size_t(255);
-    const size_t room = size_t(cap) * sizeof(Entry), slot = size_t(3) * tc * TILE_R * sizeof(double);
+    const size_t room = size_t(cap) * sizeof(Entry), slot = size_t(chans) * tc * TILE_R * sizeof(double);
     if (ext_host <= 0 || room < used + SPLIT_PLAN_BYTES + 2 * slot)
         return sp;
     sp.room = room - used - SPLIT_PLAN_BYTES;
@@ -643,12 +654,12 @@ __device__ __forceinline__ Split split_view(Entry* entries, uint32_t cap, uint32
 
 // The plan from the tile totals, by one workgroup of BWG threads.
 __device__ void split_plan(const Split& sp, const uint32_t* totals, int ntiles, uint32_t total, int ext_host, int tc,
-    uint32_t* wsum)
+    int chans, uint32_t least, uint32_t* wsum)
 {
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const size_t slot = size_t(3) * tc * TILE_R * sizeof(double);
+    const size_t slot = size_t(chans) * tc * TILE_R * sizeof(double);
     const uint32_t ext_max = uint32_t(min(size_t(ext_host), sp.room / (2 * slot)));
-    const uint32_t ch = max(SPLIT_MIN, (total + ext_max - 1) / ext_max);
+    const uint32_t ch = max(least, (total + ext_max - 1) / ext_max);
     const int per = (ntiles + BWG - 1) / BWG;
     const int i0 = min(ntiles, tid * per), i1 = min(ntiles, i0 + per);
     uint32_t s = 0; // extra chunks | split tiles << 16
@@ -732,9 +743,10 @@ __device__ __forceinline__ void bin_scatter_body(const GridGeom& g, const double
         const Prep p = prep_in(g, in[j]);
         if (!p.good)
             continue;
-            for (int pass = 0; pass <= p.dup; pass++) {
+            const int sup = plane_support(g, i);
+        for (int pass = 0; pass <= p.dup; pass++) {
             const Entry e = make_entry(g, p, pass, i);
-            visit_tiles(g, e.gx, e.gy, [&](int ct, int rt) {
+            visit_tiles(g, e.gx, e.gy, sup, [&](int ct, int rt) {
                 const uint32_t slot = atomicAdd(&cur[ct * g.tiles_r + rt], 1u);
                 if (slot < cap)
                     entries[slot] = e;
@@ -742,9 +754,10 @@ __device__ __forceinline__ void bin_scatter_body(const GridGeom& g, const double
         }
     }
     if (bid == 0 && ext_host > 0) {
-        const Split sp = split_view(entries, cap, total, ext_host, g.tc);
+        const int chans = g.wproj ? 4 : 3;
+        const Split sp = split_view(entries, cap, total, ext_host, g.tc, chans);
         if (sp.hdr)
-            split_plan(sp, totals, ntiles, total, ext_host, g.tc, wsum);
+            split_plan(sp, totals, ntiles, total, ext_host, g.tc, chans, g.wproj ? W_SPLIT_MIN : SPLIT_MIN, wsum);
     }
 }
 
@@ -861,7 +874,7 @@ __device__ __forceinline__ void tiles_mfma_body(const GridGeom& g, Entry* entrie
     const int ks = g.ks, s = g.s, N = g.N;
     const int cs = (g.os / 2) * 2 + 1;
     const int ntiles = g.tiles_r * g.tiles_c;
-    const Split sp = split_view(entries, cap, offsets[ntiles], ext_host, TC);
+    const Split sp = split_view(entries, cap, offsets[ntiles], ext_host, TC, 3);
     uint32_t chunk = 0;
     int t = bid - ext_host;
     if (t < 0) {
@@ -1152,7 +1165,8 @@ template <typename T>
 __device__ __forceinline__ void merge_body(const GridGeom& g, Entry* entries, uint32_t cap, uint32_t nent, int ext_host,
     cplx<T>* vgrid, cplx<T>* bgrid, int q, double* lds)
 {
-    const Split sp = split_view(entries, cap, nent, ext_host, g.tc);
+    const int chans = g.wproj ? 4 : 3; // W-projection: a complex beam grid
+    const Split sp = split_view(entries, cap, nent, ext_host, g.tc, chans);
     const int groups = g.tc / 4;
     const uint32_t i = uint32_t(q / groups);
     if (!sp.hdr || i >= sp.hdr[1])
@@ -1161,14 +1175,17 @@ __device__ __forceinline__ void merge_body(const GridGeom& g, Entry* entries, ui
     const uint32_t slot = sp.spl[3 * i + 1], n = sp.spl[3 * i + 2];
     const int lr = threadIdx.x & 63, lq = threadIdx.x >> 6, lc = 4 * (q % groups) + lq;
     const size_t plane = size_t(g.tc) * TILE_R;
-    const double* p = sp.part + slot * 3 * plane + size_t(lc) * TILE_R + lr;
-    double a = 0.0, b = 0.0, w = 0.0;
+    const double* p = sp.part + slot * chans * plane + size_t(lc) * TILE_R + lr;
+    double a = 0.0, b = 0.0, w = 0.0, wi = 0.0;
 #pragma unroll 4
-    for (uint32_t k = 0; k < n; k++, p += 3 * plane) {
+    for (uint32_t k = 0; k < n; k++, p += chans * plane) {
         a += p[0];
         b += p[plane];
-        if (g.beam)
+        if (g.beam) {
             w += p[2 * plane];
+            if (g.wproj)
+                wi += p[3 * plane];
+        }
     }
     const int r = (t % g.tiles_r) * TILE_R + lr, c = (t / g.tiles_r) * g.tc + lc;
     const bool cell = r < g.rows && c < g.N;
@@ -1178,7 +1195,7 @@ __device__ __forceinline__ void merge_body(const GridGeom& g, Entry* entries, ui
         return;
     if (!g.bpack) {
         if (cell)
-            bgrid[size_t(r) + size_t(c) * g.rows] = { T(w), T(0) };
+            bgrid[size_t(r) + size_t(c) * g.rows] = { T(w), T(wi) };
         return;
     }
     lds[threadIdx.x] = w;
@@ -1785,10 +1802,12 @@ __global__ void wk_fill_kernel(cplx<double>* comb, int arr, int half, const doub
     comb[e] = v;
 }
 
-// Each sub-kernel is stored column-major with WPAD zero columns on both sides
-// (ks rows x (ks + 2 WPAD) columns), so that the W tile kernel's column runs
-// starting up to WPAD columns outside the kernel read zeros.
+// Each sub-kernel is stored column-major with WPAD zero columns on both sides, so that the
+// W tile kernel's column runs starting up to WPAD columns outside the kernel read zeros.
 constexpr int WPAD = W_KERNEL_PAD_COLS;
+// A kernel of ks taps per side is a zero, then ks + 2 WPAD columns of ks values and a zero
+// each, so that the rows before and after every column read zero too.
+__host__ __device__ constexpr size_t w_slot(int ks) { return size_t(1) + size_t(ks + 1) * (ks + 2 * WPAD); }
 
 // ---------------------------------------------------------------------------
 // Hankel W-kernels (hankel_opt; aw_projection.cpp:211-287,380-411, aw_projection.h:127-213)
@@ -2027,16 +2046,15 @@ __global__ __launch_bounds__(256) void wk_hankel_extract_kernel(HankelArgs h, co
 {
     __shared__ double red[256];
     const int p = p0 + int(blockIdx.y);
-    const int cs = (h.os / 2) * 2 + 1;
+    const int cs = h.os / 2 + 1;
     const int x = blockIdx.x % cs, yy = blockIdx.x / cs;
-    const int ks = 2 * h.support + 1, kw = ks + 2 * WPAD;
     const int ts = psup[p], ko = (ts * 2 + 2) * h.os / 2;
-    const int lo = h.support - ts, hi = h.support + ts;
+    const int ks = 2 * ts + 1;
     const long long os = h.os, op = h.os / 2;
     const cplx<double>* khp = kh + size_t(p) * h.kh_stride;
     auto value = [&](int i, int j) -> cplx<double> {
-        const long long cx = -(long long)ts * os + op - x + (long long)(j - lo) * os;
-        const long long cy = -(long long)ts * os + op - yy + (long long)(i - lo) * os;
+        const long long cx = -(long long)ts * os + op - x + (long long)j * os;
+        const long long cy = -(long long)ts * os + op - yy + (long long)i * os;
         const long long dcx = cx < 0 ? -cx : cx, dcy = cy < 0 ? -cy : cy;
         const long long vi = dcx > dcy ? dcy * ko - ((dcy * (dcy + 1)) >> 1) + dcx : dcx * ko - ((dcx * (dcx + 1)) >> 1) + dcy;
         return khp[vi];
@@ -2044,8 +2062,7 @@ __global__ __launch_bounds__(256) void wk_hankel_extract_kernel(HankelArgs h, co
     double sum = 0.0;
     for (int e = threadIdx.x; e < ks * ks; e += 256) {
         const int i = e % ks, j = e / ks;
-        if (i >= lo && i <= hi && j >= lo && j <= hi)
-            sum += value(i, j).x;
+        sum += value(i, j).x;
     }
     red[threadIdx.x] = sum;
     __syncthreads();
@@ -2055,10 +2072,10 @@ __global__ __launch_bounds__(256) void wk_hankel_extract_kernel(HankelArgs h, co
         __syncthreads();
     }
     const double ksum = red[0];
-    cplx<KT>* out = cache + (size_t(p) * cs * cs + blockIdx.x) * size_t(ks) * kw;
-    for (int e = threadIdx.x; e < ks * kw; e += 256) {
-        const int i = e % ks, j = e / ks - WPAD;
-        if (j < 0 || j >= ks || i < lo || i > hi || j < lo || j > hi) {
+    cplx<KT>* out = cache + (size_t(p) * cs * cs + blockIdx.x) * w_slot(2 * h.support + 1);
+    for (int e = threadIdx.x; e < int(w_slot(ks)); e += 256) {
+        const int i = (e - 1) % (ks + 1), j = (e - 1) / (ks + 1) - WPAD;
+        if (e == 0 || i == ks || j < 0 || j >= ks) {
             out[e] = { KT(0), KT(0) };
             continue;
         }
@@ -2102,18 +2119,15 @@ __global__ __launch_bounds__(256) void wk_extract_kernel(const cplx<double>* con
 {
     __shared__ double red[256];
     conv += size_t(blockIdx.y) * arr * arr;
-    const int cs = (os / 2) * 2 + 1;
+    const int cs = os / 2 + 1;
     const int x = blockIdx.x % cs, y = blockIdx.x / cs;
-    const int ks = 2 * support + 1;
     const int sp = plane_support ? plane_support[blockIdx.y] : support;
-    const int lo = support - sp, hi = support + sp;
+    const int ks = 2 * sp + 1;
     const long long ctr = arr / 2, op = os / 2;
-    const long long oc = ctr - (long long)support * os + op;
+    const long long oc = ctr - (long long)sp * os + op;
     double sum = 0.0;
     for (int e = threadIdx.x; e < ks * ks; e += 256) {
         const int i = e % ks, j = e / ks;
-        if (i < lo || i > hi || j < lo || j > hi)
-            continue;
         const long long cxi = (oc - x + (long long)j * os + ctr) % arr;
         const long long cyi = (oc - y + (long long)i * os + ctr) % arr;
         sum += conv[cxi + cyi * arr].x;
@@ -2126,11 +2140,10 @@ __global__ __launch_bounds__(256) void wk_extract_kernel(const cplx<double>* con
         __syncthreads();
     }
     const double inv = 1.0 / red[0];
-    const int kw = ks + 2 * WPAD;
-    cplx<KT>* out = cache + (size_t(blockIdx.y) * cs * cs + blockIdx.x) * ks * kw;
-    for (int e = threadIdx.x; e < ks * kw; e += 256) {
-        const int i = e % ks, j = e / ks - WPAD;
-        if (j < 0 || j >= ks || i < lo || i > hi || j < lo || j > hi) {
+    cplx<KT>* out = cache + (size_t(blockIdx.y) * cs * cs + blockIdx.x) * w_slot(2 * support + 1);
+    for (int e = threadIdx.x; e < int(w_slot(ks)); e += 256) {
+        const int i = (e - 1) % (ks + 1), j = (e - 1) / (ks + 1) - WPAD;
+        if (e == 0 || i == ks || j < 0 || j >= ks) {
             out[e] = { KT(0), KT(0) };
             continue;
         }
@@ -2141,210 +2154,336 @@ __global__ __launch_bounds__(256) void wk_extract_kernel(const cplx<double>* con
     }
 }
 
-// W-projection tile accumulation without atomics.  The tile's 64 rows are the
-// lanes and its columns are split among the workgroup's eight waves (CPW columns
-// each), so every grid cell belongs to exactly one lane, which keeps the cell's
-// sums in registers.  Every wave walks the tile's entries (staged in LDS) and adds
-// the taps of its own columns.  Per tap (gridder.h:826-861): kval = K * w with K
-// the plane's complex kernel (conjugated for w < 0), grid += vis * kval,
-// beam += kval, summed in FP64 on every grid precision.
+// W-projection tile sums without atomics.  A wave sums 64 rows x W_COLS columns of a
+// tile: its FP64 sums stay in registers and each cell is written once.  Every lane loads
+// 16 bytes of kernel at a time (two rows of FP32 values, one of FP64), and the lanes of
+// each 16 rows take entries of their own from a queue of those that touch them, so a
+// footprint of ks rows wastes at most 15 rows at either end (one entry across all 64 rows
+// used half of the lanes at 65 taps).  Per tap (gridder.h:826-861): kval = K w with K the
+// plane's complex kernel, conjugated for w < 0, grid += vis kval, beam += kval, as six
+// FP64 FMAs with the entry's coefficients.
 //
-// Phases: the binning blocks hold the visibilities in |w| order, so a run of
-// blocks covers about one w-plane.  One launch per run of blocks (a phase) keeps
-// the W-kernels that all tiles read during the launch to about one plane's
-// cache, which stays in L2, instead of every plane at once.  A phase takes tile
-// t's entries of blocks [b0, b1) (the block cursors of the binning give their
-// range) and continues the FP64 running sums of the phase before (acc), in the
-// same order as one launch over all entries.
+// The waves walk the tile's entries 64 at a time, each by itself, and keep those that
+// touch their cells in LDS, so there is no barrier.  Kernels of mirrored oversampled
+// offsets are stored once and read backwards (the plane's kernel is even): 1.0 MB per FP32
+// plane at 65 taps and oversampling 8.
+//
+// Phases: the entries are in |w| order, and workgroups that start together read the
+// kernels of about the same planes, from L2.  Later ones start over at plane 0 while the
+// others are further on, so a launch covers a run of binning blocks (a phase) of about
+// W_PHASE_BYTES of kernels and continues the FP64 sums of the launch before: with 32
+// planes (33 MB of FP32 kernels) one launch read 66 GB past L2.
+//
+// Measured with N = 4096, 2 M visibilities, 32 planes, 65 taps, FP32: 7.2 ms (12.0 with a
+// lane per row of 64 and 81 kernels per plane), of which 4.3 are vector instructions and
+// as much the 1.2 G cache lines of the kernel reads; with all kernels in L2 it takes 6.8.
+// Truncated kernels (N = 2048, 300 k visibilities of a condensed array, FP64): 0.2 ms against 25,
+// from footprints of each plane's own support and from splitting the heavy tiles.
+constexpr int W_COLS = 8;
+constexpr int W_WAVES = 4;               // waves per workgroup (tiles of 16 columns: 2)
+constexpr int W_KEEP = 128;              // kept entries of a wave: summed above 64
+constexpr uint32_t W_OOB = 0xc0000000u;  // buffer offset past every kernel
+constexpr size_t W_BUFFER_MAX = size_t(1) << 31; // largest kernel cache of the 32-bit buffer offsets
+constexpr double W_PHASE_BYTES = 4.5 * (1 << 20); // 32 planes, 65 taps, FP32: 9.7 ms in one launch, 7.6 at 9 MB, 7.2 at 4.5 MB
+constexpr double W_PHASE_READS = 4e9;    // least kernel bytes read per phase: below, its own 50-100 us cost more
+constexpr int BUF_DWORD3 = 0x00020000;   // raw (untyped) buffer access
+static_assert(W_COLS - 1 <= WPAD, "column runs must stay within the zero padding");
+
 struct WPhase {
-    const uint32_t* bcur = nullptr; // bcur[b * ntiles + t]: entries of tile t in blocks < b (null: whole tile)
+    const uint32_t* bcur = nullptr; // bcur[b * ntiles + t]: entries of tile t in blocks < b (null: one phase)
     const uint32_t* btot = nullptr; // entries of tile t
     int b0 = 0, b1 = 0, nblk = 0;
     int first = 1, last = 1;        // first: sums start at zero; last: write the grids
     cplx<double>* acc_v = nullptr;  // FP64 running sums between phases (rows x N, grid layout)
     cplx<double>* acc_b = nullptr;
 };
-constexpr int WTW = 8;   // waves per W tile workgroup
-constexpr double W_PHASE_BYTES = 6.0 * (1 << 20); // W-kernel cache read per phase (measured best on c3)
 
-__device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
-__device__ __forceinline__ double uni(double x)
-{
-    const unsigned long long b = __double_as_longlong(x);
-    const int lo = __builtin_amdgcn_readfirstlane(int(b & 0xffffffffu)), hi = __builtin_amdgcn_readfirstlane(int(b >> 32));
-    return __longlong_as_double((long long)((unsigned long long)(unsigned)hi << 32 | (unsigned)lo));
-}
+struct alignas(16) WKept {
+    double a, b, w;      // (vis w) re, im and w
+    uint32_t first;      // byte offset of the kernel row of the wave's first row in the run's first column
+    int step;            // bytes to the next column (negative: columns mirrored)
+    int row;             // kernel row of the wave's first row
+    int ks;              // taps per side, negative for the conjugate kernel
+    int sub, pad;        // sub-kernel (BIG)
+};
+struct WaveKeep {
+    WKept e[W_KEEP + 1];             // the last one: no taps
+    uint8_t queue[2][4][W_KEEP];     // per row direction and 16 rows: positions in e
+};
 
-constexpr uint32_t W_OOB = 0x80000000u;
-constexpr int BUF_DWORD3 = 0x00020000; // raw (untyped) buffer access
-
-// One W-kernel value per lane through a range-checked buffer resource over the
-// entry's padded sub-kernel (scalar base, scalar column offset): lanes whose row
-// is outside [0, ks) carry offset W_OOB and read zero without a memory access.
+// 16 bytes of kernel values at an offset of the cache (zero past its end).
 template <typename KT>
-__device__ __forceinline__ cplx<KT> load_kval(const cplx<KT>* sub, int bytes, uint32_t voff, int soff)
+struct KRow {
+    cplx<KT> v[16 / sizeof(cplx<KT>)];
+};
+template <typename KT>
+__device__ __forceinline__ KRow<KT> load_krow(__amdgpu_buffer_rsrc_t rs, uint32_t voff)
 {
-    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)sub, (short)0, bytes, BUF_DWORD3);
-    if constexpr (std::is_same<KT, double>::value) {
-        typedef unsigned int u4 __attribute__((ext_vector_type(4)));
-        const u4 v = __builtin_amdgcn_raw_buffer_load_b128(rs, voff, soff, 0);
-        return { __longlong_as_double((long long)((unsigned long long)v.y << 32 | v.x)),
-            __longlong_as_double((long long)((unsigned long long)v.w << 32 | v.z)) };
-    } else {
-        typedef unsigned int u2 __attribute__((ext_vector_type(2)));
-        const u2 v = __builtin_amdgcn_raw_buffer_load_b64(rs, voff, soff, 0);
-        return { __uint_as_float(v.x), __uint_as_float(v.y) };
+    typedef unsigned int u4 __attribute__((ext_vector_type(4)));
+    const u4 v = __builtin_amdgcn_raw_buffer_load_b128(rs, voff, 0, 0);
+    if constexpr (std::is_same<KT, double>::value)
+        return { { { __longlong_as_double((long long)((unsigned long long)v.y << 32 | v.x)),
+            __longlong_as_double((long long)((unsigned long long)v.w << 32 | v.z)) } } };
+    else
+        return { { { __uint_as_float(v.x), __uint_as_float(v.y) }, { __uint_as_float(v.z), __uint_as_float(v.w) } } };
+}
+
+// -x where `sign` is negative
+__device__ __forceinline__ double flip_if(double x, int sign)
+{
+    return __longlong_as_double(__double_as_longlong(x) ^ ((unsigned long long)(uint32_t(sign) & 0x80000000u) << 32));
+}
+
+// BIG: kernel caches past the reach of a buffer's 32-bit offsets, by 64-bit addresses
+// (rows outside the kernel read its zero padding).
+template <typename T, typename KT, bool BEAM, bool BIG>
+__global__ __launch_bounds__(64 * W_WAVES) void grid_wtiles_kernel(GridGeom g, Entry* entries,
+    const uint32_t* __restrict__ offsets, uint32_t cap, const cplx<KT>* __restrict__ cache, uint32_t cache_bytes,
+    cplx<T>* __restrict__ vgrid, cplx<T>* __restrict__ bgrid, int ext_host, WPhase ph)
+{
+    constexpr int SZ = int(sizeof(cplx<KT>));
+    constexpr int RPL = 16 / SZ, CPL = W_COLS / RPL; // rows and columns of a lane
+    constexpr int LS = 16 / RPL;                     // lanes per 16 rows
+    __shared__ WaveKeep keeps[W_WAVES];
+    const int N = g.N, waves = int(blockDim.x) / 64, strips = g.tc / (W_COLS * waves);
+    const int ntiles = g.tiles_r * g.tiles_c;
+    const Split sp = split_view(entries, cap, offsets[ntiles], ext_host, g.tc, 4);
+    uint32_t chunk = 0;
+    const int unit = int(blockIdx.x) / strips;
+    int t = unit - ext_host;
+    if (t < 0) {
+        if (!sp.hdr || uint32_t(unit) >= sp.hdr[0])
+            return;
+        t = int(sp.ext[2 * unit]);
+        chunk = sp.ext[2 * unit + 1];
     }
-}
-
-__device__ __forceinline__ double flip_if(double x, bool neg)
-{
-    return neg ? -x : x;
-}
-
-template <typename T, typename KT, int CPW, int EB>
-__global__ __launch_bounds__(WTW * 64) void grid_wtiles_kernel(GridGeom g, const Entry* __restrict__ entries,
-    const uint32_t* __restrict__ offsets, int ostride, uint32_t cap, const cplx<KT>* __restrict__ cache,
-    cplx<T>* __restrict__ vgrid, cplx<T>* __restrict__ bgrid, WPhase ph)
-{
-    const int ks = g.ks, s = g.s, N = g.N;
-    const int t = blockIdx.x;
-    const int rt = t % g.tiles_r, ct = t / g.tiles_r;
-    const int r0 = rt * TILE_R, c0 = ct * g.tc;
-    const int wave = uni(int(threadIdx.x >> 6)), lane = threadIdx.x & 63;
-    const int r = r0 + lane;
-    const int wc = c0 + wave * CPW; // first grid column of this wave (uniform: the loads' buffer resources are scalar)
-    uint32_t eb = offsets[size_t(t) * ostride], ee = offsets[size_t(t + 1) * ostride];
+    const uint32_t tb = min(offsets[t], cap), te = min(offsets[t + 1], cap);
+    const uint32_t ch = sp.hdr ? sp.hdr[2] : 0xffffffffu;
+    const bool split = te - tb > ch;
+    uint32_t eb = tb, ee = te;
+    bool fresh = ph.first; // sums start at zero
+    if (split) {
+        eb = tb + chunk * ch;
+        ee = min(te, eb + ch);
+    }
     if (ph.bcur) {
-        const size_t nt = size_t(g.tiles_r) * g.tiles_c;
-        const uint32_t base = eb;
-        eb = base + (ph.b0 < ph.nblk ? ph.bcur[size_t(ph.b0) * nt + t] : ph.btot[t]);
-        ee = base + (ph.b1 < ph.nblk ? ph.bcur[size_t(ph.b1) * nt + t] : ph.btot[t]);
+        const uint32_t p0 = tb + (ph.b0 < ph.nblk ? ph.bcur[size_t(ph.b0) * ntiles + t] : ph.btot[t]);
+        const uint32_t p1 = tb + (ph.b1 < ph.nblk ? ph.bcur[size_t(ph.b1) * ntiles + t] : ph.btot[t]);
+        if (split)
+            fresh = eb >= p0;
+        eb = max(eb, min(p0, te));
+        ee = min(ee, min(p1, te));
     }
-    eb = uni(int(min(eb, cap)));
-    ee = uni(int(min(ee, cap)));
     // FP32 grids take the sums at the last phase; FP64 grids are their own running sums
     constexpr bool narrow = !std::is_same<T, double>::value;
-    if (!ph.first && !(narrow && ph.last) && eb >= ee)
-        return; // no entry of this tile in the phase: its sums stay as they are
-    const bool cell = r < g.rows;
-    double ar[CPW], ai[CPW], br[CPW], bi[CPW];
+    if (eb >= ee && (split || !(ph.first || (narrow && ph.last))))
+        return; // no entry in the phase: the sums stay as they are
+    const int rt = t % g.tiles_r, ct = t / g.tiles_r;
+    const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)), lane = threadIdx.x & 63;
+    const int kk = (lane / LS) & 3;                      // the lane's 16 rows
+    const int lr = 16 * kk + RPL * (lane % LS);          // its first row
+    const int lh = CPL * (lane / (4 * LS));              // its first column among the wave's
+    const int lw = W_COLS * (int(blockIdx.x) % strips * waves + wave);
+    const int rb = rt * TILE_R, cb = ct * g.tc + lw;     // the wave's cells
+    const uint32_t slot = uint32_t(w_slot(g.ks));
+    WaveKeep& keep = keeps[wave];
+    // the running sums of cell (row lr + v, column lh + u): grid or slot elements
+    double* slot_out = nullptr;
+    if (split) {
+        uint32_t lo = 0, hi = sp.hdr[1] - 1; // the tile's record among the split tiles
+        while (lo < hi) {
+            const uint32_t mid = (lo + hi) / 2;
+            if (sp.spl[3 * mid] < uint32_t(t))
+                lo = mid + 1;
+            else
+                hi = mid;
+        }
+        slot_out = sp.part + size_t(sp.spl[3 * lo + 1] + chunk) * (4 * g.tc * TILE_R) + (lw + lh) * TILE_R + lr;
+    }
+    const int plane = g.tc * TILE_R;
+    double ar[8], ai[8], br[8], bi[8];
 #pragma unroll
-    for (int u = 0; u < CPW; u++) {
-        ar[u] = ai[u] = br[u] = bi[u] = 0.0;
-        const int c = wc + u;
-        if (!ph.first && cell && c < N && c < c0 + g.tc) {
-            const size_t o = size_t(r) + size_t(c) * g.rows;
-            const cplx<double> v = ph.acc_v[o];
-            ar[u] = v.x;
-            ai[u] = v.y;
-            if (g.beam) {
-                const cplx<double> b = ph.acc_b[o];
-                br[u] = b.x;
-                bi[u] = b.y;
+    for (int k = 0; k < 8; k++) {
+        const int v = k % RPL, u = k / RPL;
+        ar[k] = ai[k] = br[k] = bi[k] = 0.0;
+        if (fresh)
+            continue;
+        if (split) {
+            const double* o = slot_out + u * TILE_R + v;
+            ar[k] = o[0];
+            ai[k] = o[plane];
+            if (BEAM) {
+                br[k] = o[2 * plane];
+                bi[k] = o[3 * plane];
+            }
+        } else if (rb + lr + v < g.rows && cb + lh + u < N) {
+            const size_t o = size_t(rb + lr + v) + size_t(cb + lh + u) * g.rows;
+            ar[k] = ph.acc_v[o].x;
+            ai[k] = ph.acc_v[o].y;
+            if (BEAM) {
+                br[k] = ph.acc_b[o].x;
+                bi[k] = ph.acc_b[o].y;
             }
         }
     }
-    static_assert(CPW - 1 <= WPAD, "column runs must stay within the zero padding");
-    const int kw = ks + 2 * WPAD;
-    const int sub_bytes = int(size_t(ks) * kw * sizeof(cplx<KT>));
-    const int col_bytes = int(ks * sizeof(cplx<KT>));
-    // EB entries at a time (scalar loads; every value uniform): all their kernel
-    // values are loaded before any is summed
-    for (uint32_t e0 = eb; e0 < ee; e0 += EB) {
-        cplx<KT> kv[EB][CPW]; // in the cache precision until summed
-        double ca[EB], cb[EB], cw[EB];
-        bool conj[EB], hit[EB];
-        // the batch's entries: their scalar loads go out together (the empty asm
-        // takes every field in scalar registers, so one wait covers the batch)
-        Entry ent[EB];
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)cache, (short)0, cache_bytes, BUF_DWORD3);
+
+    int cnt[2][4] = {}, kept = 0;
+    // one queue of each 16 rows, up to the longest one's length; MIRROR: the kernel's rows
+    // run backwards, and so do the rows of a load
+    auto sum_queues = [&](auto MIRROR) {
+        constexpr bool MR = decltype(MIRROR)::value;
+        const int* c = cnt[MR];
+        const int n = max(max(c[0], c[1]), max(c[2], c[3]));
+        const int mine = kk == 0 ? c[0] : (kk == 1 ? c[1] : (kk == 2 ? c[2] : c[3]));
+        const uint8_t* queue = keep.queue[MR][kk];
+        int nx = 0 < mine ? queue[0] : W_KEEP;
+        for (int q = 0; q < n; q++) {
+            const WKept e = keep.e[nx];
+            nx = q + 1 < mine ? queue[q + 1] : W_KEEP;
+            const int ks = e.ks < 0 ? -e.ks : e.ks;
+            // rows -1 and ks are zeros of the padding
+            const bool row = unsigned(e.row + lr + RPL - 1) < unsigned(ks + RPL - 1);
+            const int off = (MR ? -lr - (RPL - 1) : lr) * SZ + lh * e.step;
+            KRow<KT> kv[CPL];
+            if constexpr (BIG) {
+                const char* p = reinterpret_cast<const char*>(cache + size_t(e.sub) * slot);
 #pragma unroll
-        for (int b = 0; b < EB; b++)
-            ent[b] = entries[min(e0 + b, ee - 1)];
-#pragma unroll
-        for (int b = 0; b < EB; b++)
-            asm volatile("" ::"s"(ent[b].gx), "s"(ent[b].gy), "s"(ent[b].cp), "s"(ent[b].idx), "s"(ent[b].vr),
-                "s"(ent[b].vi), "s"(ent[b].w));
-#pragma unroll
-        for (int b = 0; b < EB; b++) {
-            const Entry& en = ent[b];
-            conj[b] = en.cp < 0;
-            ca[b] = en.vr;
-            cb[b] = en.vi;
-            cw[b] = en.w;
-            // kernel column of the wave's first column, mod N; the wave's columns run
-            // on from it and wrap past N
-            int j0 = wc - (en.gx - s);
-            j0 = j0 < 0 ? j0 + N : (j0 >= N ? j0 - N : j0);
-            const bool wrap = j0 > N - CPW;
-            // byte offset of each column in the padded sub-kernel: the run
-            // j0 - (wrap ? N : 0) + u (columns outside [0, ks) are padding zeros),
-            // or, when the run wraps inside the kernel (grids narrower than
-            // ks + CPW - 1), column by column with the first padding column for
-            // columns outside
-            int soff[CPW];
-            bool any;
-            if (!(wrap && j0 < ks)) {
-                const int jv = wrap ? j0 - N : j0;
-                any = jv < ks && jv + CPW > 0;
-#pragma unroll
-                for (int u = 0; u < CPW; u++)
-                    soff[u] = (jv + u + WPAD) * col_bytes;
+                for (int u = 0; u < CPL; u++)
+                    kv[u] = row ? *reinterpret_cast<const KRow<KT>*>(p + (int(e.first) + off + u * e.step)) : KRow<KT>{};
             } else {
-                any = true;
+                uint32_t v = row ? e.first + uint32_t(off) : W_OOB;
 #pragma unroll
-                for (int u = 0; u < CPW; u++) {
-                    const int j = j0 + u >= N ? j0 + u - N : j0 + u;
-                    soff[u] = (j < ks ? j + WPAD : 0) * col_bytes;
+                for (int u = 0; u < CPL; u++) {
+                    kv[u] = load_krow<KT>(rs, v);
+                    v += uint32_t(e.step);
                 }
             }
-            hit[b] = e0 + b < ee && any;
-            if (!hit[b])
-                continue;
-            // kernel row of my grid row: direct, or wrapped from >= N (rows < 0 are skipped)
-            int i = r - (en.gy - s);
-            if (i < 0)
-                i += N;
-            const uint32_t voff = (i < ks && cell) ? uint32_t(i) * uint32_t(sizeof(cplx<KT>)) : W_OOB;
-            const cplx<KT>* K = cache + size_t(uint32_t(en.idx)) * (size_t(ks) * kw);
+            const double a = e.a, b = e.b, w = e.w;
+            const double sa = flip_if(a, e.ks), sb = flip_if(b, e.ks), sw = flip_if(w, e.ks);
 #pragma unroll
-            for (int u = 0; u < CPW; u++)
-                kv[b][u] = load_kval<KT>(K, sub_bytes, voff, soff[u]);
-        }
-#pragma unroll
-        for (int b = 0; b < EB; b++) {
-            if (!hit[b])
-                continue;
-            // per tap (gridder.h:826-861): kval = K w, conjugated for w < 0; grid += vis kval,
-            // beam += kval, as FMAs with the entry's coefficients (vis w, w) and their signs
-            const double sa = flip_if(ca[b], conj[b]), sb = flip_if(cb[b], !conj[b]), sw = flip_if(cw[b], conj[b]);
-#pragma unroll
-            for (int u = 0; u < CPW; u++) {
-                const double kr = double(kv[b][u].x), ki = double(kv[b][u].y);
-                ar[u] = fma(ca[b], kr, ar[u]);
-                ar[u] = fma(sb, ki, ar[u]);
-                ai[u] = fma(cb[b], kr, ai[u]);
-                ai[u] = fma(sa, ki, ai[u]);
-                br[u] = fma(cw[b], kr, br[u]);
-                bi[u] = fma(sw, ki, bi[u]);
+            for (int k = 0; k < 8; k++) {
+                const cplx<KT> K = kv[k / RPL].v[MR ? RPL - 1 - k % RPL : k % RPL];
+                const double kr = double(K.x), ki = double(K.y);
+                ar[k] = fma(a, kr, ar[k]);
+                ar[k] = fma(-sb, ki, ar[k]);
+                ai[k] = fma(b, kr, ai[k]);
+                ai[k] = fma(sa, ki, ai[k]);
+                if (BEAM) {
+                    br[k] = fma(w, kr, br[k]);
+                    bi[k] = fma(sw, ki, bi[k]);
+                }
             }
         }
+    };
+    auto sum_kept = [&]() {
+        // the wave's LDS accesses complete in order
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        sum_queues(std::integral_constant<bool, false>{});
+        sum_queues(std::integral_constant<bool, true>{});
+        kept = 0;
+#pragma unroll
+        for (int k = 0; k < 4; k++)
+            cnt[0][k] = cnt[1][k] = 0;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+
+    if (eb < ee) {
+        if (lane == 0) {
+            WKept none{};
+            none.row = -(1 << 20);
+            none.ks = 1;
+            keep.e[W_KEEP] = none;
+        }
+        int ngx, ngy, ncp, nidx;
+        double nvr, nvi, nw;
+        auto fetch = [&](uint32_t e) {
+            const Entry* p = entries + min(e + uint32_t(lane), ee - 1);
+            ngx = p->gx;
+            ngy = p->gy;
+            ncp = p->cp;
+            nidx = p->idx;
+            nvr = p->vr;
+            nvi = p->vi;
+            nw = p->w;
+        };
+        fetch(eb);
+        const unsigned long long below = (1ull << lane) - 1ull;
+        for (uint32_t e0 = eb; e0 < ee; e0 += 64) {
+            const int gx = ngx, gy = ngy, cp = ncp, idx = nidx;
+            const double a = nvr, b = nvi, w = nw;
+            const bool valid = e0 + uint32_t(lane) < ee;
+            fetch(e0 + 64);
+            const int s = cp & 127, ks = 2 * s + 1;
+            // the footprint and its wrapped pieces: the cells' rows at +N (rows past N wrap,
+            // rows below 0 are dropped), their columns at +-N
+            const int iraw = rb - (gy - s), jraw = cb - (gx - s);
+            const bool wrapped = valid && (gy + s >= N || gx - s < 0 || gx + s >= N);
+            const int pieces = __ballot(wrapped) ? 6 : 1;
+            for (int p = 0; p < pieces; p++) {
+                const int pr = p & 1, pc = p >> 1;
+                const int i0 = iraw + (pr ? N : 0), j0 = jraw + (pc == 0 ? 0 : (pc == 1 ? N : -N));
+                const bool hit = valid && i0 < ks && i0 > -64 && j0 < ks && j0 > -W_COLS;
+                const unsigned long long mask = __ballot(hit);
+                if (!mask)
+                    continue;
+                const int pos = kept + __popcll(mask & below);
+                const bool mr = (cp >> 30) & 1, mc = (cp >> 29) & 1;
+                if (hit) {
+                    const int jp = (mc ? 2 * s - j0 : j0) + WPAD; // padded column of the run's start
+                    WKept e;
+                    e.a = a;
+                    e.b = b;
+                    e.w = w;
+                    e.first = (BIG ? 0u : uint32_t(idx) * slot * SZ) + uint32_t((1 + jp * (ks + 1) + (mr ? 2 * s - i0 : i0)) * SZ);
+                    e.step = (mc ? -(ks + 1) : ks + 1) * SZ;
+                    e.row = i0;
+                    e.ks = cp < 0 ? -ks : ks;
+                    e.sub = idx;
+                    e.pad = 0;
+                    keep.e[pos] = e;
+                }
+                kept += __popcll(mask);
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    const bool in = hit && i0 + 16 * k < ks && i0 + 16 * k > -16;
+                    const unsigned long long m0 = __ballot(in && !mr), m1 = __ballot(in && mr);
+                    if (in)
+                        keep.queue[mr][k][mr ? cnt[1][k] + __popcll(m1 & below) : cnt[0][k] + __popcll(m0 & below)] = uint8_t(pos);
+                    cnt[0][k] += __popcll(m0);
+                    cnt[1][k] += __popcll(m1);
+                }
+                if (kept > W_KEEP - 64)
+                    sum_kept();
+            }
+        }
+        if (kept)
+            sum_kept();
     }
-    if (cell) {
 #pragma unroll
-        for (int u = 0; u < CPW; u++) {
-            const int c = wc + u;
-            if (c < N && c < c0 + g.tc) {
-                const size_t o = size_t(r) + size_t(c) * g.rows;
-                if (narrow && !ph.last) {
-                    ph.acc_v[o] = { ar[u], ai[u] };
-                    if (g.beam)
-                        ph.acc_b[o] = { br[u], bi[u] };
-                } else {
-                    vgrid[o] = { T(ar[u]), T(ai[u]) };
-                    if (g.beam)
-                        bgrid[o] = { T(br[u]), T(bi[u]) };
-                }
+    for (int k = 0; k < 8; k++) {
+        const int v = k % RPL, u = k / RPL;
+        const int r = rb + lr + v, c = cb + lh + u;
+        if (split) {
+            double* o = slot_out + u * TILE_R + v;
+            o[0] = ar[k];
+            o[plane] = ai[k];
+            if (BEAM) {
+                o[2 * plane] = br[k];
+                o[3 * plane] = bi[k];
+            }
+        } else if (r < g.rows && c < N) {
+            const size_t o = size_t(r) + size_t(c) * g.rows;
+            if (narrow && !ph.last) {
+                ph.acc_v[o] = { ar[k], ai[k] };
+                if (BEAM)
+                    ph.acc_b[o] = { br[k], bi[k] };
+            } else {
+                vgrid[o] = { T(ar[k]), T(ai[k]) };
+                if (BEAM)
+                    bgrid[o] = { T(br[k]), T(bi[k]) };
             }
         }
     }
@@ -2501,7 +2640,7 @@ static GridGeom make_geom(const GridderArgs& a, size_t n, bool beam, KernelFn& k
     g.bpack = beam && a.beam_packed ? 1 : 0;
     STP_REQUIRE(!g.bpack || (!wproj && a.halfplane), "a packed real beam grid needs the half-plane grid without W-projection");
     g.tiles_r = int(div_up(g.rows, TILE_R));
-    g.tc = a.tile_cols > 0 ? a.tile_cols : TILE_C;
+    g.tc = a.tile_cols > 0 ? a.tile_cols : (wproj ? W_TILE_C : TILE_C);
     STP_REQUIRE(g.tc == 16 || g.tc == 32 || g.tc == 64, "tile width must be 16, 32 or 64 columns");
     g.tiles_c = int(div_up(N, g.tc));
     g.scale = a.uv_scale;
@@ -2582,6 +2721,7 @@ void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const doubl
     // kernels (half the bytes the W tile kernel reads per tap) on the FP32 paths
     using KT = T;
     cplx<KT>* wcache = nullptr;
+    size_t wcache_bytes = 0;
     if (wproj) {
         const int P = int(a.wproj.num_wplanes);
         // 1. |w| order
@@ -2654,7 +2794,9 @@ void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const doubl
                                                  : dev_table(ctx, key, img_dom_kernel(kf, size_t(workarea), false, a.analytic_gcf));
         // planes in groups of PB: one fill, one batched 2-D c2c and one extraction per
         // group, the image-domain arrays of a group at most 256 MB each
-        const size_t per_plane = size_t(cs) * cs * size_t(g.ks) * (g.ks + 2 * WPAD);
+        const int csw = os / 2 + 1; // offsets per axis without their mirror images
+        const size_t per_plane = size_t(csw) * csw * w_slot(g.ks);
+        wcache_bytes = sizeof(cplx<KT>) * per_plane * P;
         STP_REQUIRE(size_t(P) * cs * cs < (size_t(1) << 31), "too many W sub-kernels (planes x oversampling^2)");
         wcache = (cplx<KT>*)ws_get(ctx, "w_cache", sizeof(cplx<KT>) * per_plane * P);
         // kernel_trunc_perc > 0: every plane grids with its own truncated support
@@ -2691,6 +2833,7 @@ void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const doubl
             int* psup = (int*)ws_get(ctx, "w_psupport", sizeof(int) * P);
             launch(ctx, "w_hankel_profile", wk_hankel_profile_kernel, dim3(unsigned(P)), dim3(256), 0, h, d_aa,
                 (const double*)w_plane, prof);
+            g.psup = psup;
             launch(ctx, "w_hankel_transform", wk_hankel_transform_kernel, dim3(unsigned(div_up(h.n, 256)), unsigned(P)),
                 dim3(256), 0, h, tab, (const cplx<double>*)prof, yv);
             launch(ctx, "w_hankel_spline", wk_hankel_spline_kernel, dim3(unsigned(P)), dim3(64), 0, h, (const cplx<double>*)yv,
@@ -2698,7 +2841,7 @@ void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const doubl
             launch(ctx, "w_hankel_quad", wk_hankel_quad_kernel,
                 dim3(unsigned(std::min<long long>(1024, div_up((long long)h.kh_stride, 256))), unsigned(P)), dim3(256), 0, h,
                 (const cplx<double>*)yv, (const double*)coef, (const int*)psup, kh);
-            launch(ctx, "w_kernel_extract", wk_hankel_extract_kernel<KT>, dim3(unsigned(cs * cs), unsigned(P)), dim3(256), 0,
+            launch(ctx, "w_kernel_extract", wk_hankel_extract_kernel<KT>, dim3(unsigned(csw * csw), unsigned(P)), dim3(256), 0,
                 h, (const cplx<double>*)kh, (const int*)psup, 0, wcache);
         } else {
             const size_t arr2 = size_t(arr) * arr;
@@ -2706,6 +2849,7 @@ void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const doubl
             cplx<double>* comb = (cplx<double>*)ws_get(ctx, "w_comb", sizeof(cplx<double>) * arr2 * PB);
             cplx<double>* conv = (cplx<double>*)ws_get(ctx, "w_conv", sizeof(cplx<double>) * arr2 * PB);
             int* psup = trunc ? (int*)ws_get(ctx, "w_psupport", sizeof(int) * P) : nullptr;
+            g.psup = psup;
             for (int p0 = 0; p0 < P; p0 += PB) {
                 const int nb = std::min(PB, P - p0);
                 launch(ctx, "w_kernel_fill", wk_fill_kernel, dim3(unsigned(div_up(arr2, 256)), unsigned(nb)), dim3(256), 0, comb,
@@ -2714,7 +2858,7 @@ void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const doubl
                 if (trunc)
                     launch(ctx, "w_kernel_trunc", wk_trunc_kernel, dim3(div_up(nb, 64)), dim3(64), 0, (const cplx<double>*)conv, arr,
                         os, g.s, a.wproj.kernel_trunc_perc / 100.0, nb, psup + p0);
-                launch(ctx, "w_kernel_extract", wk_extract_kernel<KT>, dim3(unsigned(cs * cs), unsigned(nb)), dim3(256), 0,
+                launch(ctx, "w_kernel_extract", wk_extract_kernel<KT>, dim3(unsigned(csw * csw), unsigned(nb)), dim3(256), 0,
                     (const cplx<double>*)conv, arr, os, g.s, (const int*)(trunc ? psup + p0 : nullptr),
                     wcache + size_t(p0) * per_plane);
             }
@@ -2734,7 +2878,7 @@ void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const doubl
         const size_t hist_bytes = sizeof(uint32_t) * size_t(ntiles);
         HIP_CHECK(hipFuncSetAttribute((const void*)grid_bin_count_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, int(hist_bytes)));
         HIP_CHECK(hipFuncSetAttribute((const void*)grid_bin_scatter_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, int(hist_bytes)));
-        ext_host = mfma ? split_extra_max(n) : 0;
+        ext_host = wproj ? split_extra_max(n, W_SPLIT_MIN) : (mfma ? split_extra_max(n) : 0);
         launch(ctx, "grid_count", grid_bin_count_kernel, dim3(unsigned(nblk)), dim3(BWG), hist_bytes, g, d_uv, d_vis, d_w, counts,
             wpart);
         launch(ctx, "grid_colscan", bin_colscan_kernel, dim3(div_up(ntiles, 64)), dim3(1024), 0, counts, int(nblk), int(ntiles),
@@ -2759,20 +2903,15 @@ void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const doubl
         ostride = 1;
     }
     if (wproj) {
-        // eight waves split the tile's columns: 2, 4 or 8 columns per wave; 4 entries'
-        // kernel values in flight per lane
-        // eight waves split the tile's columns (2, 4 or 8 columns per wave); two
-        // entries' kernel values in flight per lane (more registers cost occupancy)
-        auto kern = g.tc == 16 ? grid_wtiles_kernel<T, KT, 2, 2>
-                               : (g.tc == 32 ? grid_wtiles_kernel<T, KT, 4, 2> : grid_wtiles_kernel<T, KT, 8, 2>);
-        // phases whose W-kernels (about 6 MB of cache each: one FP64 plane, two FP32
-        // planes) are read by all tiles while mostly held in L2
-        const int P = int(a.wproj.num_wplanes);
-        const double plane_bytes = double(cs) * cs * g.ks * (g.ks + 2 * WPAD) * sizeof(cplx<KT>);
-        int nph = bcur ? int(std::min<double>(double(nblk), std::ceil(double(P) * plane_bytes / W_PHASE_BYTES))) : 1;
-        if (a.w_phases > 0)
-            nph = bcur ? std::min(a.w_phases, int(nblk)) : 1;
-        nph = std::max(1, nph);
+        const bool big = wcache_bytes > W_BUFFER_MAX;
+        const int wv = std::min(W_WAVES, g.tc / W_COLS);
+        auto kern = big ? (g.beam ? grid_wtiles_kernel<T, KT, true, true> : grid_wtiles_kernel<T, KT, false, true>)
+                        : (g.beam ? grid_wtiles_kernel<T, KT, true, false> : grid_wtiles_kernel<T, KT, false, false>);
+        // truncated supports are not known here, and usually small: one phase
+        int nph = 1;
+        if (bcur && !g.psup)
+            nph = int(std::max(1.0, std::min({ double(nblk), std::ceil(double(wcache_bytes) / W_PHASE_BYTES),
+                double(n) * g.ks * g.ks * sizeof(cplx<KT>) / W_PHASE_READS })));
         WPhase ph;
         if (nph > 1) {
             ph.bcur = bcur;
@@ -2792,8 +2931,9 @@ void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const doubl
             ph.b1 = int(size_t(f + 1) * nblk / nph);
             ph.first = f == 0;
             ph.last = f == nph - 1;
-            launch(ctx, "grid_wtiles", kern, dim3(ntiles), dim3(WTW * 64), 0, g, (const Entry*)entries, offsets, ostride, cap,
-                (const cplx<KT>*)wcache, d_vis_grid, d_sampling_grid, ph);
+            launch(ctx, "grid_wtiles", kern, dim3(unsigned(ntiles + ext_host) * unsigned(g.tc / (W_COLS * wv))),
+                dim3(unsigned(64 * wv)), 0, g, entries, offsets, cap, (const cplx<KT>*)wcache,
+                uint32_t(big ? 0 : wcache_bytes), d_vis_grid, d_sampling_grid, ext_host, ph);
         }
     } else {
         STP_REQUIRE(a.kernel_exact || cs * g.ks <= KV_DOUBLES, "oversampled kernel table too large");

@@ -102,10 +102,10 @@ extern "C" uint64_t stp_job_device_bytes(const stp_job* j)
     b += 21 * I * I + S * I * I + (uint64_t(10) << 20);
     if (wproj) {
         const uint64_t os = std::max<uint32_t>(1, (p.oversampling >> 1) << 1);
-        const uint64_t cs = (os / 2) * 2 + 1;
+        const uint64_t cs = os / 2 + 1;         // oversampled offsets per axis, mirror images shared
         const uint64_t P = j->w_proj.num_wplanes;
         b += 26 * n + 16 * n;                   // sort keys, indices, flags, scan, plane ids
-        b += P * cs * cs * ks * (ks + 2 * stp_hip::W_KERNEL_PAD_COLS) * 16; // W-kernel caches (complex FP64, padded)
+        b += P * cs * cs * ((ks + 1) * (ks + 2 * stp_hip::W_KERNEL_PAD_COLS) + 1) * 16; // W-kernel caches (complex FP64, padded)
         if (S == 4)
             b += 2 * rows * N * 16;             // FP64 running sums between the W tile phases
         // work array (workarea * oversampling, gridder.h:467-486) for the W-kernel FFTs

@@ -172,3 +172,32 @@ def test_gpu_wproj_c3_full_size(gpu, c3_case, precision, tol):
     e_i, e_b = peak_rel_err(img, oimg), peak_rel_err(beam, obeam)
     print(f"c3 precision {precision}: image err {e_i:.3e}, beam err {e_b:.3e}", flush=True)
     assert e_i < tol and e_b < tol
+
+
+@pytest.mark.parametrize("N,n,planes,support,scale,beam,prec,tol", [
+    (64, 2_000, 3, 15, 0.5, True, capi.PRECISION_FP64, TOL),      # footprints that wrap onto their tile twice
+    (128, 257, 2, 3, 1.0, True, capi.PRECISION_FP64, TOL),        # one more entry than the least chunk
+    (256, 20_000, 5, 8, 0.05, True, capi.PRECISION_FP64, TOL),    # heavy tiles, in chunks
+    (256, 20_000, 5, 8, 0.05, True, capi.PRECISION_FP32C, 1e-4),
+    (256, 20_000, 5, 31, 0.05, False, capi.PRECISION_FP64, TOL),
+    (512, 60_000, 9, 40, 0.8, True, capi.PRECISION_FP32C, 1e-4),  # several phases
+])
+def test_gpu_wproj_tile_sums(gpu, orc, N, n, planes, support, scale, beam, prec, tol):
+    snap = simdata.snapshot(N, 20.0, n, 4, seed=700 + n, field_frac=0.5, w_max=300.0)
+    snap["uvw"][:, :2] *= scale
+    wp = capi.wproj_pars(planes, support)
+    img, bm, oimg, obeam = _wcase(gpu, orc, snap, N, 20.0, wp, precision=prec, generate_beam=beam)
+    assert peak_rel_err(img, oimg) < tol
+    if beam:
+        assert peak_rel_err(bm, obeam) < tol
+
+
+def test_gpu_wproj_large_kernel_cache(gpu):
+    """A kernel cache past 2 GB (64-bit addresses, FP64) against the same planes in half the
+    bytes (32-bit offsets, FP32)."""
+    snap = simdata.snapshot(128, 20.0, 6_000, 4, seed=717, field_frac=0.5, w_max=300.0)
+    pars = capi.imager_pars(128, 20.0)
+    wp = capi.wproj_pars(5_400, 12)
+    a = gpu.image_visibilities(snap["vis"], snap["weights"], snap["uvw"], pars, w_proj=wp)
+    b = gpu.image_visibilities(snap["vis"], snap["weights"], snap["uvw"], pars, w_proj=wp, precision=capi.PRECISION_FP32C)
+    assert peak_rel_err(b[0], a[0]) < 1e-5 and peak_rel_err(b[1], a[1]) < 1e-5

@@ -36,9 +36,9 @@ void fft_c2r_2d(stp_ctx* ctx, cplx<T>* grids, int nbatch, int n_rows, int N, con
 template <typename T, typename OT>
 void fft_c2r_2d_real(stp_ctx* ctx, cplx<T>* grids, int nbatch, int N, const OutPtrs<OT>& outs, const NormSpec& ns);
 
-// 2-D c2c of nbatch N x N column-major matrices (contiguous); `data` is
+// 2-D c2c of an N x N column-major matrix; `data` is
 // overwritten, results in `out`.
 template <typename T>
-void fft_c2c_2d(stp_ctx* ctx, cplx<T>* data, cplx<T>* out, int N, bool forward, int nbatch = 1);
+void fft_c2c_2d(stp_ctx* ctx, cplx<T>* data, cplx<T>* out, int N, bool forward);
 
 } // namespace stp_hip

@@ -800,20 +800,19 @@ void fft_c2r_2d_real(stp_ctx* ctx, cplx<T>* grids, int nbatch, int N, const OutP
 }
 
 template <typename T>
-void fft_c2c_2d(stp_ctx* ctx, cplx<T>* data, cplx<T>* out, int N, bool forward, int nbatch)
+void fft_c2c_2d(stp_ctx* ctx, cplx<T>* data, cplx<T>* out, int N, bool forward)
 {
     STP_REQUIRE(N >= 4 && (N & (N - 1)) == 0, "c2c size must be a power of two >= 4");
-    STP_REQUIRE(nbatch >= 1 && nbatch <= 65535, "1 to 65535 arrays per c2c launch");
     const Twiddles& twn = twiddles_for(ctx, N);
     const T* tw = std::is_same<T, double>::value ? (const T*)twn.d : (const T*)twn.f;
     // rows: transform along columns index (u) for every row, in place (four-step)
-    launch_u_passes<T>(ctx, data, nbatch, N, N, size_t(N) * N, tw, !forward);
+    launch_u_passes<T>(ctx, data, 1, N, N, size_t(N) * N, tw, !forward);
     int L1, L2;
     split_len<T>(N, L1, L2);
     switch (N) {
 #define CCASE(LL)                                                                                           \
     case LL:                                                                                                \
-        launch(ctx, "fft_cols_c2c", fft_cols_c2c<T, LL>, dim3(div_up(N, Shape<LL>::NT), nbatch), dim3(WG), 0, \
+        launch(ctx, "fft_cols_c2c", fft_cols_c2c<T, LL>, dim3(div_up(N, Shape<LL>::NT), 1), dim3(WG), 0,     \
             (const cplx<T>*)data, N, N, L1, L2, out, tw, int(!forward));                                    \
         break;
         CCASE(4) CCASE(8) CCASE(16) CCASE(32) CCASE(64) CCASE(128) CCASE(256) CCASE(512) CCASE(1024)
@@ -829,6 +828,6 @@ template void fft_c2r_2d<float, float>(stp_ctx*, cplx<float>*, int, int, int, co
 template void fft_c2r_2d<float, double>(stp_ctx*, cplx<float>*, int, int, int, const OutPtrs<double>&, const NormSpec&);
 template void fft_c2r_2d_real<double, double>(stp_ctx*, cplx<double>*, int, int, const OutPtrs<double>&, const NormSpec&);
 template void fft_c2r_2d_real<float, float>(stp_ctx*, cplx<float>*, int, int, const OutPtrs<float>&, const NormSpec&);
-template void fft_c2c_2d<double>(stp_ctx*, cplx<double>*, cplx<double>*, int, bool, int);
+template void fft_c2c_2d<double>(stp_ctx*, cplx<double>*, cplx<double>*, int, bool);
 
 } // namespace stp_hip

@@ -1533,8 +1533,8 @@ __global__ __launch_bounds__(TWG) void grid_tiles_os_kernel(GridGeom g, const En
 //     boundaries and plane |w| (mean or median) of average_w_planes
 //     (gridder.cpp:68-146) on the device.
 //  3. W-kernels per plane: the image-domain kernel aa(x) aa(y) exp(-2 pi i w (n-1)) / n
-//     on an (workarea * os)^2 array, a forward c2c FFT, and the (os+1)^2 oversampled
-//     (2s+1)^2 kernels cut from it, each normalised by its real sum.
+//     on an (workarea * os)^2 array, its forward 2-D DFT at the frequencies the cuts
+//     read, and the oversampled (2s+1)^2 kernels cut from it, each normalised by its real sum.
 //  4. gridding: the entries of every plane binned by tile together; the tile
 //     kernel reads each entry's complex kernel from its plane's cache, so the grid
 //     is written once for all planes.
@@ -1763,43 +1763,66 @@ __global__ void wplane_ids_kernel(const uint32_t* first, int P, long long n, uin
     plane[k] = uint16_t(lo);
 }
 
-// generate_image_domain_convolution_kernel (aw_projection.cpp:50-111): the
-// array x array image-domain kernel, zero outside the +-workarea/2 corners.
-// blockIdx.y: plane p0 + blockIdx.y, written to array blockIdx.y of comb.
-__global__ void wk_fill_kernel(cplx<double>* comb, int arr, int half, const double* aa, const double* w_plane, int p0,
+// generate_image_domain_convolution_kernel (aw_projection.cpp:50-111): the quadrant
+// q[p + r half] of the image-domain kernel at pixel offsets p, r = 0 .. half - 1 (the kernel
+// is even along both axes and zero beyond).  blockIdx.y: plane p0 + blockIdx.y.
+__global__ void wk_fill_kernel(cplx<double>* quad, int half, const double* aa, const double* w_plane, int p0,
     double scaled_cell)
 {
-    const long long e = (long long)blockIdx.x * 256 + threadIdx.x;
-    if (e >= (long long)arr * arr)
+    const int e = blockIdx.x * 256 + threadIdx.x;
+    if (e >= half * half)
         return;
-    const int p = p0 + int(blockIdx.y);
-    comb += size_t(blockIdx.y) * arr * arr;
-    const int i = int(e % arr), j = int(e / arr);
-    // distance of the sample from the origin, folded: i and arr - i map to px = i
-    const int pi = (i < half) ? i : ((i > arr - half) ? arr - i : -1);
-    const int pj = (j < half) ? j : ((j > arr - half) ? arr - j : -1);
-    cplx<double> v{ 0.0, 0.0 };
-    if (pi >= 0 && pj >= 0) {
-        // combine_2d_kernel_value (aw_projection.cpp:455-474)
-        const double a = aa[half + pi] * aa[half + pj];
-        if (pi == 0 && pj == 0) {
-            v.x = a;
-        } else {
-            const double dx = double(pi) * scaled_cell, dy = double(pj) * scaled_cell;
-            const double r2 = dx * dx + dy * dy;
-            if (r2 >= 1.0) {
-                v.x = a;
-            } else {
-                const double nn = sqrt(1.0 - r2);
-                const double ph = (-2.0 * M_PI) * w_plane[p] * (nn - 1.0);
-                double sn, cs;
-                sincos(ph, &sn, &cs);
-                v.x = ((cs / nn) * aa[half + pi]) * aa[half + pj];
-                v.y = ((sn / nn) * aa[half + pi]) * aa[half + pj];
-            }
+    const int pi = e % half, pj = e / half;
+    // combine_2d_kernel_value (aw_projection.cpp:455-474)
+    const double a = aa[half + pi] * aa[half + pj];
+    cplx<double> v{ a, 0.0 };
+    if (pi != 0 || pj != 0) {
+        const double dx = double(pi) * scaled_cell, dy = double(pj) * scaled_cell;
+        const double r2 = dx * dx + dy * dy;
+        if (r2 < 1.0) {
+            const double nn = sqrt(1.0 - r2);
+            const double ph = (-2.0 * M_PI) * w_plane[p0 + int(blockIdx.y)] * (nn - 1.0);
+            double sn, cs;
+            sincos(ph, &sn, &cs);
+            v.x = ((cs / nn) * aa[half + pi]) * aa[half + pj];
+            v.y = ((sn / nn) * aa[half + pi]) * aa[half + pj];
         }
     }
-    comb[e] = v;
+    quad[size_t(blockIdx.y) * half * half + e] = v;
+}
+
+// One axis of the forward 2-D DFT of the even image-domain kernel (aw_projection.cpp:194),
+// which is a cosine sum over the quadrant:
+//   out[i * ldo + pos] = sum_k c_k x[k * ldx + i] cos(2 pi n(pos) k / arr),  c_0 = 1, c_k = 2,
+// for the output frequencies that the oversampled cuts read: n(pos) = (pos % len) os + pos / len,
+// so that a cut's samples, os apart, lie side by side.  As FP64 matrix products, a wave per
+// 16 x 16 outputs; cos from the twiddle table of arr points.  A quadrant of 64 x 64 and 264
+// frequencies take 22 Mflop per plane; the padded 1024 x 1024 FFT moved 48 MB for it (0.87 ms
+// for 32 planes against 0.06).
+__global__ __launch_bounds__(256) void wk_cosine_kernel(const cplx<double>* x, size_t xstride, int ldx, int ni, int nk,
+    cplx<double>* out, size_t ostride, int npos, int len, int os, const cplx<double>* tw, int arr)
+{
+    const int lane = threadIdx.x & 63, m = lane & 15, kk = lane >> 4;
+    const int ib = 16 * blockIdx.y, jb = 64 * blockIdx.x + 16 * (threadIdx.x >> 6);
+    x += blockIdx.z * xstride;
+    out += blockIdx.z * ostride;
+    const int i = min(ib + m, ni - 1), pos = min(jb + m, npos - 1);
+    const int n = (pos % len) * os + pos / len;
+    double4v re = { 0, 0, 0, 0 }, im = { 0, 0, 0, 0 };
+#pragma unroll 4
+    for (int k0 = 0; k0 < nk; k0 += 4) {
+        const int k = min(k0 + kk, nk - 1);
+        const cplx<double> v = x[size_t(k) * ldx + i];
+        double c = tw[(n * k) & (arr - 1)].x;
+        c = k0 + kk >= nk ? 0.0 : (k == 0 ? c : 2.0 * c);
+        re = __builtin_amdgcn_mfma_f64_16x16x4f64(v.x, c, re, 0, 0, 0);
+        im = __builtin_amdgcn_mfma_f64_16x16x4f64(v.y, c, im, 0, 0, 0);
+    }
+    // lane (m, kk) holds rows i = kk + 4 v, position m of the block
+#pragma unroll
+    for (int v = 0; v < 4; v++)
+        if (ib + kk + 4 * v < ni && jb + m < npos)
+            out[size_t(ib + kk + 4 * v) * npos + jb + m] = { re[v], im[v] };
 }
 
 // Each sub-kernel is stored column-major with WPAD zero columns on both sides, so that the
@@ -2085,72 +2108,70 @@ __global__ __launch_bounds__(256) void wk_hankel_extract_kernel(HankelArgs h, co
 }
 
 // Truncated support of each plane of a batch (aw_projection.cpp:176-179,197-209):
-// the largest s <= support whose sample conv(s * os, 0) exceeds trunc_frac times
-// |conv(0, 0)|.  A plane truncated to 0 (the reference asserts there, gridder.h:584)
-// keeps support 1.
-__global__ void wk_trunc_kernel(const cplx<double>* conv, int arr, int os, int support, double trunc_frac, int nb,
+// the largest s <= support whose sample conv(s * os, 0) (position s of row 0) exceeds
+// trunc_frac times |conv(0, 0)|.  A plane truncated to 0 (the reference asserts there,
+// gridder.h:584) keeps support 1.
+__global__ void wk_trunc_kernel(const cplx<double>* conv, size_t stride, int support, double trunc_frac, int nb,
     int* plane_support)
 {
     const int b = blockIdx.x * 64 + threadIdx.x;
     if (b >= nb)
         return;
-    const cplx<double>* c = conv + size_t(b) * arr * arr;
+    const cplx<double>* c = conv + size_t(b) * stride;
     const double min_value = hypot(c[0].x, c[0].y) * trunc_frac;
-    long long i = min((long long)support * os, (long long)(arr >> 1));
-    while (i > 0) {
-        if (hypot(c[i].x, c[i].y) > min_value)
-            break;
-        i -= os;
-    }
-    plane_support[b] = max(1, min(int(i / os), support));
+    int s = support;
+    while (s > 0 && !(hypot(c[s].x, c[s].y) > min_value))
+        s--;
+    plane_support[b] = max(1, s);
 }
 
-// generate_kernel_cache, non-Hankel branch (aw_projection.cpp:415-443): kernel
-// (cp_x = x, cp_y = y), element (row i, column j) = conv[cxi(x, j) + cyi(y, i) * arr],
-// normalised by the sum of its real parts.  One block per (x, y); blockIdx.y:
-// array blockIdx.y of conv, written to plane blockIdx.y of cache.  With a truncated
-// plane (plane_support non-NULL) the kernel of support s_p sits centred in the
-// (2 support + 1)^2 slot, normalised over its own taps, zero outside: gridding
-// those zeros adds nothing, as the reference's smaller loop adds nothing.
-
+// generate_kernel_cache, non-Hankel branch (aw_projection.cpp:415-443): kernel (x, y) of the
+// oversampled offsets 0 .. os / 2 (the others are these, mirrored), element (row i, column
+// j) = conv at frequencies |(j - s) os + os / 2 - x| and |(i - s) os + os / 2 - y|,
+// normalised by the sum of its real parts.  One block per (x, y); blockIdx.y: array
+// blockIdx.y of conv (wk_cosine_kernel's positions, npos a side), written to plane
+// blockIdx.y of cache.  A truncated plane's kernels (plane_support non-NULL) have its own
+// support s.
 template <typename KT>
-__global__ __launch_bounds__(256) void wk_extract_kernel(const cplx<double>* conv, int arr, int os, int support,
+__global__ __launch_bounds__(256) void wk_extract_kernel(const cplx<double>* conv, int npos, int len, int os, int support,
     const int* plane_support, cplx<KT>* cache)
 {
-    __shared__ double red[256];
-    conv += size_t(blockIdx.y) * arr * arr;
-    const int cs = os / 2 + 1;
+    __shared__ double red[4];
+    conv += size_t(blockIdx.y) * npos * npos;
+    const int op = os / 2, cs = op + 1;
     const int x = blockIdx.x % cs, y = blockIdx.x / cs;
-    const int sp = plane_support ? plane_support[blockIdx.y] : support;
-    const int ks = 2 * sp + 1;
-    const long long ctr = arr / 2, op = os / 2;
-    const long long oc = ctr - (long long)sp * os + op;
+    const int s = plane_support ? plane_support[blockIdx.y] : support;
+    const int ks = 2 * s + 1;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    // position of sample d os + o, d = -s .. s, o = 0 .. os / 2
+    auto at = [&](int d, int o) { return d >= 0 ? o * len + d : (o ? (os - o) * len - d - 1 : -d); };
     double sum = 0.0;
-    for (int e = threadIdx.x; e < ks * ks; e += 256) {
-        const int i = e % ks, j = e / ks;
-        const long long cxi = (oc - x + (long long)j * os + ctr) % arr;
-        const long long cyi = (oc - y + (long long)i * os + ctr) % arr;
-        sum += conv[cxi + cyi * arr].x;
+    for (int j = wave; j < ks; j += 4) {
+        const cplx<double>* c = conv + size_t(at(j - s, op - x)) * npos;
+        for (int i = lane; i < ks; i += 64)
+            sum += c[at(i - s, op - y)].x;
     }
-    red[threadIdx.x] = sum;
+    for (int off = 32; off > 0; off >>= 1)
+        sum += __shfl_down(sum, off, 64);
+    if (lane == 0)
+        red[wave] = sum;
     __syncthreads();
-    for (int off = 128; off > 0; off >>= 1) {
-        if (threadIdx.x < off)
-            red[threadIdx.x] += red[threadIdx.x + off];
-        __syncthreads();
-    }
-    const double inv = 1.0 / red[0];
+    const double inv = 1.0 / ((red[0] + red[1]) + (red[2] + red[3]));
     cplx<KT>* out = cache + (size_t(blockIdx.y) * cs * cs + blockIdx.x) * w_slot(2 * support + 1);
-    for (int e = threadIdx.x; e < int(w_slot(ks)); e += 256) {
-        const int i = (e - 1) % (ks + 1), j = (e - 1) / (ks + 1) - WPAD;
-        if (e == 0 || i == ks || j < 0 || j >= ks) {
-            out[e] = { KT(0), KT(0) };
-            continue;
+    if (threadIdx.x == 0)
+        out[0] = { KT(0), KT(0) };
+    for (int jc = wave; jc < ks + 2 * WPAD; jc += 4) {
+        const int j = jc - WPAD;
+        const bool in = j >= 0 && j < ks;
+        const cplx<double>* c = conv + size_t(in ? at(j - s, op - x) : 0) * npos;
+        for (int i = lane; i <= ks; i += 64) {
+            cplx<KT> v{ KT(0), KT(0) };
+            if (in && i < ks) {
+                const cplx<double> k = c[at(i - s, op - y)];
+                v = { KT(k.x * inv), KT(k.y * inv) };
+            }
+            out[1 + size_t(jc) * (ks + 1) + i] = v;
         }
-        const long long cxi = (oc - x + (long long)j * os + ctr) % arr;
-        const long long cyi = (oc - y + (long long)i * os + ctr) % arr;
-        const cplx<double> v = conv[cxi + cyi * arr];
-        out[e] = { KT(v.x * inv), KT(v.y * inv) };
     }
 }
 
@@ -2792,8 +2813,8 @@ void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const doubl
             a.analytic_gcf ? 1 : 0);
         const double* d_aa = has_table(ctx, key) ? dev_table(ctx, key, {})
                                                  : dev_table(ctx, key, img_dom_kernel(kf, size_t(workarea), false, a.analytic_gcf));
-        // planes in groups of PB: one fill, one batched 2-D c2c and one extraction per
-        // group, the image-domain arrays of a group at most 256 MB each
+        // planes in groups of PB, each stage one launch per group, the transformed kernels of a
+        // group at most 256 MB
         const int csw = os / 2 + 1; // offsets per axis without their mirror images
         const size_t per_plane = size_t(csw) * csw * w_slot(g.ks);
         wcache_bytes = sizeof(cplx<KT>) * per_plane * P;
@@ -2844,22 +2865,29 @@ void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const doubl
             launch(ctx, "w_kernel_extract", wk_hankel_extract_kernel<KT>, dim3(unsigned(csw * csw), unsigned(P)), dim3(256), 0,
                 h, (const cplx<double>*)kh, (const int*)psup, 0, wcache);
         } else {
-            const size_t arr2 = size_t(arr) * arr;
-            const int PB = int(std::max<size_t>(1, std::min<size_t>(size_t(P), (size_t(1) << 28) / (arr2 * sizeof(cplx<double>)))));
-            cplx<double>* comb = (cplx<double>*)ws_get(ctx, "w_comb", sizeof(cplx<double>) * arr2 * PB);
-            cplx<double>* conv = (cplx<double>*)ws_get(ctx, "w_conv", sizeof(cplx<double>) * arr2 * PB);
+            STP_REQUIRE(arr >= 4 && (arr & (arr - 1)) == 0, "c2c size must be a power of two >= 4");
+            const int half = workarea / 2, len = g.s + 1, npos = os * len;
+            const size_t q2 = size_t(half) * half, t2 = size_t(half) * npos, c2 = size_t(npos) * npos;
+            const int PB = int(std::max<size_t>(1, std::min<size_t>(std::min(P, 65535), (size_t(1) << 28) / (c2 * sizeof(cplx<double>)))));
+            cplx<double>* quad = (cplx<double>*)ws_get(ctx, "w_quad", sizeof(cplx<double>) * q2 * PB);
+            cplx<double>* axis = (cplx<double>*)ws_get(ctx, "w_axis", sizeof(cplx<double>) * t2 * PB);
+            cplx<double>* conv = (cplx<double>*)ws_get(ctx, "w_conv", sizeof(cplx<double>) * c2 * PB);
+            const cplx<double>* tw = (const cplx<double>*)twiddles_for(ctx, arr).d;
             int* psup = trunc ? (int*)ws_get(ctx, "w_psupport", sizeof(int) * P) : nullptr;
             g.psup = psup;
             for (int p0 = 0; p0 < P; p0 += PB) {
                 const int nb = std::min(PB, P - p0);
-                launch(ctx, "w_kernel_fill", wk_fill_kernel, dim3(unsigned(div_up(arr2, 256)), unsigned(nb)), dim3(256), 0, comb,
-                    arr, workarea / 2, d_aa, (const double*)w_plane, p0, a.cell_rad * scaling);
-                fft_c2c_2d<double>(ctx, comb, conv, arr, true, nb);
+                launch(ctx, "w_kernel_fill", wk_fill_kernel, dim3(unsigned(div_up(q2, 256)), unsigned(nb)), dim3(256), 0, quad,
+                    half, d_aa, (const double*)w_plane, p0, a.cell_rad * scaling);
+                launch(ctx, "w_kernel_axis", wk_cosine_kernel, dim3(div_up(npos, 64), div_up(half, 16), unsigned(nb)), dim3(256), 0,
+                    (const cplx<double>*)quad, q2, half, half, half, axis, t2, npos, len, os, tw, arr);
+                launch(ctx, "w_kernel_axis", wk_cosine_kernel, dim3(div_up(npos, 64), div_up(npos, 16), unsigned(nb)), dim3(256), 0,
+                    (const cplx<double>*)axis, t2, npos, npos, half, conv, c2, npos, len, os, tw, arr);
                 if (trunc)
-                    launch(ctx, "w_kernel_trunc", wk_trunc_kernel, dim3(div_up(nb, 64)), dim3(64), 0, (const cplx<double>*)conv, arr,
-                        os, g.s, a.wproj.kernel_trunc_perc / 100.0, nb, psup + p0);
+                    launch(ctx, "w_kernel_trunc", wk_trunc_kernel, dim3(div_up(nb, 64)), dim3(64), 0, (const cplx<double>*)conv, c2,
+                        g.s, a.wproj.kernel_trunc_perc / 100.0, nb, psup + p0);
                 launch(ctx, "w_kernel_extract", wk_extract_kernel<KT>, dim3(unsigned(csw * csw), unsigned(nb)), dim3(256), 0,
-                    (const cplx<double>*)conv, arr, os, g.s, (const int*)(trunc ? psup + p0 : nullptr),
+                    (const cplx<double>*)conv, npos, len, os, g.s, (const int*)(trunc ? psup + p0 : nullptr),
                     wcache + size_t(p0) * per_plane);
             }
         }

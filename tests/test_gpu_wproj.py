@@ -201,3 +201,20 @@ def test_gpu_wproj_large_kernel_cache(gpu):
     a = gpu.image_visibilities(snap["vis"], snap["weights"], snap["uvw"], pars, w_proj=wp)
     b = gpu.image_visibilities(snap["vis"], snap["weights"], snap["uvw"], pars, w_proj=wp, precision=capi.PRECISION_FP32C)
     assert peak_rel_err(b[0], a[0]) < 1e-5 and peak_rel_err(b[1], a[1]) < 1e-5
+
+
+@pytest.mark.parametrize("N,os_,support,us,trunc,planes", [
+    (128, 1, 3, 1, 0.0, 2),    # one kernel per plane
+    (128, 2, 1, 1, 0.0, 2),    # the smallest quadrant (two offsets)
+    (128, 4, 7, 2, 0.0, 3),
+    (128, 16, 8, 1, 0.0, 2),   # output frequencies one past a block of 16
+    (128, 8, 15, 0, 0.0, 2),   # work area of the whole grid
+    (128, 8, 15, 1, 2.0, 3),   # truncated
+    (256, 8, 40, 1, 0.0, 2),   # a workgroup's rows in two passes
+])
+def test_gpu_wproj_kernel_shapes(gpu, orc, N, os_, support, us, trunc, planes):
+    """The W-kernels' cosine transforms and cuts over oversampling, support and work area."""
+    snap = simdata.snapshot(N, 20.0, 1_500, 4, seed=740 + support, field_frac=0.5, w_max=300.0)
+    wp = capi.wproj_pars(planes, support, undersampling_opt=us, kernel_trunc_perc=trunc)
+    img, beam, oimg, obeam = _wcase(gpu, orc, snap, N, 20.0, wp, oversampling=os_)
+    assert peak_rel_err(img, oimg) < TOL and peak_rel_err(beam, obeam) < TOL

@@ -9,6 +9,11 @@
 // The reduce driver subtracts the model from the data before imaging
 // (src/reduce/reduce.cpp:113-122).
 //
+// Bound: the FP64 instructions of the sine and cosine of every (visibility, source) pair.
+// sincospi takes the phase in half turns, whose reduction is exact and short (a general
+// argument is first multiplied by 2 pi, whose rounding it then carries: 6.8e-14 rms at
+// 460 turns): 86 us for 1 M visibilities and 50 sources against 122.
+//
 // One thread per visibility walks the sources, which the workgroup stages in LDS;
 // the per-source constants (offset, flux * n) are computed on the host in FP64,
 // as the reference computes them once per source.
@@ -37,7 +42,6 @@ __global__ __launch_bounds__(VWG) void model_vis_kernel(const double* uvw, long 
     const long long i = (long long)blockIdx.x * VWG + threadIdx.x;
     const bool on = i < n;
     const double u = on ? uvw[i] : 0.0, v = on ? uvw[n + i] : 0.0, w = on ? uvw[2 * n + i] : 0.0;
-    const double c = -2.0 * M_PI;
     double ar = 0.0, ai = 0.0;
     for (int k0 = 0; k0 < n_src; k0 += SRC_CHUNK) {
         const int cnt = min(SRC_CHUNK, n_src - k0);
@@ -49,7 +53,7 @@ __global__ __launch_bounds__(VWG) void model_vis_kernel(const double* uvw, long 
             const SrcTerm t = s[k];
             const double d = (u * t.o0 + v * t.o1) + w * t.o2;
             double sn, cs;
-            sincos(c * d, &sn, &cs);
+            sincospi(-2.0 * d, &sn, &cs);
             ar += t.amp * cs;
             ai += t.amp * sn;
         }

@@ -270,54 +270,6 @@ __global__ __launch_bounds__(256) void sf_hist_reduce(const uint32_t* bh, int nb
         atomicAdd(&out[k], s);
 }
 
-__global__ void sf_ba_gate(SFState* st)
-{
-    // sourcefind.cpp:187-191: a near-constant image takes the exact median
-    const bool exact = (st->sigma * 2) < 0.0001;
-    st->ba_active = exact ? 0 : 1;
-    st->need_exact = exact ? 1 : 0;
-}
-
-// BINAPPROX median from the histogram (matrix_math.cpp:406-452); found = 0 -> exact fallback.
-__global__ void sf_binapprox_pick(const unsigned long long* h, unsigned long long n, SFState* st)
-{
-    if (!st->ba_active)
-        return;
-    const int N = BA_BINS - 1;
-    const double scale = double(N) / (2 * st->sigma);
-    const double left = st->mean - st->sigma;
-    unsigned long long count = h[0];
-    st->need_exact = 1;
-    if (n & 1) {
-        const unsigned long long k = (n + 1) / 2;
-        for (unsigned i = 0; i < unsigned(N + 1); i++) {
-            count += h[1 + i];
-            if (count >= k) {
-                st->median = double(i + 0.5) / scale + left;
-                st->need_exact = 0;
-                return;
-            }
-        }
-    } else {
-        const unsigned long long k = n / 2;
-        for (unsigned i = 0; i < unsigned(N + 1); i++) {
-            count += h[1 + i];
-            if (count >= k) {
-                unsigned j = i;
-                while (count == k) {
-                    j++;
-                    count += h[1 + j];
-                    if (j == unsigned(N))
-                        break;
-                }
-                st->median = double(i + j + 1) / (2 * scale) + left;
-                st->need_exact = 0;
-                return;
-            }
-        }
-    }
-}
-
 // ------------------------------------------------------------------ candidate gather + sort
 struct GatherSpec {
     int shift; // candidates: key >> shift == prefix (shift 64: every element)
@@ -510,25 +462,106 @@ __device__ void sel_init_block(SFState* st, SelState* ss, const SelInit& si)
     ss->scale = double(LIN_BINS) / (hi - lo);
 }
 
-__global__ __launch_bounds__(256) void sel_init(SFState* st, SelState* ss, SelInit si)
+// BINAPPROX median from the histogram (matrix_math.cpp:406-452), then the set-up of the
+// exact search, which runs where the bins give no median.  One workgroup: its threads
+// take four bins each and a scan finds the rank's bin (one thread stepping through the
+// 1001 bins, a load each, took 32 us).
+constexpr int BP_THREADS = 256, BP_PER = 4;
+static_assert(BP_THREADS * BP_PER >= BA_BINS, "bins of the pick");
+__global__ __launch_bounds__(BP_THREADS) void sf_binapprox_pick(const unsigned long long* h, unsigned long long n, SFState* st,
+    SelState* ss, SelInit si)
 {
+    __shared__ unsigned long long wsum[BP_THREADS / 64];
+    __shared__ int at, next;
+    __shared__ unsigned long long through;
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    if (st->ba_active) {
+        constexpr int N = BA_BINS - 1;
+        const unsigned long long k = (n & 1) ? (n + 1) / 2 : n / 2;
+        unsigned long long v[BP_PER], s = 0;
+#pragma unroll
+        for (int j = 0; j < BP_PER; j++) {
+            const int i = t * BP_PER + j;
+            v[j] = h[1 + min(i, N)];
+            v[j] = i <= N ? v[j] : 0ull;
+            s += v[j];
+        }
+        unsigned long long x = s;
+        for (int off = 1; off < 64; off <<= 1) {
+            const unsigned long long y = __shfl_up(x, off, 64);
+            if (lane >= off)
+                x += y;
+        }
+        if (lane == 63)
+            wsum[w] = x;
+        if (t == 0) {
+            at = N + 1;
+            next = N;
+        }
+        __syncthreads();
+        unsigned long long cum = h[0] + x - s;
+        for (int q = 0; q < w; q++)
+            cum += wsum[q];
+        // the first bin whose running count reaches k (the first bin of all may start past it)
+#pragma unroll
+        for (int j = 0; j < BP_PER; j++) {
+            const int i = t * BP_PER + j;
+            const unsigned long long c = cum + v[j];
+            if (i <= N && c >= k && (i == 0 || cum < k)) {
+                at = i;
+                through = c;
+            }
+            cum = c;
+        }
+        __syncthreads();
+        // even counts: with exactly k values through that bin, the next bin that is not empty
+#pragma unroll
+        for (int j = 0; j < BP_PER; j++) {
+            const int i = t * BP_PER + j;
+            if (i > at && i <= N && v[j])
+                atomicMin(&next, i);
+        }
+        __syncthreads();
+        if (t == 0) {
+            const double scale = double(N) / (2 * st->sigma);
+            const double left = st->mean - st->sigma;
+            const unsigned i = unsigned(at);
+            st->need_exact = at > N;
+            if (at <= N) {
+                if (n & 1)
+                    st->median = double(i + 0.5) / scale + left;
+                else
+                    st->median = double(i + (through == k && at < N ? unsigned(next) : i) + 1) / (2 * scale) + left;
+            }
+        }
+    }
     sel_init_block(st, ss, si);
 }
 
 // Mean and sigma from the block partials of sf_sum (last canonical level), then
 // optionally the selection set-up.  clear (nclear doubles, may be null): the state
-// buffer, zeroed first.
+// buffer, zeroed first.  bahist (may be null): the BINAPPROX histogram, cleared, and its
+// gate: a near-constant image takes the exact median (sourcefind.cpp:187-191).
 __global__ __launch_bounds__(CANON_LANES) void sf_stats(const double* part, unsigned m, unsigned long long n, SFState* st,
-    SelState* ss, SelInit si, double* clear, unsigned nclear)
+    SelState* ss, SelInit si, double* clear, unsigned nclear, unsigned long long* bahist)
 {
     __shared__ double lds[2 * CANON_LANES];
     if (clear)
         for (unsigned k = threadIdx.x; k < nclear; k += CANON_LANES)
             clear[k] = 0.0;
+    if (bahist)
+        for (unsigned k = threadIdx.x; k < unsigned(BA_BINS + 1); k += CANON_LANES)
+            bahist[k] = 0;
     double a, b;
     canon_last_level(part, m, a, b, lds);  // its barriers also order the clearing before the writes
-    if (threadIdx.x == 0)
+    if (threadIdx.x == 0) {
         set_mean_sigma(a, b, n, st);
+        if (bahist) {
+            const bool exact = (st->sigma * 2) < 0.0001;
+            st->ba_active = exact ? 0 : 1;
+            st->need_exact = exact ? 1 : 0;
+        }
+    }
     if (si.enabled)
         sel_init_block(st, ss, si);
 }
@@ -621,14 +654,26 @@ __global__ __launch_bounds__(1024) void sel_pick2(SelState* ss, const unsigned l
     ss->gather = 1;
 }
 
+constexpr int GATHER_LIST = 1024;
 template <typename T>
 __global__ __launch_bounds__(HWG) void sel_gather(const T* x, size_t n, const SelState* ss, unsigned long long* cand,
     unsigned* counter)
 {
     if (!ss->gather)
         return;
+    // a workgroup's candidates are listed in LDS and take their places by one atomic
+    // (an atomic each, on one address, took 13 us of the 29 at 16.8 M values)
+    __shared__ unsigned long long list[GATHER_LIST];
+    __shared__ unsigned cnt, base;
+    if (threadIdx.x == 0)
+        cnt = 0;
+    __syncthreads();
     const double lo = ss->lo, scale = ss->scale, base2 = ss->base2, scale2 = ss->scale2;
     const int b1lo = ss->b1_lo, b1hi = ss->b1_hi, b2lo = ss->b2_lo, b2hi = ss->b2_hi, lvl = ss->level;
+    auto put = [&](unsigned slot, unsigned long long k) {
+        if (slot < unsigned(SORT_CAP))
+            cand[slot] = k;
+    };
     stream_values(x, n, [&](double v) {
         const double t = (v - lo) * scale;
         const int b = lin_bin(t);
@@ -638,31 +683,145 @@ __global__ __launch_bounds__(HWG) void sel_gather(const T* x, size_t n, const Se
             take = b2 >= b2lo && b2 <= b2hi;
         }
         if (take) {
-            const unsigned slot = atomicAdd(counter, 1u);
-            if (slot < unsigned(SORT_CAP))
-                cand[slot] = okey(v);
+            const unsigned q = atomicAdd(&cnt, 1u);
+            if (q < unsigned(GATHER_LIST))
+                list[q] = okey(v);
+            else
+                put(atomicAdd(counter, 1u), okey(v));
         }
     });
+    __syncthreads();
+    const unsigned c = min(cnt, unsigned(GATHER_LIST));
+    if (threadIdx.x == 0)
+        base = c ? atomicAdd(counter, c) : 0u;
+    __syncthreads();
+    for (unsigned k = threadIdx.x; k < c; k += HWG)
+        put(base + k, list[k]);
 }
 
-// Sorts the candidates and sets the median (mat_median_exact, matrix_math.cpp:33-45:
-// (upper + lower) / 2 for even sizes).
+// The candidates' two ranks and the median (mat_median_exact, matrix_math.cpp:33-45:
+// (upper + lower) / 2 for even sizes).  A histogram of the keys between their least and
+// largest leaves a few keys around the ranks, whose places are then counted; heavily
+// tied keys are sorted (a sort of all of them took 31 us at 1700 keys, this 6).
+constexpr int PICK_BINS = 4096, PICK_MAX = 256;
 __global__ __launch_bounds__(1024) void sel_sort(SelState* ss, const unsigned long long* cand, const unsigned* count,
     SFState* st)
 {
     __shared__ unsigned long long s[SORT_CAP];
+    __shared__ unsigned long long red[2][16];
+    __shared__ uint32_t wsum[16], nlist;
+    __shared__ int bin[2];
+    __shared__ unsigned before;
+    __shared__ unsigned long long res[2];
     if (!ss->gather)
         return;
     const unsigned c = min(*count, unsigned(SORT_CAP));
-    lds_sort_keys(cand, c, s);
-    if (threadIdx.x != 0)
-        return;
     const unsigned long long r0 = ss->k_lo - ss->before, r1 = ss->k_hi - ss->before;
     if (c != ss->cnt || r1 >= c) {
-        ss->fallback = 1; // the gather disagrees with the histogram counts
+        if (threadIdx.x == 0)
+            ss->fallback = 1; // the gather disagrees with the histogram counts
         return;
     }
-    const double lo = okey_inv(s[r0]), hi = okey_inv(s[r1]);
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+    constexpr int PER = SORT_CAP / 1024;
+    unsigned long long key[PER], kmin = ~0ull, kmax = 0ull;
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        const unsigned i = j * 1024 + t;
+        key[j] = cand[min(i, c - 1)]; // past the end: the last one again, not counted below
+        kmin = min(kmin, key[j]);
+        kmax = max(kmax, key[j]);
+    }
+    for (int off = 32; off >= 1; off >>= 1) {
+        kmin = min(kmin, (unsigned long long)__shfl_xor(kmin, off, 64));
+        kmax = max(kmax, (unsigned long long)__shfl_xor(kmax, off, 64));
+    }
+    if (lane == 0) {
+        red[0][w] = kmin;
+        red[1][w] = kmax;
+    }
+    uint32_t* h = reinterpret_cast<uint32_t*>(s);
+    for (int k = t; k < PICK_BINS; k += 1024)
+        h[k] = 0;
+    if (t == 0)
+        nlist = 0;
+    __syncthreads();
+    for (int k = 0; k < 16; k++) {
+        kmin = min(kmin, red[0][k]);
+        kmax = max(kmax, red[1][k]);
+    }
+    const unsigned long long span = kmax - kmin;
+    const int shift = span < PICK_BINS ? 0 : 64 - __clzll(span) - 12; // span >> shift < PICK_BINS
+#pragma unroll
+    for (int j = 0; j < PER; j++)
+        if (unsigned(j * 1024 + t) < c)
+            atomicAdd(&h[(key[j] - kmin) >> shift], 1u);
+    __syncthreads();
+    // the bins of both ranks, by a scan of four bins per thread
+    uint32_t v[4], sum = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        v[j] = h[4 * t + j];
+        sum += v[j];
+    }
+    uint32_t x = sum;
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t y = __shfl_up(x, off, 64);
+        if (lane >= off)
+            x += y;
+    }
+    if (lane == 63)
+        wsum[w] = x;
+    __syncthreads();
+    uint32_t cum = x - sum;
+    for (int k = 0; k < w; k++)
+        cum += wsum[k];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        if (cum <= r0 && r0 < cum + v[j]) {
+            bin[0] = 4 * t + j;
+            before = cum;
+        }
+        if (cum <= r1 && r1 < cum + v[j])
+            bin[1] = 4 * t + j;
+        cum += v[j];
+    }
+    __syncthreads();
+    const unsigned b0 = unsigned(bin[0]), b1 = unsigned(bin[1]), under = before;
+    // the histogram is done with: the same memory lists the keys of those bins
+#pragma unroll
+    for (int j = 0; j < PER; j++) {
+        const unsigned b = unsigned((key[j] - kmin) >> shift);
+        if (unsigned(j * 1024 + t) < c && b >= b0 && b <= b1) {
+            const uint32_t q = atomicAdd(&nlist, 1u);
+            if (q < PICK_MAX)
+                s[q] = key[j];
+        }
+    }
+    __syncthreads();
+    const uint32_t m = nlist;
+    if (m <= PICK_MAX) {
+        if (unsigned(t) < m) {
+            const unsigned long long k = s[t];
+            unsigned rank = under;
+            for (unsigned q = 0; q < m; q++)
+                rank += s[q] < k || (s[q] == k && q < unsigned(t)) ? 1u : 0u;
+            if (rank == r0)
+                res[0] = k;
+            if (rank == r1)
+                res[1] = k;
+        }
+        __syncthreads();
+    } else {
+        lds_sort_keys(cand, c, s);
+        if (t == 0) {
+            res[0] = s[r0];
+            res[1] = s[r1];
+        }
+    }
+    if (t != 0)
+        return;
+    const double lo = okey_inv(res[0]), hi = okey_inv(res[1]);
     st->median = ss->odd ? hi : (hi + lo) / 2;
     st->need_exact = 0;
 }
@@ -2041,10 +2200,6 @@ void radix_select(stp_ctx* ctx, const T* x, size_t n, size_t k, double* d_out)
     HIP_CHECK(hipMemcpyAsync(d_out, tmp, sizeof(double), hipMemcpyDeviceToDevice, ctx->stream));
 }
 
-// Enqueues the device-driven exact median search (SelState).  It runs when
-// st->need_exact is set on the device (force sets it), reads st->mean and
-// st->sigma, and sets st->median; ss->fallback reports data the bins cannot
-// resolve.  No host round trip.
 // Selection set-up of the exact median of n values (buffers of the search).
 SelInit sel_setup(stp_ctx* ctx, size_t n, int force)
 {
@@ -2063,17 +2218,15 @@ SelInit sel_setup(stp_ctx* ctx, size_t n, int force)
 // Enqueues the device-driven exact median search (SelState).  It runs when
 // st->need_exact is set on the device (si.force sets it), reads st->mean and
 // st->sigma, and sets st->median; ss->fallback reports data the bins cannot
-// resolve.  No host round trip.  initialised: the set-up already ran (fused into
-// the statistics kernel).
+// resolve.  No host round trip.  The set-up (sel_init_block) ran in the statistics or
+// the BINAPPROX kernel.
 template <typename T>
-void enqueue_exact_median(stp_ctx* ctx, const T* x, size_t n, SFState* st, SelState* ss, const SelInit& si, bool initialised)
+void enqueue_exact_median(stp_ctx* ctx, const T* x, size_t n, SFState* st, SelState* ss, const SelInit& si)
 {
     const unsigned nb = hist_blocks(n);
     uint32_t* bh = wsp<uint32_t>(ctx, "sf_bh", size_t(nb) * (LIN_BINS + 2));
     unsigned long long* cand = wsp<unsigned long long>(ctx, "sf_cand", SORT_CAP);
     const unsigned slices = std::min(16u, nb);
-    if (!initialised)
-        launch(ctx, "sel_init", sel_init, dim3(1), dim3(256), 0, st, ss, si);
     launch(ctx, "sel_hist1", sel_hist1<T>, dim3(nb), dim3(HWG), 0, x, n, (const SelState*)ss, bh);
     launch(ctx, "sf_hist_reduce", sf_hist_reduce, dim3(div_up(LIN_BINS + 2, 256), slices), dim3(256), 0,
         (const uint32_t*)bh, int(nb), LIN_BINS + 2, si.hist1, (const int*)&ss->run1);
@@ -2131,40 +2284,39 @@ void source_find_impl(stp_ctx* ctx, const T* x, int rows, int cols, const stp_so
         cleared = true;
     };
     // mean and sigma (canonical sums); si.enabled also sets up the exact-median search
-    auto compute_mean_sigma = [&](const SelInit& si) {
+    auto compute_mean_sigma = [&](const SelInit& si, unsigned long long* bahist) {
         launch(ctx, "sf_sum", sf_sum_kernel<T>, dim3(div_up(nblk, CANON_GROUP)), dim3(SWG), 0, x, n, nblk, part);
         size_t mfin = 0;
         const double* fin = canon_reduce_to_block(ctx, part, nblk, scr, &mfin);
         launch(ctx, "sf_stats", sf_stats, dim3(1), dim3(CANON_LANES), 0, fin, unsigned(mfin), (unsigned long long)n, st, ss, si,
-            cleared ? (double*)nullptr : (double*)stbuf, nstate);
+            cleared ? (double*)nullptr : (double*)stbuf, nstate, bahist);
         cleared = true;
         stats_valid = true;
     };
     // median (sourcefind.cpp:182-197), enqueued without host round trips: the
     // BINAPPROX pick and the exact search are gated on the device state
     if (mm == STP_MEDIAN_BINAPPROX) {
-        compute_mean_sigma(SelInit{});
-        launch(ctx, "sf_ba_gate", sf_ba_gate, dim3(1), dim3(1), 0, st);
         const unsigned nb = hist_blocks(n);
         uint32_t* bh = wsp<uint32_t>(ctx, "sf_babh", size_t(nb) * (BA_BINS + 1));
         unsigned long long* hist = wsp<unsigned long long>(ctx, "sf_bahist", BA_BINS + 1);
+        compute_mean_sigma(SelInit{}, hist);
         launch(ctx, "sf_binapprox_hist", sf_binapprox_hist<T>, dim3(nb), dim3(HWG), 0, x, n, (const SFState*)st, bh);
-        fill_u32(ctx, (uint32_t*)hist, 0u, 2 * size_t(BA_BINS + 1));
         launch(ctx, "sf_hist_reduce", sf_hist_reduce, dim3(div_up(BA_BINS + 1, 256), std::min(64u, nb)), dim3(256), 0,
             (const uint32_t*)bh, int(nb), BA_BINS + 1, hist, (const int*)&st->ba_active);
-        launch(ctx, "sf_binapprox_pick", sf_binapprox_pick, dim3(1), dim3(1), 0, (const unsigned long long*)hist,
-            (unsigned long long)n, st);
-        enqueue_exact_median<T>(ctx, x, n, st, ss, sel_setup(ctx, n, 0), false);
+        const SelInit si = sel_setup(ctx, n, 0);
+        launch(ctx, "sf_binapprox_pick", sf_binapprox_pick, dim3(1), dim3(BP_THREADS), 0, (const unsigned long long*)hist,
+            (unsigned long long)n, st, ss, si);
+        enqueue_exact_median<T>(ctx, x, n, st, ss, si);
     } else if (mm == STP_MEDIAN_BINMEDIAN || mm == STP_MEDIAN_NTHELEMENT) {
         // mean and sigma seed the selection's linear bins (and estimate_rms,
         // sourcefind.cpp:30-36)
         const SelInit si = sel_setup(ctx, n, 1);
-        compute_mean_sigma(si);
-        enqueue_exact_median<T>(ctx, x, n, st, ss, si, true);
+        compute_mean_sigma(si, nullptr);
+        enqueue_exact_median<T>(ctx, x, n, st, ss, si);
     }
     // ZEROMEDIAN: the state's median stays 0
     if (need_rms && !stats_valid)
-        compute_mean_sigma(SelInit{});
+        compute_mean_sigma(SelInit{}, nullptr);
     clear_state();  // no statistics kernel ran (ZEROMEDIAN with a given RMS)
 
     // RMS (sourcefind.cpp:206) and thresholds (:298-301)

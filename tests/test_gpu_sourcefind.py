@@ -275,3 +275,35 @@ def test_gpu_pipeline_c2_full_size(gpu, orc):
     assert [(i["label_idx"], i["extremum_x_idx"], i["extremum_y_idx"]) for i in g2.islands] == \
            [(i["label_idx"], i["extremum_x_idx"], i["extremum_y_idx"]) for i in ores[1]]
     assert len(ores[1]) >= 40
+
+
+@pytest.mark.parametrize("rows,cols,kind", [
+    (2, 2, "noise"),          # fewer values than a wave
+    (64, 64, "noise"),
+    (256, 256, "steps"),      # the median's bin holds thousands of equal values
+    (256, 256, "two"),        # the middle ranks lie at the ends of a gap
+    (512, 256, "heavy"),      # bright pixels widen the bins: a second level
+    (256, 256, "tiny"),       # sigma below BINAPPROX's limit: the exact median
+    (128, 128, "skew"),       # BINAPPROX bins empty around the median
+])
+@pytest.mark.parametrize("median", [capi.MEDIAN_BINMEDIAN, capi.MEDIAN_BINAPPROX])
+def test_gpu_median_picks(gpu, orc, rows, cols, kind, median):
+    """The picks of the median's bins and candidates: bit for bit the oracle's background."""
+    rng = np.random.default_rng(rows + cols)
+    img = rng.normal(0.3, 1.0, size=(rows, cols))
+    if kind == "steps":
+        img = np.round(img, 1)
+    elif kind == "two":
+        img = np.where(rng.permutation(rows * cols).reshape(rows, cols) % 2 == 0, img ** 2 + 0.2, -img ** 2 - 0.2)
+    elif kind == "heavy":
+        img[rng.random((rows, cols)) < 0.01] = 1e4
+    elif kind == "tiny":
+        img *= 1e-6
+    elif kind == "skew":
+        img = np.round(np.exp(1.5 * img), 0)
+    img = np.asfortranarray(img)
+    pars = capi.sourcefind_pars(8.0, 6.0, median_method=median)
+    res = gpu.source_find(img, pars)
+    _, _, st = orc.source_find(img, pars)
+    for k in ("bg_level", "rms_est", "mean", "sigma"):
+        assert getattr(res.stats, k) == getattr(st, k), k

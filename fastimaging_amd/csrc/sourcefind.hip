@@ -38,20 +38,23 @@ constexpr int LIN_BINS = 8192;     // exact-median first level
 constexpr int SORT_CAP = 8192;     // candidates sorted in one workgroup
 constexpr int BA_BINS = 1001;      // BINAPPROX: N + 1 bins (matrix_math.cpp:339,353)
 
+// Sigma-clipping state (sourcefind.cpp:39-151).
+struct ClipState {
+    double d1, d2, sigma, upper, prev_upper;
+    double cand_bound;             // |v - median| bound of the kept candidates
+    unsigned long long valid_n;
+    int iter, iters, done;
+    int compact;                   // the next pass reads the candidates only
+};
+
 struct SFState {
     double s1, s2;                 // canonical sums
     double mean, sigma, median;
     double rms;
-    // sigma-clipping state (sourcefind.cpp:39-151)
-    double d1, d2, clip_sigma, upper, prev_upper;
-    unsigned long long valid_n;
-    int iter, iters, done;
+    ClipState clip[2];             // after even and odd clipping passes
     // device-side control of the median path
     int need_exact;                // exact order statistics still required
     int ba_active;                 // the BINAPPROX histogram is in use
-    int compact;                   // the next clipping pass reads the candidates only
-    double num_sigma;
-    double cand_bound;             // |v - median| bound of the kept clipping candidates
     // thresholds (sourcefind.cpp:298-301)
     double a_pos, a_neg, d_pos, d_neg;
     // results read back by the host
@@ -464,9 +467,9 @@ __device__ void sel_init_block(SFState* st, SelState* ss, const SelInit& si)
 
 // BINAPPROX median from the histogram (matrix_math.cpp:406-452), then the set-up of the
 // exact search, which runs where the bins give no median.  One workgroup: its threads
-// take four bins each and a scan finds the rank's bin (one thread stepping through the
-// 1001 bins, a load each, took 32 us).
-constexpr int BP_THREADS = 256, BP_PER = 4;
+// take a bin each and a scan finds the rank's bin (one thread stepping through the 1001
+// bins, a load each, took 32 us).
+constexpr int BP_THREADS = 1024, BP_PER = 1;
 static_assert(BP_THREADS * BP_PER >= BA_BINS, "bins of the pick");
 __global__ __launch_bounds__(BP_THREADS) void sf_binapprox_pick(const unsigned long long* h, unsigned long long n, SFState* st,
     SelState* ss, SelInit si)
@@ -972,25 +975,7 @@ __device__ __forceinline__ void clip_block_full(const T* x, size_t n, size_t blk
     }
 }
 
-// Clipping passes after the first: one wave per canonical block, reading the kept
-// candidates while the bound allows it (every lane of the grid takes one branch).
-template <typename T>
-__global__ __launch_bounds__(SWG) void sf_clip_next_kernel(const T* x, size_t n, size_t nblk, const SFState* st,
-    double* part, uint32_t* removed, T* cand, uint32_t* ltab)
-{
-    if (st->done)
-        return;
-    const double upper = st->upper, prev = st->prev_upper, median = st->median;
-    const size_t blk = size_t(blockIdx.x) * (SWG / 64) + (threadIdx.x >> 6);
-    if (blk >= nblk)
-        return;
-    if (st->compact)
-        clip_candidates(cand, ltab, blk, median, upper, prev, part, removed);
-    else
-        clip_block_full(x, n, blk, median, upper, prev, CLIP_CAND_FRAC * upper, part, removed, cand, ltab);
-}
-
-// The first clipping pass (the state of sf_clip_init) over the whole image; keeps
+// The first clipping pass (the state of clip_init) over the whole image; keeps
 // the candidates of its bound.
 template <typename T>
 __global__ __launch_bounds__(SWG) void sf_clip_kernel(const T* x, size_t n, size_t nblk, const SFState* st,
@@ -1062,27 +1047,144 @@ __global__ __launch_bounds__(SWG) void sf_clip_kernel(const T* x, size_t n, size
     }
 }
 
-__device__ void clip_init_state(SFState* st, unsigned long long n, int iters, double num_sigma)
+// The state before the first pass.
+__device__ ClipState clip_init(const SFState* st, unsigned long long n, int iters, double num_sigma)
 {
-    const double median = st->median;
-    const double mean = st->mean - median;
+    const double mean = st->mean - st->median;
     const double sigma = st->sigma;
-    st->d1 = double(mean) * double(n);
-    st->d2 = (double(sigma) * double(sigma) + double(mean) * double(mean)) * double(n);
-    st->valid_n = n;
-    st->clip_sigma = sigma;
-    st->num_sigma = num_sigma;
-    st->upper = num_sigma * sigma;
-    st->prev_upper = DBL_MAX;
-    st->iter = 0;
-    st->iters = iters;
-    st->done = iters <= 0;
-    st->compact = 0;
+    ClipState c;
+    c.d1 = double(mean) * double(n);
+    c.d2 = (double(sigma) * double(sigma) + double(mean) * double(mean)) * double(n);
+    c.valid_n = n;
+    c.sigma = sigma;
+    c.upper = num_sigma * sigma;
+    c.prev_upper = DBL_MAX;
+    c.cand_bound = 0.0;
+    c.iter = 0;
+    c.iters = iters;
+    c.done = iters <= 0;
+    c.compact = 0;
+    return c;
 }
 
-__global__ void sf_clip_init(SFState* st, unsigned long long n, int iters, double num_sigma)
+// One clipping step (sourcefind.cpp:39-151): the state after a pass that removed rem
+// values with the sums a, b (stale and unused once the clipping has ended).
+__device__ ClipState clip_step(ClipState c, unsigned long long rem, double a, double b, double num_sigma)
 {
-    clip_init_state(st, n, iters, num_sigma);
+    if (c.done)
+        return c;
+    // a full pass kept the candidates of its own bound
+    if (!c.compact)
+        c.cand_bound = CLIP_CAND_FRAC * c.upper;
+    if (rem == 0) {
+        c.done = 1;
+        return c;
+    }
+    c.valid_n -= rem;
+    c.d1 -= a;
+    c.d2 -= b;
+    const double vn = double(c.valid_n);
+    c.sigma = sqrt(c.d2 / vn - (c.d1 / vn) * (c.d1 / vn));
+    c.prev_upper = c.upper;
+    c.upper = num_sigma * c.sigma;
+    c.compact = c.upper >= c.cand_bound;
+    c.iter++;
+    c.done = c.iter >= c.iters;
+    return c;
+}
+
+// The totals of a pass by a workgroup of CU_THREADS: the last canonical level of its m
+// (<= CANON_BLOCK) pairs by the first CANON_LANES threads, the removal counts by the
+// others.  Thread 0 gets the sums.
+constexpr int CU_THREADS = 1024;
+__device__ __forceinline__ void clip_totals(const double* cpart, unsigned m, const uint32_t* removed, int nblk, double& a,
+    double& b, unsigned long long& rem)
+{
+    __shared__ double lds[2 * CANON_LANES];
+    __shared__ unsigned long long red[CU_THREADS / 64];
+    const int t = threadIdx.x;
+    constexpr int CT = CU_THREADS - CANON_LANES, U = 8;
+    unsigned long long c = 0;
+    double va[CANON_PER_LANE], vb[CANON_PER_LANE];
+    if (t < CANON_LANES) {
+        // every load before the first sum (clamped index), as canon_last_level
+#pragma unroll
+        for (int j = 0; j < CANON_PER_LANE; j++) {
+            const unsigned i = min(unsigned(j) * CANON_LANES + t, m > 0 ? m - 1 : 0u);
+            va[j] = cpart[2 * i];
+            vb[j] = cpart[2 * i + 1];
+        }
+        a = 0.0;
+        b = 0.0;
+#pragma unroll
+        for (int j = 0; j < CANON_PER_LANE; j++) {
+            const bool ok = unsigned(j) * CANON_LANES + t < m;
+            a = ok ? a + va[j] : a;
+            b = ok ? b + vb[j] : b;
+        }
+        lds[t] = a;
+        lds[CANON_LANES + t] = b;
+    } else {
+        for (int k0 = t - CANON_LANES; k0 < nblk; k0 += CT * U) {
+            uint32_t r[U];
+#pragma unroll
+            for (int j = 0; j < U; j++)
+                r[j] = removed[min(k0 + j * CT, nblk - 1)];
+#pragma unroll
+            for (int j = 0; j < U; j++)
+                c += k0 + j * CT < nblk ? r[j] : 0u;
+        }
+    }
+    for (int off = 32; off >= 1; off >>= 1)
+        c += __shfl_down(c, off, 64);
+    if ((t & 63) == 0)
+        red[t >> 6] = c;
+    __syncthreads();
+    // canon_tree's levels: 128 and 64 apart, then the shuffles of the first wave
+    if (t < 64) {
+        double x = (lds[t] + lds[t + 128]) + (lds[t + 64] + lds[t + 192]);
+        double y = (lds[CANON_LANES + t] + lds[CANON_LANES + t + 128]) + (lds[CANON_LANES + t + 64] + lds[CANON_LANES + t + 192]);
+        for (int off = 32; off >= 1; off >>= 1) {
+            x = x + __shfl_down(x, off, 64);
+            y = y + __shfl_down(y, off, 64);
+        }
+        a = x;
+        b = y;
+    }
+    rem = 0;
+    for (int k = 0; k < CU_THREADS / 64; k++)
+        rem += red[k];
+}
+
+// Clipping passes after the first (pass: 2, 3, ...): one wave per canonical block, reading
+// the kept candidates while the bound allows it.  Every workgroup first takes the step
+// of the pass before from its partials (a kernel of one workgroup between the passes took
+// 4.5 us of 13 each); workgroup 0 stores the state.  The partials and the state
+// alternate between two buffers, since the other workgroups still read the last ones.
+template <typename T>
+__global__ __launch_bounds__(CU_THREADS) void sf_clip_next_kernel(const T* x, size_t n, size_t nblk, SFState* st, int pass,
+    int iters, double num_sigma, const double* fin, unsigned m, const uint32_t* removed_in, double* part, uint32_t* removed,
+    T* cand, uint32_t* ltab)
+{
+    __shared__ ClipState cs;
+    double a, b;
+    unsigned long long rem;
+    clip_totals(fin, m, removed_in, int(nblk), a, b, rem);
+    if (threadIdx.x == 0) {
+        const ClipState before = pass == 2 ? clip_init(st, n, iters, num_sigma) : st->clip[pass & 1];
+        cs = clip_step(before, rem, a, b, num_sigma);
+        if (blockIdx.x == 0)
+            st->clip[(pass + 1) & 1] = cs;
+    }
+    __syncthreads();
+    const size_t blk = size_t(blockIdx.x) * (CU_THREADS / 64) + (threadIdx.x >> 6);
+    if (cs.done || blk >= nblk)
+        return;
+    const double median = st->median;
+    if (cs.compact)
+        clip_candidates(cand, ltab, blk, median, cs.upper, cs.prev_upper, part, removed);
+    else
+        clip_block_full(x, n, blk, median, cs.upper, cs.prev_upper, CLIP_CAND_FRAC * cs.upper, part, removed, cand, ltab);
 }
 
 // Detection and analysis thresholds (sourcefind.cpp:298-301).
@@ -1092,9 +1194,9 @@ struct ThreshArgs {
     uint32_t* reset;     // counter cleared for the labelling (may be null)
 };
 
-__device__ void set_thresholds(SFState* st, const ThreshArgs& ta)
+__device__ void set_thresholds(SFState* st, const ThreshArgs& ta, double rms_clipped)
 {
-    const double rms = ta.estimate ? st->clip_sigma : ta.rms_in;
+    const double rms = ta.estimate ? rms_clipped : ta.rms_in;
     st->rms = rms;
     const double bg = st->median;
     st->a_pos = bg + ta.ana * rms;
@@ -1105,67 +1207,23 @@ __device__ void set_thresholds(SFState* st, const ThreshArgs& ta)
         *ta.reset = 0;
 }
 
+// Thresholds without clipping passes: the RMS is sigma, or given.
 __global__ void sf_thresholds(SFState* st, ThreshArgs ta)
 {
-    set_thresholds(st, ta);
+    set_thresholds(st, ta, st->sigma);
 }
 
-// One clipping step (sourcefind.cpp:39-151) from the block partials of sf_clip
-// (m <= CANON_BLOCK pairs after any earlier canonical levels; removed: one count
-// per block).  Iteration 0 first sets up the state; the last iteration also sets
-// the thresholds.  The partials are read before the state is: after the end of
-// the clipping they are stale and go unused.
-__global__ __launch_bounds__(256) void sf_clip_update(SFState* st, const double* cpart, unsigned m, const uint32_t* removed,
-    int nblk, int iter, unsigned long long n, int iters, double num_sigma, int last, ThreshArgs ta)
+// The step of the last clipping pass, and the thresholds.
+__global__ __launch_bounds__(CU_THREADS) void sf_clip_last(SFState* st, const double* fin, unsigned m, const uint32_t* removed,
+    int nblk, unsigned long long n, int iters, double num_sigma, ThreshArgs ta)
 {
-    __shared__ double lds[2 * CANON_LANES];
-    __shared__ unsigned long long red[256 / 64];
-    const int t = threadIdx.x;
-    unsigned long long c = 0;
-    for (int k0 = 0; k0 < nblk; k0 += 256 * 16) {
-        // unconditional loads (clamped index) so that none waits on another
-        uint32_t r[16];
-#pragma unroll
-        for (int j = 0; j < 16; j++)
-            r[j] = removed[min(k0 + j * 256 + t, nblk - 1)];
-#pragma unroll
-        for (int j = 0; j < 16; j++)
-            c += k0 + j * 256 + t < nblk ? r[j] : 0u;
-    }
     double a, b;
-    canon_last_level(cpart, m, a, b, lds);
-    for (int off = 32; off >= 1; off >>= 1)
-        c += __shfl_down(c, off, 64);
-    if ((t & 63) == 0)
-        red[t >> 6] = c;
-    __syncthreads();
-    if (t != 0)
+    unsigned long long rem;
+    clip_totals(fin, m, removed, nblk, a, b, rem);
+    if (threadIdx.x != 0)
         return;
-    if (iter == 0)
-        clip_init_state(st, n, iters, num_sigma);
-    if (!st->done) {
-        const unsigned long long rem = red[0] + red[1] + red[2] + red[3];
-        // a full pass kept the candidates of its own bound
-        if (!st->compact)
-            st->cand_bound = CLIP_CAND_FRAC * st->upper;
-        if (rem == 0) {
-            st->done = 1;
-        } else {
-            st->valid_n -= rem;
-            st->d1 -= a;
-            st->d2 -= b;
-            const double vn = double(st->valid_n);
-            st->clip_sigma = sqrt(st->d2 / vn - (st->d1 / vn) * (st->d1 / vn));
-            st->prev_upper = st->upper;
-            st->upper = st->num_sigma * st->clip_sigma;
-            st->compact = st->upper >= st->cand_bound;
-            st->iter++;
-            if (st->iter >= st->iters)
-                st->done = 1;
-        }
-    }
-    if (last)
-        set_thresholds(st, ta);
+    const ClipState before = iters == 1 ? clip_init(st, n, iters, num_sigma) : st->clip[(iters + 1) & 1];
+    set_thresholds(st, ta, clip_step(before, rem, a, b, num_sigma).sigma);
 }
 
 // ------------------------------------------------------------------ labelling
@@ -2325,25 +2383,29 @@ void source_find_impl(stp_ctx* ctx, const T* x, int rows, int cols, const stp_so
         const ThreshArgs ta{ int(need_rms), p.rms_est, p.detection_n_sigma, p.analysis_n_sigma, reset };
         const int iters = need_rms ? std::max(0, p.sigma_clip_iters) : 0;
         if (iters > 0) {
-            uint32_t* removed = wsp<uint32_t>(ctx, "sf_removed", nblk);
-            double* cpart = wsp<double>(ctx, "sf_cpart", 2 * nblk + 2);
+            // two sets of partials: a pass reads those of the pass before
+            uint32_t* removed = wsp<uint32_t>(ctx, "sf_removed", 2 * nblk);
+            double* cpart = wsp<double>(ctx, "sf_cpart", 2 * (2 * nblk + 2));
+            double* cscr = wsp<double>(ctx, "sf_cscr", 2 * canon_scratch_doubles(nblk));
             T* cand = wsp<T>(ctx, "sf_clip_cand", nblk * CANON_BLOCK);
             uint32_t* ltab = wsp<uint32_t>(ctx, "sf_clip_lanes", nblk * CANON_LANES);
-            for (int it = 0; it < iters; it++) {
-                if (it == 0)
+            const double* fin = nullptr;
+            size_t mfin = 0;
+            for (int pass = 1; pass <= iters; pass++) {
+                double* cp = cpart + (pass & 1) * (2 * nblk + 2);
+                uint32_t* rm = removed + (pass & 1) * nblk;
+                if (pass == 1)
                     launch(ctx, "sf_clip", sf_clip_kernel<T>, dim3(div_up(nblk, CANON_GROUP)), dim3(SWG), 0, x, n, nblk,
-                        (const SFState*)st, 3.0, cpart, removed, cand, ltab);
+                        (const SFState*)st, 3.0, cp, rm, cand, ltab);
                 else
-                    launch(ctx, "sf_clip_next", sf_clip_next_kernel<T>, dim3(div_up(nblk, SWG / 64)), dim3(SWG), 0, x, n,
-                        nblk, (const SFState*)st, cpart, removed, cand, ltab);
-                size_t mfin = 0;
-                const double* fin = canon_reduce_to_block(ctx, cpart, nblk, scr, &mfin);
-                launch(ctx, "sf_clip_update", sf_clip_update, dim3(1), dim3(256), 0, st, fin, unsigned(mfin),
-                    (const uint32_t*)removed, int(nblk), it, (unsigned long long)n, iters, 3.0, int(it == iters - 1), ta);
+                    launch(ctx, "sf_clip_next", sf_clip_next_kernel<T>, dim3(div_up(nblk, CU_THREADS / 64)), dim3(CU_THREADS), 0,
+                        x, n, nblk, st, pass, iters, 3.0, fin, unsigned(mfin), (const uint32_t*)(removed + ((pass + 1) & 1) * nblk),
+                        cp, rm, cand, ltab);
+                fin = canon_reduce_to_block(ctx, cp, nblk, cscr + (pass & 1) * canon_scratch_doubles(nblk), &mfin);
             }
+            launch(ctx, "sf_clip_last", sf_clip_last, dim3(1), dim3(CU_THREADS), 0, st, fin, unsigned(mfin),
+                (const uint32_t*)(removed + (iters & 1) * nblk), int(nblk), (unsigned long long)n, iters, 3.0, ta);
         } else {
-            if (need_rms)
-                launch(ctx, "sf_clip_init", sf_clip_init, dim3(1), dim3(1), 0, st, (unsigned long long)n, 0, 3.0);
             launch(ctx, "sf_thresholds", sf_thresholds, dim3(1), dim3(1), 0, st, ta);
         }
     };

@@ -218,3 +218,20 @@ def test_gpu_wproj_kernel_shapes(gpu, orc, N, os_, support, us, trunc, planes):
     wp = capi.wproj_pars(planes, support, undersampling_opt=us, kernel_trunc_perc=trunc)
     img, beam, oimg, obeam = _wcase(gpu, orc, snap, N, 20.0, wp, oversampling=os_)
     assert peak_rel_err(img, oimg) < TOL and peak_rel_err(beam, obeam) < TOL
+
+
+@pytest.mark.parametrize("n", [1, 64, 4_096, 4_097, 524_288, 524_289, (1 << 20) + 1])
+def test_gpu_wproj_order(gpu, orc, n):
+    """The |w| order over the sort's block sizes and ways of adding up the counts, with many ties,
+    zeros of both signs and values down to the subnormals: a visibility out of order would be
+    gridded with another plane's kernel."""
+    rng = np.random.default_rng(760)
+    N, cell, planes = 64, 20.0, min(n, 37)
+    cell_rad = cell / 3600.0 * np.pi / 180.0
+    uvw = np.zeros((n, 3), order="F")
+    uvw[:, :2] = rng.uniform(-0.4, 0.4, (n, 2)) / cell_rad
+    uvw[:, 2] = rng.choice(np.concatenate([rng.uniform(-900.0, 900.0, 200), [0.0, -0.0, 5e-324, 1e-300, -1e-9]]), n)
+    uvw[n // 2:, 2] = rng.uniform(-900.0, 900.0, n - n // 2)
+    snap = dict(uvw=uvw, vis=rng.normal(size=n) + 1j * rng.normal(size=n), weights=rng.uniform(0.5, 2.0, n))
+    img, beam, oimg, obeam = _wcase(gpu, orc, snap, N, cell, capi.wproj_pars(planes, 2))
+    assert peak_rel_err(img, oimg) < TOL and peak_rel_err(beam, obeam) < TOL

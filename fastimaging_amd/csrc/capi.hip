@@ -114,9 +114,9 @@ std::string tune_key(const stp_imager_pars* p, const stp_wproj_pars* wp, size_t 
 }
 
 // Gridder arguments of one imaging call (imager.h:233-376) with the autotuned
-// launch shape of its imaging shape; the FFT's u split in *fft_l1.
+// launch shape of its imaging shape.
 GridderArgs imager_args(stp_ctx* ctx, const stp_imager_pars* p, const stp_wproj_pars* wp, const stp_kernel_spec& kern,
-    size_t n, int precision, int* fft_l1)
+    size_t n, int precision)
 {
     const int N = int(p->padded_image_size);
     GridderArgs a;
@@ -134,12 +134,9 @@ GridderArgs imager_args(stp_ctx* ctx, const stp_imager_pars* p, const stp_wproj_
         a.wproj = *wp;
     a.cell_rad = (p->cell_size / 3600.0) * (M_PI / 180.0);
     a.analytic_gcf = p->analytic_gcf != 0;
-    *fft_l1 = 0;
     auto tc = ctx->tune.find(tune_key(p, wp, n, precision));
-    if (tc != ctx->tune.end()) {
+    if (tc != ctx->tune.end())
         a.tile_cols = tc->second.tile_cols;
-        *fft_l1 = tc->second.fft_l1;
-    }
     return a;
 }
 
@@ -167,10 +164,9 @@ void run_imager(stp_ctx* ctx, const stp_imager_pars* p, const stp_wproj_pars* wp
     const int N = int(p->padded_image_size);
     const bool beam = p->generate_beam != 0;
     STP_REQUIRE(!beam || d_beam != nullptr, "beam buffer is NULL with generate_beam");
-    int fft_l1 = 0;
     const int precision = std::is_same<T, double>::value ? STP_PRECISION_FP64
                                                           : (twofloat ? STP_PRECISION_FP32_TWOFLOAT : STP_PRECISION_FP32C);
-    GridderArgs a = imager_args(ctx, p, wp, kern, n, precision, &fft_l1);
+    GridderArgs a = imager_args(ctx, p, wp, kern, n, precision);
     a.d_nentries = d_nentries;
     // without W-projection the sampling grid is real: packed, half the bytes in the
     // grid and the FFT
@@ -182,7 +178,6 @@ void run_imager(stp_ctx* ctx, const stp_imager_pars* p, const stp_wproj_pars* wp
     NormSpec ns;
     ns.image_size = int(p->image_size);
     ns.total_ptr = d_total;
-    ns.u_l1 = fft_l1;
     ns.gcf = gcf_table(ctx, p, kern);
     OutPtrs<OT> outs{};
     outs.p[0] = d_image;
@@ -203,23 +198,22 @@ bool batch_fusable(stp_ctx* ctx, const stp_batch_item& it, const stp_kernel_spec
     if (it.w_proj.num_wplanes > 0)
         return false;
     const stp_kernel_spec kern = kspec ? *kspec : dispatch_kernel(&it.img_pars);
-    int l1;
-    return grid_batch_eligible(imager_args(ctx, &it.img_pars, nullptr, kern, it.n_vis, precision, &l1), it.n_vis);
+    return grid_batch_eligible(imager_args(ctx, &it.img_pars, nullptr, kern, it.n_vis, precision), it.n_vis);
 }
 
 // A chunk of the fused items of a batch: one gridding launch per stage over all of
 // them (grid_batch_bin, then grid_batch_tiles), then one c2r per group of equal
-// transform shape (padded size, image size, gcf, u split, beam) over the group's
+// transform shape (padded size, image size, gcf, beam) over the group's
 // grids, which lie contiguous.  The three phases run on the context stream current
 // at each call, so a caller can give them different, ordered streams.
 template <typename T, typename OT>
 struct FusedChunk {
     struct Shape {
-        int N, image, l1, beam;
+        int N, image, beam;
         const double* gcf;
         bool operator<(const Shape& o) const
         {
-            return std::tie(N, image, l1, beam, gcf) < std::tie(o.N, o.image, o.l1, o.beam, o.gcf);
+            return std::tie(N, image, beam, gcf) < std::tie(o.N, o.image, o.beam, o.gcf);
         }
     };
     struct Run {
@@ -242,9 +236,8 @@ struct FusedChunk {
             const stp_imager_pars* p = &it.img_pars;
             const stp_kernel_spec kern = kspec ? *kspec : dispatch_kernel(p);
             check_kernel_spec(&kern);
-            int l1 = 0;
             BatchGridItem& b = bg[q];
-            b.a = imager_args(ctx, p, nullptr, kern, it.n_vis, precision, &l1);
+            b.a = imager_args(ctx, p, nullptr, kern, it.n_vis, precision);
             b.a.beam_packed = p->generate_beam != 0;  // eligible snapshots: no W-projection, N >= 8
             b.n = it.n_vis;
             b.uv = it.d_uvw_lambda;
@@ -252,7 +245,7 @@ struct FusedChunk {
             b.wts = it.d_vis_weights;
             b.total = totals + 2 * idx[q];
             b.ngood = (unsigned long long*)(totals + 2 * idx[q] + 1);
-            groups[Shape{ int(p->padded_image_size), int(p->image_size), l1, p->generate_beam ? 1 : 0,
+            groups[Shape{ int(p->padded_image_size), int(p->image_size), p->generate_beam ? 1 : 0,
                        gcf_table(ctx, p, kern) }]
                 .push_back(q);
         }
@@ -302,7 +295,6 @@ struct FusedChunk {
             NormSpec ns;
             ns.image_size = r.s.image;
             ns.total_tab = (const double* const*)(d_extra + r.tot_off);
-            ns.u_l1 = r.s.l1;
             ns.gcf = r.s.gcf;
             OutPtrs<OT> outs{};
             outs.tab = (OT* const*)(d_extra + r.out_off);
@@ -359,8 +351,8 @@ void run_imaging(stp_ctx* ctx, const stp_imager_pars* p, const stp_wproj_pars* w
 }
 
 // Autotuner: times the imaging of this very input with each candidate launch
-// configuration (gridder tile width 16 / 32 / 64 columns, then the u-axis FFT
-// split around the balanced one) and keeps the fastest for the shape.
+// configuration (gridder tile width 16 / 32 / 64 columns) and keeps the fastest for the
+// shape.
 void autotune_shape(stp_ctx* ctx, const stp_imager_pars* p, const stp_wproj_pars* wp, const stp_kernel_spec* kernel, size_t n,
     const double* d_vis, const double* d_w, const double* d_uvw, int32_t precision, void* d_image, void* d_beam,
     double* d_total, unsigned long long* d_ngood)
@@ -391,20 +383,6 @@ void autotune_shape(stp_ctx* ctx, const stp_imager_pars* p, const stp_wproj_pars
         for (int tcw : { 16, 32, 64 }) {
             TuneChoice c;
             c.tile_cols = tcw;
-            c.us = time_one(c);
-            if (c.us < best.us)
-                best = c;
-        }
-        const int N = int(p->padded_image_size);
-        int lg = 0;
-        while ((1 << lg) < N)
-            lg++;
-        const int bal = 1 << ((lg + 1) / 2);
-        for (int l1 : { bal / 2, bal * 2 }) {
-            if (l1 < 2 || l1 > 128 || N / l1 < 2 || N / l1 > 128)
-                continue;
-            TuneChoice c = best;
-            c.fft_l1 = l1;
             c.us = time_one(c);
             if (c.us < best.us)
                 best = c;

@@ -54,7 +54,7 @@ struct TimingAcc {
 // Launch configuration picked by the autotuner for one imaging shape.
 struct TuneChoice {
     int tile_cols = 0; // gridder tile width
-    int fft_l1 = 0;    // four-step split of the u-axis FFT
+    int fft_l1 = 0;    // a u-axis FFT split read from a tuning file (kept, without effect)
     double us = 0.0;   // measured imaging time with this choice
 };
 

@@ -3,14 +3,15 @@
 //
 // Layout: a half-plane grid is (n/2+1) rows (v) x N columns (u), column-major,
 // complex.  The 2-D c2r runs
-//   U1, U2 : four-step c2c along u (N = L1 * L2), in place; element (v, x) of
-//            the transformed grid sits in column slot (x % L1) * L2 + x / L1;
+//   U      : c2c along u, in place (16 to 8192 columns);
+//   U1, U2 : the same as a four-step c2c (N = L1 * L2) for the other lengths; element
+//            (v, x) of the transformed grid sits in column slot (x % L1) * L2 + x / L1;
 //   V      : per output column x, c2r along v of length n via one complex FFT
 //            of length n/2 (even/odd packing); the imaginary parts of the v=0
 //            and v=n/2 rows are ignored, as FFTW's c2r does.  Normalisation,
 //            padding crop and grid correction of the imager are fused here.
 // A real grid (the imager's sampling grid without W-projection) is stored packed,
-// two real columns per complex one: U1, U2 run at half the length, and the V pass
+// two real columns per complex one: the u passes run at half the length, and the V pass
 // splits each column pair into the two u-transformed columns first (fft_v_c2r_real).
 // Each transform runs in LDS with 64-wide waves (radix-8 Stockham stages after
 // one radix-2 or radix-4 stage); a workgroup holds NT transforms of length L,
@@ -167,6 +168,48 @@ __device__ __forceinline__ void bfly8(cplx<T>* v, bool inverse)
     }
 }
 
+// x (c + i s), or its conjugate factor for the forward transform
+template <typename T, bool INV>
+__device__ __forceinline__ cplx<T> rot(cplx<T> x, T c, T s)
+{
+    return INV ? cplx<T>{ x.x * c - x.y * s, x.x * s + x.y * c } : cplx<T>{ x.x * c + x.y * s, x.y * c - x.x * s };
+}
+
+// Radix-16 DFT, y_k = sum_r v_r w^{rk}, w = exp(+-i pi/8), r = r0 + 4 r1, k = k1 + 4 k2:
+// four radix-4 DFTs over r1, times w^{r0 k1}, four over r0.
+template <typename T, bool INV>
+__device__ __forceinline__ void bfly16(cplx<T>* v)
+{
+    const T c = T(0.92387953251128675612818318939678829L), s = T(0.38268343236508977172845998403039887L);
+    const T h = T(0.70710678118654752440084436210484904L);
+    cplx<T> t[4][4];  // t[r0][k1]
+#pragma unroll
+    for (int r0 = 0; r0 < 4; r0++) {
+#pragma unroll
+        for (int r1 = 0; r1 < 4; r1++)
+            t[r0][r1] = v[r0 + 4 * r1];
+        bfly4(t[r0], INV);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    t[1][1] = rot<T, INV>(t[1][1], c, s);
+    t[1][2] = rot<T, INV>(t[1][2], h, h);
+    t[1][3] = rot<T, INV>(t[1][3], s, c);
+    t[2][1] = rot<T, INV>(t[2][1], h, h);
+    t[2][2] = rot<T, INV>(t[2][2], T(0), T(1));
+    t[2][3] = rot<T, INV>(t[2][3], -h, h);
+    t[3][1] = rot<T, INV>(t[3][1], s, c);
+    t[3][2] = rot<T, INV>(t[3][2], -h, h);
+    t[3][3] = rot<T, INV>(t[3][3], -c, -s);
+#pragma unroll
+    for (int k1 = 0; k1 < 4; k1++) {
+        cplx<T> a[4] = { t[0][k1], t[1][k1], t[2][k1], t[3][k1] };
+        bfly4(a, INV);
+#pragma unroll
+        for (int k2 = 0; k2 < 4; k2++)
+            v[k1 + 4 * k2] = a[k2];
+    }
+}
+
 // One Stockham stage of radix R on a length-L transform held at buf.
 template <typename T, int L, int TPT, int R, typename TW>
 __device__ __forceinline__ void stockham_stage(cplx<T>* buf, int lt, int Ns, const TW& tw, bool inverse)
@@ -260,6 +303,147 @@ struct UShape {
     static constexpr int NT = WG / TPT;
     static constexpr int PAD = 1;
 };
+
+// U: the whole transform along u in one pass, in place, for lengths of 16 to 8192.  A
+// workgroup takes NR rows; a thread holds EPT elements of one row in registers through
+// all stages (one of radix 2, 4, 8 or 16, the others of radix 16), and the elements change
+// threads between stages through LDS, real parts first, then imaginary parts, which halves
+// the LDS a row needs.  Lanes run over the rows first, so an access to a column is NR
+// elements long; neighbouring row blocks run on the same XCD and find the rest of their
+// cache lines in its L2.  Bound by the phases of a workgroup (loads, the vector unit at a
+// third of the time, stores), which overlap little while one image's rows fit the chip at
+// once.  N=4096 half plane with its half-length beam: 72 us FP32, 130 us FP64, against 87
+// and 166 us for two passes of the four-step split (fft_u1, fft_u2), with a launch less per
+// grid; 8192 FP32 236 us against 247 us.  Two FP32 rows per workgroup take 338 us at 8192
+// and two FP64 rows 144 us at 4096 (shorter runs); the whole complex row in LDS would
+// leave half as many rows per CU.
+template <typename T, int N>
+struct URow {
+    // 16 elements leave a wave 64 FP32 registers (128 FP64), so two workgroups fit a CU
+    static constexpr int EPT = N == 8192 && sizeof(T) == 4 ? 32 : 16;
+    static constexpr int TPR = N / EPT;                              // threads per row
+    static constexpr int NR = TPR < 16 ? 64 / TPR : (N == 8192 && sizeof(T) == 8 ? 2 : 4);
+    static constexpr int THREADS = TPR * NR;
+    static constexpr int PADN = N + N / 16;
+    static constexpr int FIRST = (N == 16 || N == 256 || N == 4096) ? 16
+        : (N == 32 || N == 512 || N == 8192)                       ? 2
+        : (N == 64 || N == 1024)                                   ? 4
+                                                                   : 8;
+};
+
+// Element e of a row in the exchange buffer: one word of padding per 16 spreads both the
+// strided writes and the contiguous reads of a wave over all banks.  u_pad(a + c) = u_pad(a)
+// + u_pad(c) wherever it is used: a mod 16 and the multiples c mod 16 never carry.
+__device__ __forceinline__ constexpr int u_pad(int e) { return e + (e >> 4); }
+
+// One stage of radix R on the thread's elements v[b * R + r] = x[j + r N / R], j = lt + b TPR,
+// then the exchange and the stages after it.  NS: product of the radices before.
+template <typename T, int N, bool INV, int R, int NS>
+__device__ __forceinline__ void u_stages(cplx<T>* v, T* s, int lt, int vv, const cplx<T>* tw)
+{
+    using U = URow<T, N>;
+    constexpr int B = U::EPT / R;
+#pragma unroll
+    for (int b = 0; b < B; b++) {
+        cplx<T>* x = v + b * R;
+        if constexpr (NS > 1) {
+            // W^k, W = exp(+-2 pi i / (16 NS)): six table twiddles, the other nine as products of two
+            static_assert(R == 16, "later stages");
+            const int k = (lt + b * U::TPR) & (NS - 1);
+            constexpr int step = N / (NS * R);
+            cplx<T> w[4], q[4];
+#pragma unroll
+            for (int r = 1; r < 4; r++) {
+                w[r] = tw[r * k * step];
+                q[r] = tw[4 * r * k * step];
+                if (!INV) {
+                    w[r].y = -w[r].y;
+                    q[r].y = -q[r].y;
+                }
+            }
+#pragma unroll
+            for (int r = 1; r < 16; r++) {
+                x[r] = cmul(x[r], r < 4 ? w[r & 3] : (r & 3) == 0 ? q[r >> 2] : cmul(q[r >> 2], w[r & 3]));
+                if ((r & 3) == 3)
+                    __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        if constexpr (R == 16)
+            bfly16<T, INV>(x);
+        else if constexpr (R == 8)
+            bfly8(x, INV);
+        else if constexpr (R == 4)
+            bfly4(x, INV);
+        else
+            bfly2(x);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (NS * R < N) {
+        T* row = s + vv;
+#pragma unroll
+        for (int part = 0; part < 2; part++) {
+            if (NS > 1 || part)
+                __syncthreads();  // the words before are read
+#pragma unroll
+            for (int b = 0; b < B; b++) {
+                const int j = lt + b * U::TPR, k = j & (NS - 1);
+                T* to = row + u_pad((j - k) * R + k) * U::NR;
+#pragma unroll
+                for (int r = 0; r < R; r++)
+                    to[u_pad(r * NS) * U::NR] = part ? v[b * R + r].y : v[b * R + r].x;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int b = 0; b < U::EPT / 16; b++) {
+                const T* from = row + u_pad(lt + b * U::TPR) * U::NR;
+#pragma unroll
+                for (int r = 0; r < 16; r++) {
+                    const T w = from[u_pad(r * (N / 16)) * U::NR];
+                    if (part)
+                        v[b * 16 + r].y = w;
+                    else
+                        v[b * 16 + r].x = w;
+                }
+            }
+        }
+        u_stages<T, N, INV, 16, NS * R>(v, s, lt, vv, tw);
+    }
+}
+
+template <typename T, int N, bool INV>
+__global__ __launch_bounds__((URow<T, N>::THREADS), 4) void fft_u(cplx<T>* grids, int rows, int per_xcd, size_t grid_elems,
+    const cplx<T>* tw)
+{
+    using U = URow<T, N>;
+    __shared__ T s[U::PADN * U::NR];
+    // consecutive row blocks on one XCD (workgroups go round the XCDs in turn)
+    const int rb = int(blockIdx.x & 7) * per_xcd + int(blockIdx.x >> 3);
+    if (rb * U::NR >= rows)
+        return;
+    const int vv = threadIdx.x % U::NR, lt = threadIdx.x / U::NR;
+    const bool on = rb * U::NR + vv < rows;
+    cplx<T>* g = grids + size_t(blockIdx.y) * grid_elems + size_t(rb) * U::NR;
+    const uint32_t at = uint32_t(lt) * uint32_t(rows) + uint32_t(vv);
+    cplx<T> v[U::EPT];
+    constexpr int R0 = U::FIRST;
+#pragma unroll
+    for (int b = 0; b < U::EPT / R0; b++)
+#pragma unroll
+        for (int r = 0; r < R0; r++) {
+            v[b * R0 + r] = { T(0), T(0) };
+            if (on)
+                v[b * R0 + r] = (g + size_t(b * U::TPR + r * (N / R0)) * rows)[at];
+        }
+    u_stages<T, N, INV, R0, 1>(v, s, lt, vv, tw);
+    constexpr int RL = N == R0 ? R0 : 16;
+    if (on) {
+#pragma unroll
+        for (int b = 0; b < U::EPT / RL; b++)
+#pragma unroll
+            for (int r = 0; r < RL; r++)
+                (g + size_t(b * U::TPR + r * (N / RL)) * rows)[at] = v[b * RL + r];
+    }
+}
 
 // U1: for each u2 and block of NT rows, FFT over u1 (stride L2 columns), then
 // multiply by exp(+-2 pi i k1 u2 / N).
@@ -686,14 +870,13 @@ __global__ __launch_bounds__(WG) void fft_cols_c2c(const cplx<T>* in, int rows, 
             out[size_t(x) * rows + r] = b[r];
 }
 
-// N = L1 * L2 for the four-step u transform: `req` when it is a valid split
-// (both factors in [2, 128]), otherwise the balanced one.
-template <typename T>
-void split_len(int N, int& L1, int& L2, int req = 0)
+// N = L1 * L2 of the slot order that launch_u_passes leaves: natural (1 x N) after one
+// pass, else the balanced four-step split.
+void split_len(int N, int& L1, int& L2)
 {
-    if (req >= 2 && req <= 128 && (req & (req - 1)) == 0 && N % req == 0 && N / req >= 2 && N / req <= 128) {
-        L1 = req;
-        L2 = N / req;
+    if (N >= 16 && N <= 8192) {
+        L1 = 1;
+        L2 = N;
         return;
     }
     int lg = 0;
@@ -703,22 +886,39 @@ void split_len(int N, int& L1, int& L2, int req = 0)
     L2 = N / L1;
 }
 
-#define STP_POW2_CASES(X) X(2) X(4) X(8) X(16) X(32) X(64) X(128)
+template <typename T, int N, bool INV>
+void launch_u(stp_ctx* ctx, cplx<T>* grids, int nbatch, int rows, size_t grid_elems, const T* tw)
+{
+    using namespace stp_hip;
+    const unsigned per_xcd = div_up(div_up(rows, URow<T, N>::NR), 8);
+    launch(ctx, "fft_u", fft_u<T, N, INV>, dim3(8 * per_xcd, nbatch), dim3(URow<T, N>::THREADS), 0, grids, rows, int(per_xcd),
+        grid_elems, (const cplx<T>*)tw);
+}
 
 template <typename T>
-void launch_u_passes(stp_ctx* ctx, cplx<T>* grids, int nbatch, int rows, int N, size_t grid_elems, const T* tw, bool inverse,
-    int req_l1 = 0)
+void launch_u_passes(stp_ctx* ctx, cplx<T>* grids, int nbatch, int rows, int N, size_t grid_elems, const T* tw, bool inverse)
 {
-    int L1, L2;
-    split_len<T>(N, L1, L2, req_l1);
     using namespace stp_hip;
+    switch (N) {
+#define UCASE(NN)                                                                 \
+    case NN:                                                                      \
+        if (inverse)                                                              \
+            launch_u<T, NN, true>(ctx, grids, nbatch, rows, grid_elems, tw);      \
+        else                                                                      \
+            launch_u<T, NN, false>(ctx, grids, nbatch, rows, grid_elems, tw);     \
+        return;
+        UCASE(16) UCASE(32) UCASE(64) UCASE(128) UCASE(256) UCASE(512) UCASE(1024) UCASE(2048) UCASE(4096) UCASE(8192)
+#undef UCASE
+    }
+    int L1, L2;
+    split_len(N, L1, L2);
     switch (L1) {
 #define U1CASE(LL)                                                                                          \
     case LL:                                                                                                \
         launch(ctx, "fft_u1", fft_u1<T, LL>, dim3(L2, div_up(rows, UShape<LL>::NT), nbatch), dim3(WG), 0,   \
             grids, rows, N, L2, grid_elems, tw, int(inverse));                                              \
         break;
-        STP_POW2_CASES(U1CASE)
+        U1CASE(2) U1CASE(4) U1CASE(128)
 #undef U1CASE
     default:
         throw Error(STP_ERR_UNSUPPORTED, "FFT length not supported: " + std::to_string(N));
@@ -729,7 +929,7 @@ void launch_u_passes(stp_ctx* ctx, cplx<T>* grids, int nbatch, int rows, int N, 
         launch(ctx, "fft_u2", fft_u2<T, LL>, dim3(L1, div_up(rows, UShape<LL>::NT), nbatch), dim3(WG), 0,   \
             grids, rows, N, L1, grid_elems, tw, int(inverse));                                              \
         break;
-        STP_POW2_CASES(U2CASE)
+        U2CASE(2) U2CASE(128)
 #undef U2CASE
     default:
         throw Error(STP_ERR_UNSUPPORTED, "FFT length not supported: " + std::to_string(N));
@@ -749,9 +949,9 @@ void fft_c2r_2d(stp_ctx* ctx, cplx<T>* grids, int nbatch, int n_rows, int N, con
     const size_t grid_elems = size_t(rows) * N;
     const Twiddles& twu = twiddles_for(ctx, N);
     const T* tw = std::is_same<T, double>::value ? (const T*)twu.d : (const T*)twu.f;
-    launch_u_passes<T>(ctx, grids, nbatch, rows, N, grid_elems, tw, true, ns.u_l1);
+    launch_u_passes<T>(ctx, grids, nbatch, rows, N, grid_elems, tw, true);
     int L1, L2;
-    split_len<T>(N, L1, L2, ns.u_l1);
+    split_len(N, L1, L2);
     const Twiddles& twv = twiddles_for(ctx, n_rows);
     const T* tvn = std::is_same<T, double>::value ? (const T*)twv.d : (const T*)twv.f;
     STP_REQUIRE(nbatch >= 1 && nbatch <= (outs.tab ? 65535 : 4), "1 to 4 grids per FFT launch (65535 with an output table)");
@@ -779,9 +979,9 @@ void fft_c2r_2d_real(stp_ctx* ctx, cplx<T>* grids, int nbatch, int N, const OutP
     const size_t grid_elems = size_t(rows) * U;
     const Twiddles& twu = twiddles_for(ctx, U);
     const T* tw = std::is_same<T, double>::value ? (const T*)twu.d : (const T*)twu.f;
-    launch_u_passes<T>(ctx, grids, nbatch, rows, U, grid_elems, tw, true, 0);
+    launch_u_passes<T>(ctx, grids, nbatch, rows, U, grid_elems, tw, true);
     int L1, L2;
-    split_len<T>(U, L1, L2, 0);
+    split_len(U, L1, L2);
     const Twiddles& twv = twiddles_for(ctx, N);
     const T* tvn = std::is_same<T, double>::value ? (const T*)twv.d : (const T*)twv.f;
     const int M = N / 2;
@@ -808,7 +1008,7 @@ void fft_c2c_2d(stp_ctx* ctx, cplx<T>* data, cplx<T>* out, int N, bool forward)
     // rows: transform along columns index (u) for every row, in place (four-step)
     launch_u_passes<T>(ctx, data, 1, N, N, size_t(N) * N, tw, !forward);
     int L1, L2;
-    split_len<T>(N, L1, L2);
+    split_len(N, L1, L2);
     switch (N) {
 #define CCASE(LL)                                                                                           \
     case LL:                                                                                                \

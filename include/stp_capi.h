@@ -479,9 +479,9 @@ stp_status stp_host_free(stp_ctx* ctx, void* ptr);
 /* No reference counterpart.  With autotuning on, the first imaging call of a
  * shape (padded size, support, oversampling, kernel mode, precision, W planes,
  * visibility-count octave) times the gridder tile widths 16 / 32 / 64 columns
- * and the u-axis FFT splits next to the balanced one on that call's input and
- * keeps the fastest for the context; `tune_file` (NULL: none) is read at once
- * and appended with every new choice.  mode: 0 off, 1 tune new shapes. */
+ * on that call's input and keeps the fastest for the context; `tune_file`
+ * (NULL: none) is read at once and appended with every new choice.  fft_l1
+ * (a u-axis FFT split of older files, now without effect) is 0 in new choices.  mode: 0 off, 1 tune new shapes. */
 stp_status stp_ctx_set_autotune(stp_ctx* ctx, int32_t mode, const char* tune_file);
 /* The configuration chosen for a shape (tile_cols 0: none yet). */
 stp_status stp_ctx_get_tuning(stp_ctx* ctx, const stp_imager_pars* img_pars, const stp_wproj_pars* w_proj, size_t n_vis,

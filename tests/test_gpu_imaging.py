@@ -72,6 +72,29 @@ def test_gpu_fft_c2r(gpu, orc, n):
     assert peak_rel_err(out, ref) < 1e-12
 
 
+@pytest.mark.parametrize("n,cols", [(16, 16), (32, 16), (64, 32), (128, 64), (128, 128), (512, 256), (512, 512),
+                                    (2048, 1024), (4096, 2048), (8192, 4096)])
+def test_gpu_fft_c2r_narrow(gpu, n, cols):
+    """Lengths along u that differ from those along v: row blocks of every size with a last one
+    of a single row."""
+    rng = np.random.default_rng(n + cols)
+    g = rng.normal(size=(n // 2 + 1, cols)) + 1j * rng.normal(size=(n // 2 + 1, cols))
+    out = gpu.fft_c2r(g)
+    ref = (np.fft.irfftn(g.T, s=(cols, n), axes=(0, 1)) * n * cols).T
+    assert peak_rel_err(out, ref) < 1e-12
+
+
+@pytest.mark.parametrize("n", [16, 32, 64, 128, 256, 512, 1024, 2048, 8192])
+def test_gpu_fft_fp32(gpu, n):
+    """The FP32 transforms, complex image and packed real beam, against FP64: a few hundred
+    rounding errors of 2^-24 at most between them."""
+    snap = simdata.snapshot(n, 20.0, 4_000, 4, seed=820 + n, field_frac=0.4)
+    pars = capi.imager_pars(n, 20.0, kernel_support=1 if n < 64 else 3)
+    a = gpu.image_visibilities(snap["vis"], snap["weights"], snap["uvw"], pars)
+    b = gpu.image_visibilities(snap["vis"], snap["weights"], snap["uvw"], pars, precision=capi.PRECISION_FP32C)
+    assert peak_rel_err(b[0], a[0]) < 1e-5 and peak_rel_err(b[1], a[1]) < 1e-5
+
+
 @pytest.mark.parametrize("n,cols", [(16384, 64), (16384, 512)])
 def test_gpu_fft_c2r_16384(gpu, n, cols):
     """The 2^14-point c2r along v (the reference's production image size,

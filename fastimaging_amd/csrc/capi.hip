@@ -140,18 +140,22 @@ GridderArgs imager_args(stp_ctx* ctx, const stp_imager_pars* p, const stp_wproj_
     return a;
 }
 
-// Gridding correction table of the padded size (imager.h:96-213), or NULL when
+// Inverse of the gridding correction of the padded size (imager.h:96-213), or NULL when
 // the call has none.
-const double* gcf_table(stp_ctx* ctx, const stp_imager_pars* p, const stp_kernel_spec& kern)
+const double* inv_gcf_table(stp_ctx* ctx, const stp_imager_pars* p, const stp_kernel_spec& kern)
 {
     if (!p->gridding_correction)
         return nullptr;
     const int N = int(p->padded_image_size);
     const KernelFn kf = kernel_fn(kern);
     char key[192];
-    snprintf(key, sizeof(key), "gcf:%d:%.17g:%.17g:%.17g:%d:%d", kf.kind, kf.param, kf.width_g, kf.width_s, N, p->analytic_gcf);
-    return has_table(ctx, key) ? dev_table(ctx, key, {})
-                               : dev_table(ctx, key, img_dom_kernel(kf, size_t(N), false, p->analytic_gcf != 0));
+    snprintf(key, sizeof(key), "igcf:%d:%.17g:%.17g:%.17g:%d:%d", kf.kind, kf.param, kf.width_g, kf.width_s, N, p->analytic_gcf);
+    if (has_table(ctx, key))
+        return dev_table(ctx, key, {});
+    std::vector<double> t = img_dom_kernel(kf, size_t(N), false, p->analytic_gcf != 0);
+    for (double& g : t)
+        g = 1.0 / g;
+    return dev_table(ctx, key, t);
 }
 
 template <typename T, typename OT>
@@ -178,7 +182,7 @@ void run_imager(stp_ctx* ctx, const stp_imager_pars* p, const stp_wproj_pars* wp
     NormSpec ns;
     ns.image_size = int(p->image_size);
     ns.total_ptr = d_total;
-    ns.gcf = gcf_table(ctx, p, kern);
+    ns.inv_gcf = inv_gcf_table(ctx, p, kern);
     OutPtrs<OT> outs{};
     outs.p[0] = d_image;
     if (a.beam_packed) {
@@ -246,7 +250,7 @@ struct FusedChunk {
             b.total = totals + 2 * idx[q];
             b.ngood = (unsigned long long*)(totals + 2 * idx[q] + 1);
             groups[Shape{ int(p->padded_image_size), int(p->image_size), p->generate_beam ? 1 : 0,
-                       gcf_table(ctx, p, kern) }]
+                       inv_gcf_table(ctx, p, kern) }]
                 .push_back(q);
         }
         // grids: each group's vis grids contiguous in item order, then its packed beam grids
@@ -295,7 +299,7 @@ struct FusedChunk {
             NormSpec ns;
             ns.image_size = r.s.image;
             ns.total_tab = (const double* const*)(d_extra + r.tot_off);
-            ns.gcf = r.s.gcf;
+            ns.inv_gcf = r.s.gcf;
             OutPtrs<OT> outs{};
             outs.tab = (OT* const*)(d_extra + r.out_off);
             if (r.real)

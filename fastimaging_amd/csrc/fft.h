@@ -6,12 +6,12 @@
 namespace stp_hip {
 
 // Normalisation fused into the last c2r pass (imager.h:96-213, non-FFTSHIFT):
-// out(i, j) = img(oi, oj) / *total_ptr [/ (gcf[ii] * gcf[jj])], cropped from the
+// out(i, j) = img(oi, oj) / *total_ptr [* inv_gcf[ii] * inv_gcf[jj]], cropped from the
 // padded transform size to image_size.
 struct NormSpec {
     int image_size = 0;
     const double* total_ptr = nullptr; // device scalar; NULL = no scaling
-    const double* gcf = nullptr;       // device array of the padded size; NULL = none
+    const double* inv_gcf = nullptr;   // device array of the padded size, 1 / gcf; NULL = none
     const double* const* total_tab = nullptr; // device array: grid g's scalar (replaces total_ptr)
 };
 

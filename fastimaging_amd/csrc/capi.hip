@@ -178,8 +178,9 @@ void run_imager(stp_ctx* ctx, const stp_imager_pars* p, const stp_wproj_pars* wp
     const int rows = N / 2 + 1;
     const size_t ge = size_t(rows) * N, gb = a.beam_packed ? ge / N * (N / 2) : ge;
     cplx<T>* grids = (cplx<T>*)ws_get(ctx, "imager_grids", sizeof(cplx<T>) * (ge + (beam ? gb : 0)));
-    grid_visibilities<T>(ctx, a, n, d_uvw, d_vis, d_w, grids, beam ? grids + ge : nullptr, d_total, d_ngood);
     NormSpec ns;
+    a.skip_empty = fft_reads_occ(N);
+    grid_visibilities<T>(ctx, a, n, d_uvw, d_vis, d_w, grids, beam ? grids + ge : nullptr, d_total, d_ngood, &ns.occ);
     ns.image_size = int(p->image_size);
     ns.total_ptr = d_total;
     ns.inv_gcf = inv_gcf_table(ctx, p, kern);
@@ -225,7 +226,7 @@ struct FusedChunk {
         cplx<T>* grids;
         int nbatch;
         bool real;       // packed real beam grids
-        size_t out_off, tot_off;
+        size_t out_off, tot_off, idx_off;
     };
     std::vector<Run> runs;
     BatchPlan plan;
@@ -242,6 +243,7 @@ struct FusedChunk {
             check_kernel_spec(&kern);
             BatchGridItem& b = bg[q];
             b.a = imager_args(ctx, p, nullptr, kern, it.n_vis, precision);
+            b.a.skip_empty = fft_reads_occ(int(p->padded_image_size));
             b.a.beam_packed = p->generate_beam != 0;  // eligible snapshots: no W-projection, N >= 8
             b.n = it.n_vis;
             b.uv = it.d_uvw_lambda;
@@ -266,7 +268,7 @@ struct FusedChunk {
         size_t cur = 0;
         auto add_run = [&](const Shape& s, bool real, const std::vector<size_t>& members) {
             const size_t ge = size_t(s.N / 2 + 1) * (real ? s.N / 2 : s.N);
-            Run r{ s, grids + cur, int(members.size()), real, 0, 0 };
+            Run r{ s, grids + cur, int(members.size()), real, 0, 0, 0 };
             std::vector<OT*> outs;
             std::vector<const double*> tots;
             for (size_t q : members) {
@@ -280,6 +282,10 @@ struct FusedChunk {
             extra.insert(extra.end(), (const uint8_t*)outs.data(), (const uint8_t*)(outs.data() + outs.size()));
             r.tot_off = extra.size();
             extra.insert(extra.end(), (const uint8_t*)tots.data(), (const uint8_t*)(tots.data() + tots.size()));
+            std::vector<uint32_t> rec(members.begin(), members.end());
+            rec.resize((rec.size() + 1) & ~size_t(1)); // the pointers after it stay aligned
+            r.idx_off = extra.size();
+            extra.insert(extra.end(), (const uint8_t*)rec.data(), (const uint8_t*)(rec.data() + rec.size()));
             runs.push_back(r);
         };
         for (auto& gr : groups) {
@@ -299,6 +305,8 @@ struct FusedChunk {
             NormSpec ns;
             ns.image_size = r.s.image;
             ns.total_tab = (const double* const*)(d_extra + r.tot_off);
+            ns.occ_tab = plan.d_occ;
+            ns.occ_idx = (const uint32_t*)(d_extra + r.idx_off);
             ns.inv_gcf = r.s.gcf;
             OutPtrs<OT> outs{};
             outs.tab = (OT* const*)(d_extra + r.out_off);

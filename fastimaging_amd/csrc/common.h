@@ -51,6 +51,15 @@ struct TimingAcc {
     uint64_t count = 0;
 };
 
+// Which tiles of a grid hold entries: totals[rt + ct * tiles_r] entries in the tile of rows
+// 64 rt .. and columns ct << tc_log .. (cells of the others are zero and need not have
+// been written).  totals NULL: every cell is written.
+constexpr int OCC_ROWS = 64;
+struct TileOcc {
+    const uint32_t* totals = nullptr;
+    int tiles_r = 0, tc_log = 0;
+};
+
 // Launch configuration picked by the autotuner for one imaging shape.
 struct TuneChoice {
     int tile_cols = 0; // gridder tile width

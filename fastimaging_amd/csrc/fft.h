@@ -13,6 +13,10 @@ struct NormSpec {
     const double* total_ptr = nullptr; // device scalar; NULL = no scaling
     const double* inv_gcf = nullptr;   // device array of the padded size, 1 / gcf; NULL = none
     const double* const* total_tab = nullptr; // device array: grid g's scalar (replaces total_ptr)
+    // tiles of the grid that hold entries; grid g's in occ_tab[occ_idx[g]] when these are set
+    TileOcc occ;
+    const TileOcc* occ_tab = nullptr;
+    const uint32_t* occ_idx = nullptr;
 };
 
 // Outputs of the batch's grids: p[g] for up to 4 grids, or the device array tab.
@@ -39,5 +43,12 @@ void fft_c2r_2d_real(stp_ctx* ctx, cplx<T>* grids, int nbatch, int N, const OutP
 // overwritten, results in `out`.
 template <typename T>
 void fft_c2c_2d(stp_ctx* ctx, cplx<T>* data, cplx<T>* out, int N, bool forward);
+
+// Whether the c2r of size N takes empty tiles as zero (NormSpec::occ) instead of reading
+// them.  The look at the tile counts costs a workgroup about a microsecond before its
+// loads: with a third of the tiles empty, tile sums and u pass together take 261 against
+// 282 us at 4096 FP64, 676 against 695 us at 8192 FP32, 170 against 174 us at 4096 FP32,
+// but 41.5 against 41.0 us at 1024 FP64.  Above 8192 the u pass has two halves.
+constexpr bool fft_reads_occ(int N) { return N >= 4096 && N <= 8192; }
 
 } // namespace stp_hip

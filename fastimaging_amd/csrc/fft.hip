@@ -24,7 +24,9 @@
 namespace {
 
 using stp_hip::NormSpec;
+using stp_hip::OCC_ROWS;
 using stp_hip::OutPtrs;
+using stp_hip::TileOcc;
 
 constexpr int WG = 256;
 
@@ -314,7 +316,7 @@ struct UShape {
 // third of the time, stores), which overlap little while one image's rows fit the chip at
 // once.  N=4096 half plane with its half-length beam: 72 us FP32, 130 us FP64, against 87
 // and 166 us for two passes of the four-step split (fft_u1, fft_u2), with a launch less per
-// grid; 8192 FP32 236 us against 247 us.  Two FP32 rows per workgroup take 338 us at 8192
+// grid; 8192 FP32 236 us against 247 us (every tile read).  Two FP32 rows per workgroup take 338 us at 8192
 // and two FP64 rows 144 us at 4096 (shorter runs); the whole complex row in LDS would
 // leave half as many rows per CU.
 template <typename T, int N>
@@ -410,9 +412,18 @@ __device__ __forceinline__ void u_stages(cplx<T>* v, T* s, int lt, int vv, const
     }
 }
 
+// Occupied tiles of the grids (NormSpec): columns of a packed grid are 1 << pack grid
+// columns.
+struct UOcc {
+    TileOcc one;
+    const TileOcc* tab = nullptr;
+    const uint32_t* idx = nullptr;
+    int pack = 0;
+};
+
 template <typename T, int N, bool INV>
 __global__ __launch_bounds__((URow<T, N>::THREADS), 4) void fft_u(cplx<T>* grids, int rows, int per_xcd, size_t grid_elems,
-    const cplx<T>* tw)
+    const cplx<T>* tw, UOcc uo)
 {
     using U = URow<T, N>;
     __shared__ T s[U::PADN * U::NR];
@@ -423,6 +434,23 @@ __global__ __launch_bounds__((URow<T, N>::THREADS), 4) void fft_u(cplx<T>* grids
     const int vv = threadIdx.x % U::NR, lt = threadIdx.x / U::NR;
     const bool on = rb * U::NR + vv < rows;
     cplx<T>* g = grids + size_t(blockIdx.y) * grid_elems + size_t(rb) * U::NR;
+    // bit i: the tile of the thread's element i holds entries
+    static_assert(OCC_ROWS % U::NR == 0, "a row block lies in one row of tiles");
+    uint32_t full = ~0u;
+    if constexpr (N >= 2048) { // fft_reads_occ
+        const TileOcc occ = uo.tab ? uo.tab[uo.idx[blockIdx.y]] : uo.one;
+        if (occ.totals) {
+            const uint32_t* tot = occ.totals + rb * U::NR / OCC_ROWS;
+            full = 0;
+#pragma unroll
+            for (int b = 0; b < U::EPT / U::FIRST; b++)
+#pragma unroll
+                for (int r = 0; r < U::FIRST; r++) {
+                    const int c = (lt + b * U::TPR + r * (N / U::FIRST)) << uo.pack;
+                    full |= (tot[(c >> occ.tc_log) * occ.tiles_r] != 0 ? 1u : 0u) << (b * U::FIRST + r);
+                }
+        }
+    }
     const uint32_t at = uint32_t(lt) * uint32_t(rows) + uint32_t(vv);
     cplx<T> v[U::EPT];
     constexpr int R0 = U::FIRST;
@@ -431,7 +459,7 @@ __global__ __launch_bounds__((URow<T, N>::THREADS), 4) void fft_u(cplx<T>* grids
 #pragma unroll
         for (int r = 0; r < R0; r++) {
             v[b * R0 + r] = { T(0), T(0) };
-            if (on)
+            if (on && (full >> (b * R0 + r) & 1u))
                 v[b * R0 + r] = (g + size_t(b * U::TPR + r * (N / R0)) * rows)[at];
         }
     u_stages<T, N, INV, R0, 1>(v, s, lt, vv, tw);
@@ -886,25 +914,26 @@ void split_len(int N, int& L1, int& L2)
 }
 
 template <typename T, int N, bool INV>
-void launch_u(stp_ctx* ctx, cplx<T>* grids, int nbatch, int rows, size_t grid_elems, const T* tw)
+void launch_u(stp_ctx* ctx, cplx<T>* grids, int nbatch, int rows, size_t grid_elems, const T* tw, const UOcc& uo)
 {
     using namespace stp_hip;
     const unsigned per_xcd = div_up(div_up(rows, URow<T, N>::NR), 8);
     launch(ctx, "fft_u", fft_u<T, N, INV>, dim3(8 * per_xcd, nbatch), dim3(URow<T, N>::THREADS), 0, grids, rows, int(per_xcd),
-        grid_elems, (const cplx<T>*)tw);
+        grid_elems, (const cplx<T>*)tw, uo);
 }
 
 template <typename T>
-void launch_u_passes(stp_ctx* ctx, cplx<T>* grids, int nbatch, int rows, int N, size_t grid_elems, const T* tw, bool inverse)
+void launch_u_passes(stp_ctx* ctx, cplx<T>* grids, int nbatch, int rows, int N, size_t grid_elems, const T* tw, bool inverse,
+    const UOcc& uo = {})
 {
     using namespace stp_hip;
     switch (N) {
 #define UCASE(NN)                                                                 \
     case NN:                                                                      \
         if (inverse)                                                              \
-            launch_u<T, NN, true>(ctx, grids, nbatch, rows, grid_elems, tw);      \
+            launch_u<T, NN, true>(ctx, grids, nbatch, rows, grid_elems, tw, uo);  \
         else                                                                      \
-            launch_u<T, NN, false>(ctx, grids, nbatch, rows, grid_elems, tw);     \
+            launch_u<T, NN, false>(ctx, grids, nbatch, rows, grid_elems, tw, uo); \
         return;
         UCASE(16) UCASE(32) UCASE(64) UCASE(128) UCASE(256) UCASE(512) UCASE(1024) UCASE(2048) UCASE(4096) UCASE(8192)
 #undef UCASE
@@ -948,7 +977,7 @@ void fft_c2r_2d(stp_ctx* ctx, cplx<T>* grids, int nbatch, int n_rows, int N, con
     const size_t grid_elems = size_t(rows) * N;
     const Twiddles& twu = twiddles_for(ctx, N);
     const T* tw = std::is_same<T, double>::value ? (const T*)twu.d : (const T*)twu.f;
-    launch_u_passes<T>(ctx, grids, nbatch, rows, N, grid_elems, tw, true);
+    launch_u_passes<T>(ctx, grids, nbatch, rows, N, grid_elems, tw, true, UOcc{ ns.occ, ns.occ_tab, ns.occ_idx, 0 });
     int L1, L2;
     split_len(N, L1, L2);
     const Twiddles& twv = twiddles_for(ctx, n_rows);
@@ -978,7 +1007,7 @@ void fft_c2r_2d_real(stp_ctx* ctx, cplx<T>* grids, int nbatch, int N, const OutP
     const size_t grid_elems = size_t(rows) * U;
     const Twiddles& twu = twiddles_for(ctx, U);
     const T* tw = std::is_same<T, double>::value ? (const T*)twu.d : (const T*)twu.f;
-    launch_u_passes<T>(ctx, grids, nbatch, rows, U, grid_elems, tw, true);
+    launch_u_passes<T>(ctx, grids, nbatch, rows, U, grid_elems, tw, true, UOcc{ ns.occ, ns.occ_tab, ns.occ_idx, 1 });
     int L1, L2;
     split_len(U, L1, L2);
     const Twiddles& twv = twiddles_for(ctx, N);

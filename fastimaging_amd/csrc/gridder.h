@@ -23,6 +23,8 @@ struct GridderArgs {
     int tile_cols = 0;      // tile width (16, 32 or 64 grid columns); 0 = default
     bool beam_packed = false; // sampling grid as packed real values: rows x N/2 complex, element (v, u') =
                               // (G(v, 2u'), G(v, 2u'+1)) (the kernels are real without W-projection)
+    bool skip_empty = false;  // cells of tiles without entries need not be written; the tiles in occ (or
+                              // BatchPlan::d_occ), if the path knows them
     unsigned long long* d_nentries = nullptr; // device u64: receives the gridding entries written (may be NULL)
 };
 
@@ -33,7 +35,8 @@ struct GridderArgs {
 // be NULL.
 template <typename T>
 void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const double* d_uv, const double* d_vis,
-    const double* d_w, cplx<T>* d_vis_grid, cplx<T>* d_sampling_grid, double* d_total, unsigned long long* d_ngood);
+    const double* d_w, cplx<T>* d_vis_grid, cplx<T>* d_sampling_grid, double* d_total, unsigned long long* d_ngood,
+    TileOcc* occ = nullptr);
 
 // One snapshot of a fused batch (grid_batch): its arguments, inputs, grids and
 // the device scalars that receive sample_grid_total and the good count.
@@ -70,6 +73,7 @@ struct BatchPlan {
     static constexpr int CLASSES = 6;  // tile width (16, 32, 64); two-float: x kernel width (8 or 16 taps)
     const void* d_tab = nullptr;       // device tables (snapshot records first)
     const void* d_extra = nullptr;     // the caller's tables
+    const TileOcc* d_occ = nullptr;    // per snapshot
     int items = 0;
     bool twofloat = false;
     size_t pre_t_off = 0;              // byte offset of the tile-class prefixes in d_tab

@@ -32,6 +32,7 @@ namespace stp_hip {
 namespace {
 
 constexpr int TILE_R = 64;  // grid rows (v) per tile: 64 contiguous complex per column
+static_assert(TILE_R == OCC_ROWS, "rows of TileOcc");
 constexpr int W_TILE_C = 64; // with W-projection: its wide footprints touch fewer tiles
 constexpr int TILE_C = 32;  // default grid columns (u) per tile; GridderArgs::tile_cols overrides
 constexpr int GWG = 256;
@@ -40,6 +41,7 @@ struct GridGeom {
     int N, rows, half, s, ks, os;
     int halfplane, shift, exact, beam;
     int bpack = 0; // beam grid packed real (rows x N/2 complex: columns 2u', 2u'+1)
+    int skip = 0;  // cells of tiles without entries are not written
     int tiles_r, tiles_c;
     int tc;       // tile width in grid columns (TILE_R rows per tile)
     double scale;
@@ -1110,6 +1112,8 @@ __device__ __forceinline__ void tiles_mfma_body(const GridGeom& g, Entry* entrie
     // complex (imaginary part 0) or, with g.bpack, packed real: cell (r, c) is component
     // c & 1 of element (r, c / 2) of a rows x N/2 complex array
     const bool some = eb < ee;
+    if (!some && g.skip)
+        return;
     double* o0 = area;
     double* o1 = area + TC * OUT_STRIDE;
     if (some) {
@@ -2778,7 +2782,7 @@ static void twofloat_tiles(stp_ctx* ctx, const GridGeom& g, int cs, const Entry*
 
 template <typename T>
 void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const double* d_uv, const double* d_vis,
-    const double* d_w, cplx<T>* d_vis_grid, cplx<T>* d_sampling_grid, double* d_total, unsigned long long* d_ngood)
+    const double* d_w, cplx<T>* d_vis_grid, cplx<T>* d_sampling_grid, double* d_total, unsigned long long* d_ngood, TileOcc* occ)
 {
     const bool wproj = a.wproj.num_wplanes > 0;
     KernelFn kf;
@@ -2996,6 +3000,10 @@ void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const doubl
             totals);
         launch(ctx, "grid_scatter", grid_bin_scatter_kernel, dim3(unsigned(nblk)), dim3(BWG), hist_bytes, g, d_uv, d_vis, d_w,
             (const uint32_t*)totals, (const uint32_t*)counts, entries, cap, toffs, ext_host);
+        if (mfma && a.skip_empty && occ) {
+            g.skip = 1;
+            *occ = { totals, g.tiles_r, __builtin_ctz(unsigned(g.tc)) };
+        }
         offsets = toffs;
         ostride = 1;
         bcur = counts;
@@ -3126,6 +3134,7 @@ BatchPlan grid_batch_bin(stp_ctx* ctx, const std::vector<BatchGridItem>& items, 
         b.bgrid = g.beam ? it.bgrid : nullptr;
         b.total = it.total;
         b.ngood = it.ngood;
+        b.g.skip = it.a.skip_empty && !twofloat ? 1 : 0;
         b.cap = uint32_t(cap64);
         b.nblk = int(nblk);
         Place& p = pl[k];
@@ -3165,17 +3174,20 @@ BatchPlan grid_batch_bin(stp_ctx* ctx, const std::vector<BatchGridItem>& items, 
     STP_REQUIRE(nb < (size_t(1) << 31) && *std::max_element(nt, nt + NCLS) < (size_t(1) << 31),
         "too many workgroups for one fused batch");
     uint8_t* base = (uint8_t*)ws_get(ctx, "bat_pool", pool);
+    std::vector<TileOcc> occ(K);
     for (int k = 0; k < K; k++) {
         bi[k].counts = (uint32_t*)(base + pl[k].counts);
         bi[k].totals = (uint32_t*)(base + pl[k].totals);
         bi[k].toffs = (uint32_t*)(base + pl[k].toffs);
         bi[k].wpart = (double*)(base + pl[k].wpart);
         bi[k].entries = (Entry*)(base + pl[k].entries);
+        if (bi[k].g.skip)
+            occ[k] = { bi[k].totals, bi[k].g.tiles_r, __builtin_ctz(unsigned(bi[k].g.tc)) };
     }
-    // tables: items, the stage prefixes, the caller's tables; one upload from the
+    // tables: items, the stage prefixes, the occupied tiles, the caller's tables; one upload from the
     // page-locked stage once the previous batch's upload has left it
     const size_t o_items = 0, o_b = al(sizeof(BItem) * K), o_c = o_b + al(4 * K), o_t = o_c + al(4 * K);
-    const size_t o_m = o_t + al(4 * size_t(NCLS) * K), o_x = o_m + al(4 * K), tab_bytes = o_x + std::max<size_t>(extra.size(), 1);
+    const size_t o_m = o_t + al(4 * size_t(NCLS) * K), o_o = o_m + al(4 * K), o_x = o_o + al(sizeof(TileOcc) * K), tab_bytes = o_x + std::max<size_t>(extra.size(), 1);
     hipEvent_t& up = ctx->batch_tab_events[ctx->ws_slot];
     if (!up)
         HIP_CHECK(hipEventCreateWithFlags(&up, hipEventDisableTiming));
@@ -3187,6 +3199,7 @@ BatchPlan grid_batch_bin(stp_ctx* ctx, const std::vector<BatchGridItem>& items, 
     memcpy(h + o_c, pre_c.data(), 4 * K);
     memcpy(h + o_t, pre_t.data(), 4 * size_t(NCLS) * K);
     memcpy(h + o_m, pre_m.data(), 4 * K);
+    memcpy(h + o_o, occ.data(), sizeof(TileOcc) * K);
     if (!extra.empty())
         memcpy(h + o_x, extra.data(), extra.size());
     HIP_CHECK(hipMemcpyAsync(d, h, tab_bytes, hipMemcpyHostToDevice, ctx->stream));
@@ -3201,6 +3214,7 @@ BatchPlan grid_batch_bin(stp_ctx* ctx, const std::vector<BatchGridItem>& items, 
     BatchPlan plan;
     plan.d_tab = d;
     plan.d_extra = d + o_x;
+    plan.d_occ = (const TileOcc*)(d + o_o);
     plan.items = K;
     plan.twofloat = twofloat;
     plan.pre_t_off = o_t;
@@ -3271,8 +3285,8 @@ size_t gridder_entry_capacity(int N, bool halfplane, int support, bool exact, in
 }
 
 template void grid_visibilities<double>(stp_ctx*, const GridderArgs&, size_t, const double*, const double*,
-    const double*, cplx<double>*, cplx<double>*, double*, unsigned long long*);
+    const double*, cplx<double>*, cplx<double>*, double*, unsigned long long*, TileOcc*);
 template void grid_visibilities<float>(stp_ctx*, const GridderArgs&, size_t, const double*, const double*,
-    const double*, cplx<float>*, cplx<float>*, double*, unsigned long long*);
+    const double*, cplx<float>*, cplx<float>*, double*, unsigned long long*, TileOcc*);
 
 } // namespace stp_hip

@@ -284,3 +284,24 @@ def test_fused_batch_only_eligible_and_autotuned(gpu, orc):
             assert peak_rel_err(got[k][0], oimg) < 1e-4 and peak_rel_err(got[k][1], obeam) < 1e-4, k
     finally:
         b.free()
+
+
+@pytest.mark.parametrize("precision", [capi.PRECISION_FP64, capi.PRECISION_FP32C])
+def test_batch_empty_tiles(gpu, precision):
+    """A batch of 4096^2 snapshots with few and many occupied tiles beside smaller ones, eager and
+    as a graph replayed with other batches between, against the single calls."""
+    b = _Batch(gpu, [(4096, 1.0, 3, 1, 711, None, 0.0), (512, 2.0, 900, 2, 712, None, 0.0),
+                     (4096, 1.0, 40_000, 3, 713, None, 0.0), (4096, 1.0, 60, 1, 714, None, 0.0)], precision)
+    try:
+        for it in b.items:
+            gpu.image_visibilities_device(it.img_pars, it.n_vis, it.d_vis, it.d_vis_weights, it.d_uvw_lambda,
+                                          it.d_image, it.d_beam, precision=precision, synchronize=True)
+        single = b.images()
+        tol = 1e-12 if precision == capi.PRECISION_FP64 else 1e-6
+        for flags in (0, capi.BATCH_GRAPH, 0, capi.BATCH_GRAPH):
+            b.clear()
+            gpu.image_batch(b.items[::-1] if flags == 0 else b.items, precision=precision, max_concurrent=3, flags=flags)
+            for (a, ab), (c, cb) in zip(single, b.images()):
+                assert peak_rel_err(c, a) <= tol and peak_rel_err(cb, ab) <= tol
+    finally:
+        b.free()

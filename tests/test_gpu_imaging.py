@@ -259,3 +259,22 @@ def test_gpu_beam_real_transform(gpu, orc, N, padding, gcf, precision):
     if padding == 1.0:
         refl = np.roll(np.roll(beam[::-1, ::-1], 1, axis=0), 1, axis=1)  # B(-y, -x)
         assert np.max(np.abs(refl - beam)) <= (1e-12 if precision == capi.PRECISION_FP64 else 1e-5) * np.max(np.abs(beam))
+
+
+@pytest.mark.parametrize("precision", [capi.PRECISION_FP64, capi.PRECISION_FP32C])
+def test_gpu_empty_tiles(gpu, orc, precision):
+    """4096^2 images whose grid is almost empty, after one that filled the same workspace: cells of
+    tiles without entries are not written, so none may be read.  One visibility, and two at opposite
+    corners of the grid."""
+    N, cell = 4096, 1.0
+    lam = N / (N * cell / 3600.0 * np.pi / 180.0) * 0.5
+    pars = capi.imager_pars(N, cell)
+    full = simdata.snapshot(N, cell, 30_000, 3, seed=830)
+    one = dict(uvw=np.asfortranarray([[0.3 * lam, 0.4 * lam, 0.0]]), vis=np.array([1.0 - 2.0j]), weights=np.ones(1))
+    two = dict(uvw=np.asfortranarray([[0.99 * lam, 0.98 * lam, 0.0], [-0.99 * lam, 0.01 * lam, 0.0]]),
+               vis=np.array([0.5 + 1.0j, 2.0 + 0.0j]), weights=np.array([1.0, 0.25]))
+    tol = TOL if precision == capi.PRECISION_FP64 else 1e-5
+    for s in (full, one, two):
+        img, beam = gpu.image_visibilities(s["vis"], s["weights"], s["uvw"], pars, precision=precision)
+        oimg, obeam, _, _ = orc.image_visibilities(pars, s["vis"], s["weights"], s["uvw"])
+        assert peak_rel_err(img, oimg) < tol and peak_rel_err(beam, obeam) < tol

@@ -278,3 +278,26 @@ def test_gpu_empty_tiles(gpu, orc, precision):
         img, beam = gpu.image_visibilities(s["vis"], s["weights"], s["uvw"], pars, precision=precision)
         oimg, obeam, _, _ = orc.image_visibilities(pars, s["vis"], s["weights"], s["uvw"])
         assert peak_rel_err(img, oimg) < tol and peak_rel_err(beam, obeam) < tol
+
+
+@pytest.mark.parametrize("n,beam,precision", [(2_000, True, capi.PRECISION_FP64), (30_000, False, capi.PRECISION_FP64),
+                                              (30_000, False, capi.PRECISION_FP32C), (130_000, False, capi.PRECISION_FP64),
+                                              (1, True, capi.PRECISION_FP32C), (0, False, capi.PRECISION_FP64)])
+def test_gpu_host_call_staging(gpu, orc, n, beam, precision):
+    """Host calls through the page-locked buffers (up to 14 MB) and past them, against the oracle;
+    no good visibility leaves the images empty, and the next call is a full one again."""
+    size = 256 if beam else 1024
+    pars = capi.imager_pars(size, 2.0, generate_beam=beam)
+    snap = simdata.snapshot(size, 2.0, max(n, 1), 2, seed=850)
+    vis, w, uvw = snap["vis"][:n], snap["weights"][:n], snap["uvw"][:n]
+    oimg, obeam, _, _ = orc.image_visibilities(pars, vis, w, uvw) if n else (None,) * 4
+    tol = TOL if precision == capi.PRECISION_FP64 else 1e-4
+    for weights in (w, np.zeros(n), w):
+        img, beam_out, diag = gpu.image_visibilities(vis, weights, uvw, pars, precision=precision, return_diag=True)
+        if n == 0 or not weights.any():
+            assert img.size == 0 and diag.image_rows == 0
+            continue
+        assert diag.num_good_vis == n and diag.image_rows == size
+        assert peak_rel_err(img, oimg) < tol
+        if beam:
+            assert peak_rel_err(beam_out, obeam) < tol

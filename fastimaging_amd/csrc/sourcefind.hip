@@ -1248,9 +1248,17 @@ __global__ __launch_bounds__(CU_THREADS) void sf_clip_last(SFState* st, const do
 // Label ids are ranks of roots in key order: a 64-bit root mask per segment (one
 // tile's rows of one column) and a scan of the segment counts give every root's
 // id without a pass over the image.
-constexpr int CT_W = 64, CT_H = 64, CT_PIX = CT_W * CT_H, CT_THREADS = 1024, CT_WAVES = CT_THREADS / 64;
-constexpr int CT_PPT = CT_PIX / CT_THREADS;  // pixels per thread: columns w + CT_WAVES j, row = lane
-constexpr int CT_RCAP = 480;  // components of a tile summed in LDS; more go to global atomics
+// A tile's phases over its list are chains of LDS accesses and barriers, so ccl_tile is
+// bound by how many tiles a CU holds: 512 threads and 52 KB (lists of 16 bits, run ends from the
+// class masks) let three in, 107 -> 59 us at 4096 x 4096 (57 -> 38 us at 3000 x 2600 FP64)
+// against two of 1024 threads and 70 KB.  A tile of its own CU is done sooner by 1024
+// threads: up to 256 tiles take those (208 tiles 11.6 against 13.0 us).
+constexpr int CT_W = 64, CT_H = 64, CT_PIX = CT_W * CT_H;
+constexpr unsigned CT_FEW = 256;
+// Components of a tile summed in LDS; more go to global atomics: with room for 208 (four
+// tiles of 512 threads to a CU) 4096 x 4096 took 299 instead of 307 us in all, but a 1024 x
+// 1024 snapshot, whose tiles hold more, 333 instead of 306 us.
+constexpr int ct_rcap(int threads) { return threads == 1024 ? 480 : 384; }
 constexpr uint32_t P_BG = 0xFFFFFFFFu, P_OPEN = 0x80000000u, P_NEG = 0x40000000u, P_KEY = 0x3FFFFFFFu;
 constexpr uint32_t L_KEY = 0xFFFu, L_OPEN = 0x1000u;
 
@@ -1424,15 +1432,16 @@ __device__ void g_union(uint32_t* P, uint32_t a, uint32_t b, uint32_t flags)
     } while (!done);
 }
 
-template <typename T>
-__global__ __launch_bounds__(CT_THREADS) void ccl_tile(const T* __restrict__ x, TileGeom g, const SFState* st, int find_neg,
+template <typename T, int CT_THREADS>
+__global__ __launch_bounds__(CT_THREADS, 8) void ccl_tile(const T* __restrict__ x, TileGeom g, const SFState* st, int find_neg,
     int conn4, uint32_t* __restrict__ P, unsigned long long* __restrict__ rmask, CompRecords rec)
 {
+    constexpr int CT_RCAP = ct_rcap(CT_THREADS);
+    constexpr int CT_WAVES = CT_THREADS / 64, CT_PPT = CT_PIX / CT_THREADS;  // pixels per thread: columns w + CT_WAVES j, row = lane
     __shared__ uint32_t s_par[CT_PIX];
-    __shared__ uint32_t s_list[CT_PIX];  // foreground pixels in key order: li | class << 12 | run start << 14 | run end << 20
-    __shared__ uint8_t s_cls[CT_PIX];
+    __shared__ uint16_t s_list[CT_PIX];  // foreground pixels in key order: li | class << 12
     __shared__ uint8_t s_fl[CT_H + 2], s_fr[CT_H + 2], s_ft[CT_W], s_fb[CT_W];
-    __shared__ unsigned long long s_mask[CT_W];        // foreground of each column
+    __shared__ unsigned long long s_mask[2][CT_W];     // pixels of each class in each column
     __shared__ unsigned long long s_rmp[CT_W], s_rmn[CT_W];  // closed roots of each column
     __shared__ uint32_t s_pre[CT_W + 1];
     __shared__ uint32_t s_base, s_nroot;
@@ -1451,9 +1460,19 @@ __global__ __launch_bounds__(CT_THREADS) void ccl_tile(const T* __restrict__ x, 
     auto pix = [&](int cv, int vr) -> double { return ldv(x, size_t(mem_col(g, cv)) * size_t(g.R) + size_t(flip_row(g, vr))); };
     auto mem_index = [&](int c, int rr) -> uint32_t { return uint32_t(mem_col(g, cv0 + c)) * uint32_t(g.R) + uint32_t(rbase + rr); };
     const unsigned long long lt = (1ull << lane) - 1ull;
+    // first and last row of the run of mask m that holds row r
+    auto run_start = [](unsigned long long m, int r) -> int {
+        const unsigned long long z = ~m & ((1ull << r) - 1ull);
+        return z ? 64 - __builtin_clzll(z) : 0;
+    };
+    auto run_end = [](unsigned long long m, int r) -> int {
+        const unsigned long long z = ~m & ~((2ull << r) - 1ull);
+        return z ? __builtin_ctzll(z) - 1 : 63;
+    };
 
     // 1. classification and vertical runs (a wave holds one tile column per step)
-    uint32_t info[CT_PPT];  // class | run start << 2 | run end << 8
+    uint32_t info = 0;  // classes, two bits each
+    static_assert(2 * CT_PPT <= 32, "classes of a thread");
 #pragma unroll
     for (int j = 0; j < CT_PPT; j++) {
         const int c = w + CT_WAVES * j, li = c * CT_H + lane;
@@ -1461,15 +1480,12 @@ __global__ __launch_bounds__(CT_THREADS) void ccl_tile(const T* __restrict__ x, 
         if (c < nc && lane < nr)
             cl = classify(ldv(x, size_t(mem_index(c, lane))));
         const unsigned long long m1 = __ballot(cl == 1u), m2 = __ballot(cl == 2u);
-        const unsigned long long M = cl == 2u ? m2 : m1;
-        const unsigned long long zb = ~M & lt, za = ~M & ~(lt | (1ull << lane));
-        const uint32_t rs = zb ? uint32_t(64 - __builtin_clzll(zb)) : 0u;
-        const uint32_t re = za ? uint32_t(__builtin_ctzll(za) - 1) : 63u;
-        info[j] = cl | (rs << 2) | (re << 8);
-        s_cls[li] = uint8_t(cl);
-        s_par[li] = uint32_t(c * CT_H) + (cl ? rs : uint32_t(lane));
-        if (lane == 0)
-            s_mask[c] = m1 | m2;
+        info |= cl << (2 * j);
+        s_par[li] = uint32_t(c * CT_H + (cl ? run_start(cl == 2u ? m2 : m1, lane) : lane));
+        if (lane == 0) {
+            s_mask[0][c] = m1;
+            s_mask[1][c] = m2;
+        }
     }
     if (t < CT_W) {
         s_rmp[t] = 0;
@@ -1499,7 +1515,7 @@ __global__ __launch_bounds__(CT_THREADS) void ccl_tile(const T* __restrict__ x, 
     __syncthreads();
     // list of the foreground pixels (key order)
     if (w == 0) {
-        const uint32_t cnt = uint32_t(__popcll(s_mask[lane]));
+        const uint32_t cnt = uint32_t(__popcll(s_mask[0][lane] | s_mask[1][lane]));
         uint32_t incl = cnt;
         for (int off = 1; off < 64; off <<= 1) {
             const uint32_t o = __shfl_up(incl, off);
@@ -1514,9 +1530,9 @@ __global__ __launch_bounds__(CT_THREADS) void ccl_tile(const T* __restrict__ x, 
 #pragma unroll
     for (int j = 0; j < CT_PPT; j++) {
         const int c = w + CT_WAVES * j;
-        if (info[j] & 3u)
-            s_list[s_pre[c] + uint32_t(__popcll(s_mask[c] & lt))] =
-                uint32_t(c * CT_H + lane) | ((info[j] & 3u) << 12) | (((info[j] >> 2) & 63u) << 14) | (((info[j] >> 8) & 63u) << 20);
+        const uint32_t cl = info >> (2 * j) & 3u;
+        if (cl)
+            s_list[s_pre[c] + uint32_t(__popcll((s_mask[0][c] | s_mask[1][c]) & lt))] = uint16_t(uint32_t(c * CT_H + lane) | (cl << 12));
     }
     const int nfg = int(s_pre[64]);
     __syncthreads();
@@ -1527,12 +1543,13 @@ __global__ __launch_bounds__(CT_THREADS) void ccl_tile(const T* __restrict__ x, 
     for (int e = t; e < nfg; e += CT_THREADS) {
         const uint32_t en = s_list[e];
         const int li = int(en & 0xFFFu), c = li >> 6, rr = li & 63;
-        const uint32_t cl = (en >> 12) & 3u;
-        const int rs = int((en >> 14) & 63u), re = int((en >> 20) & 63u);
+        const uint32_t cl = en >> 12;
         if (c == 0)
             continue;
+        const unsigned long long mine = s_mask[cl - 1][c], left = s_mask[cl - 1][c - 1];
+        const int rs = run_start(mine, rr), re = run_end(mine, rr);
         const uint32_t a = uint32_t(c * CT_H + rs), lb = uint32_t((c - 1) * CT_H);
-        auto lsame = [&](int r) { return r >= 0 && r < nr && s_cls[lb + r] == cl; };
+        auto lsame = [&](int r) { return r >= 0 && r < CT_H && (left >> r & 1ull); };
         if (conn4) {
             if (lsame(rr) && (rr == rs || !lsame(rr - 1)))
                 lds_union(s_par, a, lb + rr);
@@ -1549,8 +1566,8 @@ __global__ __launch_bounds__(CT_THREADS) void ccl_tile(const T* __restrict__ x, 
     // 3. roots of the run starts (a component's root, its smallest index, starts a run)
     for (int e = t; e < nfg; e += CT_THREADS) {
         const uint32_t en = s_list[e];
-        const int li = int(en & 0xFFFu);
-        if ((li & 63) == int((en >> 14) & 63u))
+        const int li = int(en & 0xFFFu), rr = li & 63;
+        if (rr == 0 || !(s_mask[(en >> 12) - 1][li >> 6] >> (rr - 1) & 1ull))
             s_par[li] = lds_find(s_par, li);
     }
     __syncthreads();
@@ -1560,7 +1577,7 @@ __global__ __launch_bounds__(CT_THREADS) void ccl_tile(const T* __restrict__ x, 
         const uint32_t en = s_list[e];
         const int li = int(en & 0xFFFu), c = li >> 6, rr = li & 63;
         const uint32_t cl = (en >> 12) & 3u;
-        const int rs = int((en >> 14) & 63u);
+        const int rs = run_start(s_mask[cl - 1][c], rr);
         const uint32_t root = s_par[c * CT_H + rs] & L_KEY;
         if (rr != rs)
             s_par[li] = root;
@@ -1612,7 +1629,7 @@ __global__ __launch_bounds__(CT_THREADS) void ccl_tile(const T* __restrict__ x, 
         const unsigned seg = seg_index(g, cv0 + lane, ty);
         rmask[seg] = s_rmp[lane];
         rmask[g.nseg + seg] = s_rmn[lane];
-        rmask[2 * size_t(g.nseg) + seg] = s_mask[lane];  // foreground of either sign (for the label map)
+        rmask[2 * size_t(g.nseg) + seg] = s_mask[0][lane] | s_mask[1][lane];  // foreground of either sign (for the label map)
     }
     const uint32_t pool_base = s_base;
     const bool ok = total <= rec.rt || size_t(pool_base) + size_t(total - rec.rt) <= size_t(rec.pool_cap);
@@ -1644,19 +1661,12 @@ __global__ __launch_bounds__(CT_THREADS) void ccl_tile(const T* __restrict__ x, 
     __syncthreads();
 
     // 5. island sums: count, extremum, moments (sourcefind.cpp:337-628)
-    double ev[CT_PPT];
-#pragma unroll
-    for (int k = 0; k < CT_PPT; k++) {
-        const int e = k * CT_THREADS + t;
-        ev[k] = 0.0;
-        if (e >= nfg)
-            continue;
+    for (int e = t; e < nfg; e += CT_THREADS) {
         const uint32_t en = s_list[e];
         const int li = int(en & 0xFFFu), c = li >> 6, rr = li & 63;
         const uint32_t cl = (en >> 12) & 3u;
         const uint32_t slot = (s_par[s_par[li] & L_KEY] >> 16) & 0xFFFu;
         const double val = ldv(x, size_t(mem_index(c, rr)));
-        ev[k] = val;
         const unsigned long long kv = okey(val);
         const double x_idx = double(cv0 + c), y_idx = double(vr0 + rr);
         const double xb = x_idx * val, yb = y_idx * val;
@@ -1690,15 +1700,11 @@ __global__ __launch_bounds__(CT_THREADS) void ccl_tile(const T* __restrict__ x, 
     }
     __syncthreads();
     // smallest memory index holding the extremum
-#pragma unroll
-    for (int k = 0; k < CT_PPT; k++) {
-        const int e = k * CT_THREADS + t;
-        if (e >= nfg)
-            continue;
+    for (int e = t; e < nfg; e += CT_THREADS) {
         const uint32_t en = s_list[e];
         const int li = int(en & 0xFFFu), c = li >> 6, rr = li & 63;
         const uint32_t slot = (s_par[s_par[li] & L_KEY] >> 16) & 0xFFFu;
-        const unsigned long long kv = okey(ev[k]);
+        const unsigned long long kv = okey(double(ldv(x, size_t(mem_index(c, rr)))));
         if (slot < uint32_t(CT_RCAP)) {
             if (kv == r_ext[slot])
                 atomicMin(&r_idx[slot], mem_index(c, rr));
@@ -1728,7 +1734,7 @@ __global__ __launch_bounds__(CT_THREADS) void ccl_tile(const T* __restrict__ x, 
         const int c = w + CT_WAVES * j;
         if (c >= nc || lane >= nr)
             continue;
-        const uint32_t cl = info[j] & 3u;
+        const uint32_t cl = info >> (2 * j) & 3u;
         const uint32_t gk = uint32_t(cv0 + c) * uint32_t(g.R) + uint32_t(rbase + lane);
         uint32_t out = P_BG;
         if (cl) {
@@ -2444,7 +2450,8 @@ void source_find_impl(stp_ctx* ctx, const T* x, int rows, int cols, const stp_so
     auto label = [&](bool clear_pool) {
         if (clear_pool)
             fill_u32(ctx, pool_count, 0u, 1);
-        launch(ctx, "ccl_tile", ccl_tile<T>, dim3(ntiles), dim3(CT_THREADS), 0, x, tg, (const SFState*)st, find_neg, conn4, P,
+        launch(ctx, "ccl_tile", ntiles <= CT_FEW ? ccl_tile<T, 1024> : ccl_tile<T, 512>, dim3(ntiles),
+            dim3(ntiles <= CT_FEW ? 1024 : 512), 0, x, tg, (const SFState*)st, find_neg, conn4, P,
             rmask, rec);
         launch(ctx, "ccl_border", ccl_border, dim3(ntiles), dim3(128), 0, P, tg, conn4);
         launch(ctx, "ccl_open_roots", ccl_open_roots, dim3(div_up(size_t(ntiles) * CT_RT + rec.pool_cap, 256)), dim3(256), 0, P,

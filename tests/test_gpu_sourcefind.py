@@ -307,3 +307,21 @@ def test_gpu_median_picks(gpu, orc, rows, cols, kind, median):
     _, _, st = orc.source_find(img, pars)
     for k in ("bg_level", "rms_est", "mean", "sigma"):
         assert getattr(res.stats, k) == getattr(st, k), k
+
+
+@pytest.mark.parametrize("rows,cols,analysis", [
+    (1024, 1024, 1.0),  # 256 tiles: the last that take 1024 threads
+    (1026, 1090, 1.0),  # more: 512 threads; tiles of 2 columns and 1 row at the edges
+    (1088, 1024, 2.0),  # about as many components as a tile sums in LDS
+    (1152, 1216, 3.0),
+])
+@pytest.mark.parametrize("conn4", [False, True])
+def test_gpu_tile_labelling(gpu, orc, rows, cols, analysis, conn4):
+    """The tile labelling with either number of threads, below, near and past the components that a
+    tile sums in LDS, with runs that span a tile's whole column."""
+    img = noise(rows, cols, seed=rows + cols)
+    img[:, 70] = 4.0 + 0.01 * np.arange(rows)
+    img[130:300, 65:67] = -5.0
+    pars = capi.sourcefind_pars(analysis + 0.5, analysis, rms_est=1.0, median_method=capi.MEDIAN_ZEROMEDIAN,
+                                ccl_4connectivity=conn4)
+    compare(gpu.source_find(img, pars, capacity=1 << 18), orc.source_find(img, pars, capacity=1 << 18))

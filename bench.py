@@ -32,11 +32,10 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0  # MI355X HBM3E, GB/s
 # LDS atomic-add rate of one MI355X, measured with every lane of 2048 workgroups of 512
-# threads adding 1024 times to random addresses of a 32 x 71 LDS array (G atomics/s),
-# by precision path: FP64 and FP32C sum with ds_add_f64 (1850 G/s); two-float with
-# ds_add_f32 / ds_add_rtn_f32 (204 G/s, returning or not: FP32 LDS atomics run at a
-# ninth of the FP64 rate on this part)
-LDS_ATOMIC_PEAK_G = {0: 1850.0, 1: 1850.0, 2: 204.0}
+# threads adding 1024 times to random addresses of a 32 x 71 LDS array (G atomics/s):
+# the two-float path's ds_add_f32 / ds_add_rtn_f32 run at 204 G/s, returning or not (FP64
+# and FP32C sum on the matrix cores, without atomics)
+LDS_ATOMIC_PEAK_G = {2: 204.0}
 METRIC = "snapshots/s + p50/p99 latency, FP32-comp vs FP64 GPU at <=1e-4 peak err"
 
 
@@ -65,22 +64,41 @@ def parse():
     return ap.parse_args()
 
 
-def kernel_bytes(name, N, rows, nvis, n_entries, nb, S):
+def occupied_tiles(uvw, N, cell, s):
+    """Share of the half-plane grid's cells in the 64 x 32 tiles that a footprint of support s
+    touches (the others are neither written by the tile sums nor read by the u pass)."""
+    scale = cell / 3600.0 * np.pi / 180.0 * N
+    u, v = np.rint(uvw[:, 0] * scale).astype(int), np.rint(uvw[:, 1] * scale).astype(int)
+    u, v = np.where(v < 0, -u, u), np.abs(v)
+    u, v = np.concatenate([u, -u[v <= s]]), np.concatenate([v, -v[v <= s]])
+    rows, occ = N // 2 + 1, np.zeros((-(-(N // 2 + 1) // 64), N // 32), dtype=bool)
+    for dv in (-s, s):
+        r = v + dv
+        for du in (-s, s):
+            ok = (r >= 0) & (r < rows)
+            occ[r[ok] // 64, (u[ok] + du) % N // 32] = True
+            occ[0, (u[(r < 0) & (v >= 0)] + du) % N // 32] = True
+    height = np.minimum(64, rows - 64 * np.arange(occ.shape[0]))
+    return float((occ * height[:, None]).sum() * 32) / (rows * N)
+
+
+def kernel_bytes(name, N, rows, nvis, n_entries, nb, S, occ=1.0):
     """Algorithmic HBM bytes per launch (S = bytes per real of the grid and image).  With a
     beam (nb = 2) the beam grid is real, stored packed in half the bytes of the vis grid, and
-    its FFT passes are launches of their own under the same names (u1, u2: the mean of the
-    vis and beam launches)."""
+    its FFT passes are launches of their own under the same names (fft_u: the mean of the
+    vis and beam launches).  occ: share of the grid that the tile sums write and the u pass
+    reads."""
     grid = rows * N * 2 * S  # one complex half-plane grid
     img = N * N * S
     grids = grid + (grid // 2 if nb == 2 else 0)
-    if name in ("fft_u1", "fft_u2"):
-        return 2 * grids // (2 if nb == 2 else 1)  # read + write every grid once, per launch
+    if name == "fft_u":
+        return int((1 + occ) * grids) // (2 if nb == 2 else 1)  # read and write every grid once, per launch
     if name == "fft_v_c2r":
         return grid + img               # read the vis grid, write the image
     if name == "fft_v_c2r_real":
         return grid // 2 + img          # read the packed beam grid, write the beam
     if name == "grid_tiles":
-        return grids + 40 * n_entries   # write every grid element once, read the binned entries
+        return int(occ * grids) + 40 * n_entries   # write the grids' occupied tiles once, read the binned entries
     if name == "grid_count":
         return 48 * nvis                # read u, v, w(unused), vis, weight
     if name == "grid_scatter":
@@ -105,7 +123,7 @@ def pmc_traffic(workload, path, kernel):
         f = line.split()
         if line.startswith("#") or len(f) < 4:
             continue
-        # the profile names the kernel function ("grid_tiles_os_kernel<float, AccF64, 8>"),
+        # the profile names the kernel function ("grid_tiles_kernel<float, 32, 0>"),
         # the library's timing names the launch ("grid_tiles")
         name = " ".join(f[:-3])
         if name == kernel or name.startswith(kernel + "_") or name.startswith(kernel + "<"):
@@ -133,6 +151,11 @@ def measure(ctx, capi, args, pars, sfp, prec, n, N, bufs, do_sf):
     # gridding entries written and good visibilities, as the gridder reports them
     diag = ctx.image_visibilities_device(pars, n, d_vis, d_w, d_uvw, d_img, d_beam, precision=prec, synchronize=True)
     n_entries = int(diag.num_grid_entries)
+    occ = 1.0
+    if prec != capi.PRECISION_FP32_TWOFLOAT and 4096 <= N <= 8192:
+        uvw = np.empty((n, 3), order="F")
+        ctx.dtoh(uvw, d_uvw)
+        occ = occupied_tiles(uvw, N, pars.cell_size, pars.kernel_support)
 
     # per-kernel breakdown: every launch bracketed by HIP events (untimed pass)
     ctx.set_timing(True)
@@ -147,7 +170,7 @@ def measure(ctx, capi, args, pars, sfp, prec, n, N, bufs, do_sf):
         if name in ("image_visibilities", "fill"):
             continue
         avg_ms = ms / max(cnt, 1)
-        kb = kernel_bytes(name, N, rows, n, n_entries, 2, S)
+        kb = kernel_bytes(name, N, rows, n, n_entries, 2, S, occ)
         kernels[name] = {"avg_us": round(avg_ms * 1000.0, 2), "per_step": round(cnt / nb_steps, 2),
                          "GBs": (round(kb / (avg_ms * 1e-3) / 1e9, 1) if kb else None)}
     dominant = max((k for k in kernels if kernel_bytes(k, N, rows, n, n_entries, 2, S)),
@@ -171,18 +194,18 @@ def measure(ctx, capi, args, pars, sfp, prec, n, N, bufs, do_sf):
     ctx.set_timing(False)
     ctx.set_timing_filter(None)
 
-    dom_bytes = kernel_bytes(dominant, N, rows, n, n_entries, 2, S)
+    dom_bytes = kernel_bytes(dominant, N, rows, n, n_entries, 2, S, occ)
     dom_avg_s = dom_ms * 1e-3 / max(dom_cnt, 1)
     achieved = dom_bytes / dom_avg_s / 1e9
-    # LDS atomic adds of the tile kernel: 3 per tap (re, im, beam) and 49 taps per good
-    # visibility (the conjugate copies near v = 0, under 1 %, are not counted)
+    # LDS atomic adds of the two-float tile kernel: two for each of 3 sums per tap (re, im,
+    # beam) and 49 taps per good visibility (the conjugate copies near v = 0, under 1 %, are
+    # not counted)
     lds_atomics = None
-    if dominant == "grid_tiles":
-        per_launch = 3.0 * 49.0 * float(diag.num_good_vis) * (2 if prec == capi.PRECISION_FP32_TWOFLOAT else 1)
+    if dominant == "grid_tiles" and prec == capi.PRECISION_FP32_TWOFLOAT:
+        per_launch = 3.0 * 49.0 * float(diag.num_good_vis) * 2
         rate = per_launch / dom_avg_s / 1e9
         lds_atomics = {"per_launch": per_launch, "achieved_G_per_s": round(rate, 1),
-                       "op": "ds_add_rtn_f32 (hi) + ds_add_f32 (lo)" if prec == capi.PRECISION_FP32_TWOFLOAT
-                       else "ds_add_f64",
+                       "op": "ds_add_rtn_f32 (hi) + ds_add_f32 (lo)",
                        "peak_G_per_s": LDS_ATOMIC_PEAK_G.get(prec),
                        "frac": (round(rate / LDS_ATOMIC_PEAK_G[prec], 4) if LDS_ATOMIC_PEAK_G.get(prec) else None)}
     ms_per_step = 1000.0 * t_total / args.steps

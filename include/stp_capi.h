@@ -66,11 +66,11 @@ typedef enum stp_median_method {
 
 /* Arithmetic of the gridder + FFT.  FP64 is the reference's USE_FLOAT=OFF build.
  * The FP32 forms keep the uv-to-pixel index and phase math, the kernel-sum
- * normalisation and the weight total in FP64, compute the taps in FP32, store
+ * normalisation and the weight total in FP64 (the two-float taps are FP32), store
  * FP32 grids and images and run the FFT in FP32 (twiddles rounded from long
- * double).  They differ in how each grid cell's taps are summed in the LDS tile:
- *   FP32C           FP64 sums (ds_add_f64), rounded to FP32 once per cell;
- *   FP32_TWOFLOAT   two-float hi + lo sums: TwoSum on the old value returned by
+ * double).  They differ in how each grid cell's taps are summed:
+ *   FP32C           FP64 sums on the matrix cores, rounded to FP32 once per cell;
+ *   FP32_TWOFLOAT   two-float hi + lo sums in the LDS tile: TwoSum on the old value returned by
  *                   the FP32 LDS atomic, the exact rounding error added to lo.
  * Source finding on an FP32 image reads FP32 and accumulates in FP64. */
 typedef enum stp_precision {

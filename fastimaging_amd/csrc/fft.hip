@@ -19,6 +19,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "crop.h"
 #include "fft.h"
 
 namespace {
@@ -577,20 +578,19 @@ struct __attribute__((packed, aligned(sizeof(OT)))) Pair {
 template <typename OT>
 __device__ __forceinline__ void store_rows(OT* out, int n, int img, const double* inv_gcf, int ya, double va, int yb, double vb)
 {
-    const int hi = img / 2, lo = n - (img - hi);
+    const stp_hip::CropPair c = stp_hip::crop_pair(ya, yb, n, img);
     if (inv_gcf) {
-        va *= inv_gcf[ya < hi ? ya : ya - n];
-        vb *= inv_gcf[yb < hi ? yb : yb - n];
+        va *= inv_gcf[stp_hip::crop_table_at(c.ia, img)];
+        vb *= inv_gcf[stp_hip::crop_table_at(c.ib, img)];
     }
-    const int ia = ya < hi ? ya : ya >= lo ? ya - n + img : -1, ib = yb < hi ? yb : yb >= lo ? yb - n + img : -1;
-    if (ia >= 0 && ib == ia + 1) {
-        *reinterpret_cast<Pair<OT>*>(out + ia) = Pair<OT>{ OT(va), OT(vb) };
+    if (c.pair) {
+        *reinterpret_cast<Pair<OT>*>(out + c.ia) = Pair<OT>{ OT(va), OT(vb) };
         return;
     }
-    if (ia >= 0)
-        out[ia] = OT(va);
-    if (ib >= 0)
-        out[ib] = OT(vb);
+    if (c.ia >= 0)
+        out[c.ia] = OT(va);
+    if (c.ib >= 0)
+        out[c.ib] = OT(vb);
 }
 
 // V: c2r along v of length n = 2M for output column x (natural order), reading

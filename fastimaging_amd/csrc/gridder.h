@@ -91,6 +91,19 @@ void grid_batch_tiles(stp_ctx* ctx, const BatchPlan& plan);
 // sides (ks rows x (ks + 2 W_KERNEL_PAD_COLS) columns).
 constexpr int W_KERNEL_PAD_COLS = 7;
 
+// W-kernels are made in groups of planes.  A plane takes the quadrant of its image-domain
+// kernel (half of the work area a side), the quadrant transformed along one axis (npos output
+// frequencies) and along both.  A group's take at most W_GROUP_BYTES, one plane's at least:
+// without undersampling the quadrant is that of the whole grid (4 MB at N = 1024, 64 MB at
+// N = 4096) however few frequencies the kernels need.
+constexpr size_t W_GROUP_BYTES = size_t(1) << 28;
+constexpr size_t w_plane_bytes(size_t half, size_t npos) { return (half * half + half * npos + npos * npos) * 16; }
+constexpr size_t w_group_planes(size_t planes, size_t half, size_t npos)
+{
+    const size_t fit = W_GROUP_BYTES / w_plane_bytes(half, npos);
+    return fit < 1 ? 1 : (fit < planes ? fit : planes);
+}
+
 // Entries (40 bytes each) the gridder's binning reserves for n visibilities: the
 // most tiles one footprint can touch on this grid, times two passes, times n.
 size_t gridder_entry_capacity(int N, bool halfplane, int support, bool exact, int tile_cols, size_t n);

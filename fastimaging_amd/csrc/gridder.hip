@@ -2900,8 +2900,6 @@ void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const doubl
             a.analytic_gcf ? 1 : 0);
         const double* d_aa = has_table(ctx, key) ? dev_table(ctx, key, {})
                                                  : dev_table(ctx, key, img_dom_kernel(kf, size_t(workarea), false, a.analytic_gcf));
-        // planes in groups of PB, each stage one launch per group, the transformed kernels of a
-        // group at most 256 MB
         const int csw = os / 2 + 1; // offsets per axis without their mirror images
         const size_t per_plane = size_t(csw) * csw * w_slot(g.ks);
         wcache_bytes = sizeof(cplx<KT>) * per_plane * P;
@@ -2955,7 +2953,8 @@ void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const doubl
             STP_REQUIRE(arr >= 4 && (arr & (arr - 1)) == 0, "c2c size must be a power of two >= 4");
             const int half = workarea / 2, len = g.s + 1, npos = os * len;
             const size_t q2 = size_t(half) * half, t2 = size_t(half) * npos, c2 = size_t(npos) * npos;
-            const int PB = int(std::max<size_t>(1, std::min<size_t>(std::min(P, 65535), (size_t(1) << 28) / (c2 * sizeof(cplx<double>)))));
+            const int PB = int(w_group_planes(size_t(P), size_t(half), size_t(npos)));
+            // planes in groups of PB, each stage one launch per group
             cplx<double>* quad = (cplx<double>*)ws_get(ctx, "w_quad", sizeof(cplx<double>) * q2 * PB);
             cplx<double>* axis = (cplx<double>*)ws_get(ctx, "w_axis", sizeof(cplx<double>) * t2 * PB);
             cplx<double>* conv = (cplx<double>*)ws_get(ctx, "w_conv", sizeof(cplx<double>) * c2 * PB);

@@ -126,11 +126,9 @@ extern "C" uint64_t stp_job_device_bytes(const stp_job* j)
             const uint64_t ko = (s + 1) * os;
             b += P * (2 * n * 16 + 10 * n * 8 + ko * (ko + 1) / 2 * 16) + (j->w_proj.hankel_proj_slice ? 16 * n : 8 * n * n);
         } else {
-            // quadrant, half-transformed and transformed arrays of one group of planes (the
-            // transformed ones at most 256 MB), and the twiddle table
+            // the arrays of one group of planes, and the twiddle table
             const uint64_t half = workarea / 2, npos = os * (s + 1);
-            const uint64_t PB = std::max<uint64_t>(1, std::min<uint64_t>(P, (uint64_t(1) << 28) / (npos * npos * 16)));
-            b += PB * (half * half + half * npos + npos * npos) * 16 + 24 * arr;
+            b += stp_hip::w_group_planes(P, half, npos) * stp_hip::w_plane_bytes(half, npos) + 24 * arr;
         }
         b += 4 * P;
     }

@@ -211,6 +211,7 @@ def test_gpu_wproj_large_kernel_cache(gpu):
     (128, 8, 15, 0, 0.0, 2),   # work area of the whole grid
     (128, 8, 15, 1, 2.0, 3),   # truncated
     (256, 8, 40, 1, 0.0, 2),   # a workgroup's rows in two passes
+    (1024, 1, 3, 0, 0.0, 70),  # planes in two groups, the quadrants being those of the whole grid
 ])
 def test_gpu_wproj_kernel_shapes(gpu, orc, N, os_, support, us, trunc, planes):
     """The W-kernels' cosine transforms and cuts over oversampling, support and work area."""

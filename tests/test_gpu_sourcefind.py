@@ -325,3 +325,28 @@ def test_gpu_tile_labelling(gpu, orc, rows, cols, analysis, conn4):
     pars = capi.sourcefind_pars(analysis + 0.5, analysis, rms_est=1.0, median_method=capi.MEDIAN_ZEROMEDIAN,
                                 ccl_4connectivity=conn4)
     compare(gpu.source_find(img, pars, capacity=1 << 18), orc.source_find(img, pars, capacity=1 << 18))
+
+
+@pytest.mark.parametrize("rows,cols,iters,steps", [
+    (5792, 5792, 5, 0),  # the largest image whose clipping passes take the steps themselves
+    (5794, 5796, 1, 0),  # past it: a launch between two passes
+    (5794, 5796, 2, 1),
+    (5794, 5796, 5, 4),
+])
+def test_gpu_clip_steps(gpu, orc, rows, cols, iters, steps):
+    """Sigma clipping on both sides of the image size from which a step is taken by one workgroup
+    instead of by every one of the next pass: bit for bit the oracle's RMS."""
+    img = np.asfortranarray(np.random.default_rng(rows + iters).standard_normal((cols, rows)).T)
+    img[::97, ::89] *= 20.0
+    pars = capi.sourcefind_pars(120.0, 110.0, sigma_clip_iters=iters, median_method=capi.MEDIAN_BINAPPROX)
+    gpu.set_timing(True)
+    try:
+        gpu.reset_timings()
+        res = gpu.source_find(img, pars)
+        launches = {k: v[1] for k, v in gpu.timings().items()}
+    finally:
+        gpu.set_timing(False)
+    _, _, st = orc.source_find(img, pars)
+    for k in ("bg_level", "rms_est", "mean", "sigma"):
+        assert getattr(res.stats, k) == getattr(st, k), k
+    assert launches.get("sf_clip_next", 0) == iters - 1 and launches.get("sf_clip_step", 0) == steps

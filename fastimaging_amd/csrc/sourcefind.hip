@@ -1173,18 +1173,18 @@ __device__ __forceinline__ ClipState clip_after(const SFState* st, int pass, uns
 constexpr size_t CLIP_SELF = 8192;
 
 // Clipping passes after the first (pass: 2, 3, ...): one wave per canonical block, reading
-// the kept candidates while the bound allows it.  fin: every workgroup first takes the step
+// the kept candidates while the bound allows it.  SELF: every workgroup first takes the step
 // of the pass before from its partials (a kernel of one workgroup between the passes took
 // 4.5 us of 13 each); workgroup 0 stores the state.  The partials and the state
 // alternate between two buffers, since the other workgroups still read the last ones.
-// fin NULL: the step is taken (sf_clip_step).
-template <typename T>
+// Without SELF the step is taken (sf_clip_step).
+template <typename T, bool SELF>
 __global__ __launch_bounds__(CU_THREADS) void sf_clip_next_kernel(const T* x, size_t n, size_t nblk, SFState* st, int pass,
     int iters, double num_sigma, const double* fin, unsigned m, const uint32_t* removed_in, double* part, uint32_t* removed,
     T* cand, uint32_t* ltab)
 {
     __shared__ ClipState cs;
-    if (fin) {
+    if constexpr (SELF) {
         double a, b;
         unsigned long long rem;
         clip_totals(fin, m, removed_in, int(nblk), a, b, rem);
@@ -2438,9 +2438,9 @@ void source_find_impl(stp_ctx* ctx, const T* x, int rows, int cols, const stp_so
                     if (!self)
                         launch(ctx, "sf_clip_step", sf_clip_step, dim3(1), dim3(CU_THREADS), 0, st, pass - 1, fin, unsigned(mfin),
                             before, int(nblk), (unsigned long long)n, iters, 3.0);
-                    launch(ctx, "sf_clip_next", sf_clip_next_kernel<T>, dim3(div_up(nblk, CU_THREADS / 64)), dim3(CU_THREADS), 0,
-                        x, n, nblk, st, pass, iters, 3.0, self ? fin : (const double*)nullptr, unsigned(mfin), before, cp, rm, cand,
-                        ltab);
+                    launch(ctx, "sf_clip_next", self ? sf_clip_next_kernel<T, true> : sf_clip_next_kernel<T, false>,
+                        dim3(div_up(nblk, CU_THREADS / 64)), dim3(CU_THREADS), 0, x, n, nblk, st, pass, iters, 3.0, fin,
+                        unsigned(mfin), before, cp, rm, cand, ltab);
                 }
                 fin = canon_reduce_to_block(ctx, cp, nblk, cscr + (pass & 1) * canon_scratch_doubles(nblk), &mfin);
             }

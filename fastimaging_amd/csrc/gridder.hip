@@ -988,8 +988,9 @@ __device__ __forceinline__ void tiles_mfma_body(const GridGeom& g, Entry* entrie
             fetch(e0 + uint32_t(batch));
             const double a = vr * w, b = vi * w;
             // the products multiply zeros outside the footprint: entries that are not
-            // finite are added tap by tap instead, so they touch their own taps only
-            const bool odd = !(fmax(fmax(fabs(a), fabs(b)), fabs(w)) < 1.0e290) || vr != vr || vi != vi || w != w;
+            // finite (among them an infinite visibility of weight 0, whose product is not) are
+            // added tap by tap instead, so they touch their own taps only
+            const bool odd = !(fabs(a) < 1.0e290 && fabs(b) < 1.0e290 && fabs(w) < 1.0e290);
             // the footprint and its wrapped pieces that overlap the tile: raw rows at +N (rows
             // past N wrap) and, for exact kernels, -N; raw columns at +-N.  One piece a round:
             // a second one exists only on grids hardly wider than the tile.

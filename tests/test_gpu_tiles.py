@@ -64,6 +64,29 @@ def test_gpu_tile_values_not_finite(gpu, exact, bad):
     assert np.isfinite(got[foot].imag).all()
 
 
+@pytest.mark.parametrize("exact", [False, True])
+@pytest.mark.parametrize("value,weight", [(np.inf, 0.0), (-np.inf, -0.0), (np.nan, 0.0), (0.0, np.inf), (1.0, np.nan)])
+def test_gpu_tile_products_not_finite(gpu, exact, value, weight):
+    """A visibility whose product with its weight is not finite reaches its own footprint only,
+    also where neither or only one of the two is finite."""
+    N, s = 128, 3
+    uv, vis, w = scene(N, 500, s, 60.0, 8)
+    uv[100] = (20.3, 30.7)
+    kw = dict(kernel_exact=exact, oversampling=8, shift_uv=False, halfplane=False, generate_beam=True)
+    run = lambda v, wt: gpu.convolve_to_grid(capi.KERNEL_GAUSSIANSINC, float(s), s, N, uv, v, wt, **kw)[:2]  # noqa: E731
+    w[100] = 0.0
+    vis[100] = 0.0
+    clean = run(vis, w)
+    vis[100], w[100] = complex(0.0, value), weight
+    foot = np.zeros((N, N), dtype=bool)
+    foot[31 + 64 - s:31 + 64 + s + 1, 20 + 64 - s:20 + 64 + s + 1] = True
+    got = run(vis, w)
+    for g, c in zip(got, clean):
+        assert np.allclose(g[~foot], c[~foot], rtol=0, atol=1e-12 * np.abs(c).max())
+    assert not np.isfinite(got[0][foot].imag).any()
+    assert np.isfinite(got[1][foot]).any() == np.isfinite(weight)
+
+
 def test_gpu_split_tiles_in_batches(gpu):
     """Fused batches split heavy tiles too: the same images as single calls."""
     ctx, items, singles, bufs = gpu, [], [], []

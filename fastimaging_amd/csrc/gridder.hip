@@ -3028,7 +3028,7 @@ void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const doubl
                         : (g.beam ? grid_wtiles_kernel<T, KT, true, false> : grid_wtiles_kernel<T, KT, false, false>);
         // truncated supports are not known here, and usually small: one phase
         int nph = 1;
-        if (bcur && !g.psup)
+        if (bcur && !(a.wproj.kernel_trunc_perc > 0.0))
             nph = int(std::max(1.0, std::min({ double(nblk), std::ceil(double(wcache_bytes) / W_PHASE_BYTES),
                 double(n) * g.ks * g.ks * sizeof(cplx<KT>) / W_PHASE_READS })));
         WPhase ph;

@@ -180,7 +180,7 @@ def test_gpu_wproj_c3_full_size(gpu, c3_case, precision, tol):
     (256, 20_000, 5, 8, 0.05, True, capi.PRECISION_FP64, TOL),    # heavy tiles, in chunks
     (256, 20_000, 5, 8, 0.05, True, capi.PRECISION_FP32C, 1e-4),
     (256, 20_000, 5, 31, 0.05, False, capi.PRECISION_FP64, TOL),
-    (512, 60_000, 9, 40, 0.8, True, capi.PRECISION_FP32C, 1e-4),  # several phases
+    (512, 60_000, 9, 40, 0.8, True, capi.PRECISION_FP32C, 1e-4),  # tiles of many planes
 ])
 def test_gpu_wproj_tile_sums(gpu, orc, N, n, planes, support, scale, beam, prec, tol):
     snap = simdata.snapshot(N, 20.0, n, 4, seed=700 + n, field_frac=0.5, w_max=300.0)
@@ -190,6 +190,34 @@ def test_gpu_wproj_tile_sums(gpu, orc, N, n, planes, support, scale, beam, prec,
     assert peak_rel_err(img, oimg) < tol
     if beam:
         assert peak_rel_err(bm, obeam) < tol
+
+
+@pytest.mark.parametrize("hankel", [False, True])
+@pytest.mark.parametrize("scale", [0.8, 0.05])  # 0.05: heavy tiles, in chunks that span phases
+def test_gpu_wproj_phases(gpu, orc, hankel, scale):
+    """Kernel caches that are read in several launches (phases), whichever way the kernels are
+    made; truncated kernels take one."""
+    n, planes, support = 80_000, 9, 60
+    snap = simdata.snapshot(512, 20.0, n, 4, seed=730, field_frac=0.5, w_max=300.0)
+    snap["uvw"][:, :2] *= scale
+    pars = capi.imager_pars(512, 20.0)
+    wp = capi.wproj_pars(planes, support, hankel_opt=hankel)
+    oimg, obeam, _, _ = orc.image_visibilities(pars, snap["vis"], snap["weights"], snap["uvw"], wproj=wp)
+
+    def run(w_proj, precision):
+        gpu.set_timing(True)
+        try:
+            gpu.reset_timings()
+            img, beam = gpu.image_visibilities(snap["vis"], snap["weights"], snap["uvw"], pars, w_proj=w_proj, precision=precision)
+            return img, beam, gpu.timings()["grid_wtiles"][1]
+        finally:
+            gpu.set_timing(False)
+
+    for precision, tol, phases in ((capi.PRECISION_FP64, TOL, 4), (capi.PRECISION_FP32C, 1e-4, 2)):
+        img, beam, launches = run(wp, precision)
+        assert peak_rel_err(img, oimg) < tol and peak_rel_err(beam, obeam) < tol
+        assert launches == phases
+    assert run(capi.wproj_pars(planes, support, hankel_opt=hankel, kernel_trunc_perc=1.0), capi.PRECISION_FP32C)[2] == 1
 
 
 def test_gpu_wproj_large_kernel_cache(gpu):

@@ -53,6 +53,8 @@ struct GridGeom {
     const uint32_t* perm = nullptr;
     const uint16_t* plane = nullptr;
     const int* psup = nullptr; // truncated support of each plane (null: s)
+    int planes = 0;            // truncated planes, where the tile sums may take phases; they do
+    double phase_taps = 0.0;   // from this many taps of one kernel of each plane, added up
 };
 
 struct Entry {
@@ -745,7 +747,7 @@ __device__ __forceinline__ void bin_scatter_body(const GridGeom& g, const double
         const Prep p = prep_in(g, in[j]);
         if (!p.good)
             continue;
-            const int sup = plane_support(g, i);
+        const int sup = plane_support(g, i);
         for (int pass = 0; pass <= p.dup; pass++) {
             const Entry e = make_entry(g, p, pass, i);
             visit_tiles(g, e.gx, e.gy, sup, [&](int ct, int rt) {
@@ -753,6 +755,23 @@ __device__ __forceinline__ void bin_scatter_body(const GridGeom& g, const double
                 if (slot < cap)
                     entries[slot] = e;
             });
+        }
+    }
+    if (bid == 0 && g.planes > 0) {
+        // tile_off[ntiles + 1]: the W tile sums in one phase
+        double taps = 0.0;
+        for (int p = threadIdx.x; p < g.planes; p += BWG)
+            taps += double(2 * g.psup[p] + 1) * double(2 * g.psup[p] + 1);
+        for (int off = 32; off >= 1; off >>= 1)
+            taps += __shfl_xor(taps, off, 64);
+        __shared__ double tsum[BWG / 64];
+        if ((threadIdx.x & 63) == 0)
+            tsum[threadIdx.x >> 6] = taps;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            for (int k = 1; k < BWG / 64; k++)
+                taps += tsum[k];
+            tile_off[ntiles + 1] = taps < g.phase_taps ? 1u : 0u;
         }
     }
     if (bid == 0 && ext_host > 0) {
@@ -2285,6 +2304,12 @@ constexpr uint32_t W_OOB = 0xc0000000u;  // buffer offset past every kernel
 constexpr size_t W_BUFFER_MAX = size_t(1) << 31; // largest kernel cache of the 32-bit buffer offsets
 constexpr double W_PHASE_BYTES = 4.5 * (1 << 20); // 32 planes, 65 taps, FP32: 9.7 ms in one launch, 7.6 at 9 MB, 7.2 at 4.5 MB
 constexpr double W_PHASE_READS = 4e9;    // least kernel bytes read per phase: below, its own 50-100 us cost more
+// With truncated kernels the host counts the reads of the whole ones, and the device takes
+// one phase where the planes' own come to less than two phases' worth (WPhase::one); the
+// other phases then cost 5 us each for nothing.  N = 4096, 2 M visibilities, 32 planes, FP64,
+// truncated at 0.01 % (whole supports remain): 22.2 ms in one phase, 11.6 in eight; at 1 % 1.65
+// and 1.68 ms.  Below 32 GB of reads one phase loses less than 1.5 ms.
+constexpr double W_TRUNC_PHASE_READS = 16e9;
 constexpr int BUF_DWORD3 = 0x00020000;   // raw (untyped) buffer access
 static_assert(W_COLS - 1 <= WPAD, "column runs must stay within the zero padding");
 
@@ -2293,6 +2318,7 @@ struct WPhase {
     const uint32_t* btot = nullptr; // entries of tile t
     int b0 = 0, b1 = 0, nblk = 0;
     int first = 1, last = 1;        // first: sums start at zero; last: write the grids
+    const uint32_t* one = nullptr;  // not 0: the first phase takes all blocks after all (null: no)
     cplx<double>* acc_v = nullptr;  // FP64 running sums between phases (rows x N, grid layout)
     cplx<double>* acc_b = nullptr;
 };
@@ -2350,6 +2376,12 @@ __global__ __launch_bounds__(64 * W_WAVES) void grid_wtiles_kernel(GridGeom g, E
     uint32_t chunk = 0;
     const int unit = int(blockIdx.x) / strips;
     int t = unit - ext_host;
+    if (ph.one && *ph.one) {
+        if (!ph.first)
+            return;
+        ph.b1 = ph.nblk;
+        ph.last = 1;
+    }
     if (t < 0) {
         if (!sp.hdr || uint32_t(unit) >= sp.hdr[0])
             return;
@@ -2980,6 +3012,19 @@ void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const doubl
         }
     }
 
+    int nph = 1; // W-projection: phases of the tile sums
+    if (wproj && ntiles <= MAX_LDS_TILES) {
+        const bool trunc = a.wproj.kernel_trunc_perc > 0.0;
+        const double tap_bytes = sizeof(cplx<KT>);
+        nph = int(std::max(1.0, std::min({ double(nblk), std::ceil(double(wcache_bytes) / W_PHASE_BYTES),
+            double(n) * g.ks * g.ks * tap_bytes / (trunc ? W_TRUNC_PHASE_READS : W_PHASE_READS) })));
+        if (trunc && nph > 1) {
+            // two phases' reads and one phase's bytes for the planes' own supports
+            const int csw = os / 2 + 1;
+            g.planes = int(a.wproj.num_wplanes);
+            g.phase_taps = std::max(2.0 * W_PHASE_READS / (double(n) * tap_bytes) * g.planes, W_PHASE_BYTES / (tap_bytes * csw * csw));
+        }
+    }
     int ext_host = 0; // extra workgroups for split tiles
     const uint32_t* offsets;
     int ostride;
@@ -2989,7 +3034,7 @@ void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const doubl
         const size_t m = size_t(ntiles) * nblk;
         uint32_t* counts = (uint32_t*)ws_get(ctx, "grid_bcounts", sizeof(uint32_t) * m);
         uint32_t* totals = (uint32_t*)ws_get(ctx, "grid_btotals", sizeof(uint32_t) * ntiles);
-        uint32_t* toffs = (uint32_t*)ws_get(ctx, "grid_boffsets", sizeof(uint32_t) * (ntiles + 1));
+        uint32_t* toffs = (uint32_t*)ws_get(ctx, "grid_boffsets", sizeof(uint32_t) * (ntiles + 2));
         const size_t hist_bytes = sizeof(uint32_t) * size_t(ntiles);
         HIP_CHECK(hipFuncSetAttribute((const void*)grid_bin_count_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, int(hist_bytes)));
         HIP_CHECK(hipFuncSetAttribute((const void*)grid_bin_scatter_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, int(hist_bytes)));
@@ -3026,13 +3071,9 @@ void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const doubl
         const int wv = std::min(W_WAVES, g.tc / W_COLS);
         auto kern = big ? (g.beam ? grid_wtiles_kernel<T, KT, true, true> : grid_wtiles_kernel<T, KT, false, true>)
                         : (g.beam ? grid_wtiles_kernel<T, KT, true, false> : grid_wtiles_kernel<T, KT, false, false>);
-        // truncated supports are not known here, and usually small: one phase
-        int nph = 1;
-        if (bcur && !(a.wproj.kernel_trunc_perc > 0.0))
-            nph = int(std::max(1.0, std::min({ double(nblk), std::ceil(double(wcache_bytes) / W_PHASE_BYTES),
-                double(n) * g.ks * g.ks * sizeof(cplx<KT>) / W_PHASE_READS })));
         WPhase ph;
         if (nph > 1) {
+            ph.one = g.planes > 0 ? offsets + ntiles + 1 : nullptr;
             ph.bcur = bcur;
             ph.btot = btot;
             ph.nblk = int(nblk);

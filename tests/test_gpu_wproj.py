@@ -217,7 +217,30 @@ def test_gpu_wproj_phases(gpu, orc, hankel, scale):
         img, beam, launches = run(wp, precision)
         assert peak_rel_err(img, oimg) < tol and peak_rel_err(beam, obeam) < tol
         assert launches == phases
-    assert run(capi.wproj_pars(planes, support, hankel_opt=hankel, kernel_trunc_perc=1.0), capi.PRECISION_FP32C)[2] == 1
+
+
+@pytest.mark.parametrize("precision,n,hankel,tol", [
+    (capi.PRECISION_FP64, 150_000, False, TOL),
+    (capi.PRECISION_FP64, 150_000, True, TOL),
+    (capi.PRECISION_FP32C, 280_000, False, 1e-4),
+])
+@pytest.mark.parametrize("perc", [1e-6, 20.0])  # whole supports remain; small ones: the first launch takes everything
+def test_gpu_wproj_truncated_phases(gpu, orc, precision, n, hankel, tol, perc):
+    """Truncated kernels in phases: the host launches those of the whole supports, and the device
+    takes them or not by the supports that remain."""
+    snap = simdata.snapshot(512, 20.0, n, 4, seed=731, field_frac=0.5, w_max=300.0)
+    pars = capi.imager_pars(512, 20.0)
+    wp = capi.wproj_pars(9, 60, hankel_opt=hankel, kernel_trunc_perc=perc)
+    oimg, obeam, _, _ = orc.image_visibilities(pars, snap["vis"], snap["weights"], snap["uvw"], wproj=wp)
+    gpu.set_timing(True)
+    try:
+        gpu.reset_timings()
+        img, beam = gpu.image_visibilities(snap["vis"], snap["weights"], snap["uvw"], pars, w_proj=wp, precision=precision)
+        launches = gpu.timings()["grid_wtiles"][1]
+    finally:
+        gpu.set_timing(False)
+    assert peak_rel_err(img, oimg) < tol and peak_rel_err(beam, obeam) < tol
+    assert launches == 2
 
 
 def test_gpu_wproj_large_kernel_cache(gpu):

@@ -915,6 +915,9 @@ __device__ __forceinline__ void tiles_mfma_body(const GridGeom& g, Entry* entrie
     }
     const int rt = t % g.tiles_r, ct = t / g.tiles_r;
     const int r0 = rt * TILE_R, c0 = ct * TC;
+    // the tile's rows and columns on the grid (pieces of a footprint past them are not stored:
+    // with a 32-column tile on a 16 x 16 grid most entries had one)
+    const int nr = min(TILE_R, g.rows - r0), nc = min(TC, N - c0);
     const int wave = __builtin_amdgcn_readfirstlane(int(threadIdx.x >> 6)), lane = threadIdx.x & 63;
     const int pitch = FORM == KERNEL_PADDED ? ks + 2 * KPAD : ks;
     double* kt = dyn;
@@ -1018,9 +1021,9 @@ __device__ __forceinline__ void tiles_mfma_body(const GridGeom& g, Entry* entrie
             if (valid && lead) {
                 uint32_t rp = 0, cpz = 0;
                 auto meets = [&](int o, int len) { return o < ks && o > -len; };
-                rp = (meets(iraw, TILE_R) ? 1u : 0u) | (meets(iraw + N, TILE_R) ? 2u : 0u) |
-                    (FORM == KERNEL_EXACT && meets(iraw - N, TILE_R) ? 4u : 0u);
-                cpz = (meets(jraw, TC) ? 1u : 0u) | (meets(jraw + N, TC) ? 2u : 0u) | (meets(jraw - N, TC) ? 4u : 0u);
+                rp = (meets(iraw, nr) ? 1u : 0u) | (meets(iraw + N, nr) ? 2u : 0u) |
+                    (FORM == KERNEL_EXACT && meets(iraw - N, nr) ? 4u : 0u);
+                cpz = (meets(jraw, nc) ? 1u : 0u) | (meets(jraw + N, nc) ? 2u : 0u) | (meets(jraw - N, nc) ? 4u : 0u);
                 pieces = ((rp & 1u) ? cpz : 0u) | ((rp & 2u) ? cpz << 3 : 0u) | ((rp & 4u) ? cpz << 6 : 0u);
             }
             bool more;

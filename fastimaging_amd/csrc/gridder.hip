@@ -895,18 +895,24 @@ __device__ __forceinline__ void tiles_mfma_body(const GridGeom& g, Entry* entrie
     const int ks = g.ks, s = g.s, N = g.N;
     const int cs = (g.os / 2) * 2 + 1;
     const int ntiles = g.tiles_r * g.tiles_c;
-    const Split sp = split_view(entries, cap, offsets[ntiles], ext_host, TC, 3);
+    Split sp{ nullptr, nullptr, nullptr, nullptr, 0 };
     uint32_t chunk = 0;
     int t = bid - ext_host;
     if (t < 0) {
         // an extra chunk of a split tile
+        sp = split_view(entries, cap, offsets[ntiles], ext_host, TC, 3);
         if (!sp.hdr || uint32_t(bid) >= sp.hdr[0])
             return;
         t = int(sp.ext[2 * bid]);
         chunk = sp.ext[2 * bid + 1];
     }
     uint32_t eb = min(offsets[t], cap), ee = min(offsets[t + 1], cap);
-    const uint32_t ch = sp.hdr ? sp.hdr[2] : 0xffffffffu;
+    uint32_t ch = 0xffffffffu;
+    if (ee - eb > SPLIT_MIN) { // light tiles do not wait for the plan
+        if (bid >= ext_host)
+            sp = split_view(entries, cap, offsets[ntiles], ext_host, TC, 3);
+        ch = sp.hdr ? sp.hdr[2] : ch;
+    }
     const bool split = ee - eb > ch;
     if (split) {
         const uint32_t e0 = eb + chunk * ch;
@@ -940,15 +946,6 @@ __device__ __forceinline__ void tiles_mfma_body(const GridGeom& g, Entry* entrie
     };
 
     if (eb < ee) {
-        if constexpr (FORM == KERNEL_PADDED) {
-            for (int k = threadIdx.x; k < cs * pitch; k += NTH) {
-                const int c = k / pitch, i = k - c * pitch - KPAD;
-                kt[k] = unsigned(i) < unsigned(ks) ? ktab[c * ks + i] : 0.0;
-            }
-        } else if constexpr (FORM == KERNEL_TABLE) {
-            for (int k = threadIdx.x; k < cs * ks; k += NTH)
-                kt[k] = ktab[k];
-        }
         if (threadIdx.x < NB)
             qcnt[threadIdx.x] = 0;
         if (threadIdx.x < 2)
@@ -971,6 +968,15 @@ __device__ __forceinline__ void tiles_mfma_body(const GridGeom& g, Entry* entrie
             nw = p->w;
         };
         fetch(eb);
+        if constexpr (FORM == KERNEL_PADDED) {
+            for (int k = threadIdx.x; k < cs * pitch; k += NTH) {
+                const int c = k / pitch, i = k - c * pitch - KPAD;
+                kt[k] = unsigned(i) < unsigned(ks) ? ktab[c * ks + i] : 0.0;
+            }
+        } else if constexpr (FORM == KERNEL_TABLE) {
+            for (int k = threadIdx.x; k < cs * ks; k += NTH)
+                kt[k] = ktab[k];
+        }
         __syncthreads();
         int round = 0;
         for (uint32_t e0 = eb; e0 < ee; e0 += uint32_t(batch)) {

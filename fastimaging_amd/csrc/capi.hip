@@ -320,11 +320,15 @@ struct FusedChunk {
 
 // Fused items in chunks on two streams: every chunk's binning, then every chunk's
 // tile sums, in turn on the first stream, and each chunk's FFTs on the second once
-// its tile sums are done, so the tile sums of chunk c (LDS-bound) overlap the FFTs
-// of chunk c-1 (HBM-bound), while the binning, whose 1024-thread workgroups wait
+// its tile sums are done, so the tile sums of chunk c overlap the FFTs
+// of chunk c-1, while the binning, whose 1024-thread workgroups wait
 // long for whole CUs beside other kernels, runs alone.  (Two streams, not three:
 // the device's few hardware queues may put a third on the queue of one of them.)
-// events[c] marks the end of chunk c's tile sums.
+// events[c] marks the end of chunk c's tile sums.  Two chunks: beside the u pass, whose
+// workgroups take half a CU each, either kernel runs longer (12 FP32 snapshots: tile sums
+// 346 -> 546 us, u pass 575 -> 830), and every chunk has its launches.  With four chunks from
+// eight snapshots on, 12 of 2048 and 4096 pixels took 1632 us at 10-20 k visibilities each
+// (now 1500) and 1930 at 20 k-2 M (1785), 64 of 1024 1338 (1275), 32 of 512 549 (387).
 template <typename T, typename OT>
 void run_fused_chunks(stp_ctx* ctx, const stp_batch_item* items, const std::vector<std::vector<size_t>>& part,
     const stp_kernel_spec* kspec, int precision, double* totals, const hipStream_t* streams, const hipEvent_t* events,
@@ -1085,7 +1089,7 @@ stp_status stp_image_batch(stp_ctx* ctx, size_t n_items, const stp_batch_item* i
             if (fused.empty())
                 return;
             // chunks of about equal work (visibilities, and grid cells for the FFT)
-            const int P = fused.size() >= 8 ? 4 : (fused.size() >= 4 ? 2 : 1);
+            const int P = fused.size() >= 4 ? 2 : 1;
             std::vector<std::vector<size_t>> part(P);
             auto cost = [&](size_t i) {
                 const double N = double(items[i].img_pars.padded_image_size);

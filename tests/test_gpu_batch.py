@@ -1,6 +1,6 @@
 """GPU tests of batches (stp_image_batch) and the autotuner: a batch of snapshots
 with uneven sizes gives the images each snapshot gives alone (FP64: within 1e-12 of
-the peak, the order of the LDS atomics being the only difference), every replay of
+the peak, the order of a tile's entries being the only difference), every replay of
 the captured hipGraph matches the eager run, and autotuned launch configurations
 keep the oracle parity."""
 import numpy as np
@@ -305,3 +305,22 @@ def test_batch_empty_tiles(gpu, precision):
                 assert peak_rel_err(c, a) <= tol and peak_rel_err(cb, ab) <= tol
     finally:
         b.free()
+
+
+@pytest.mark.parametrize("count", [3, 9])
+def test_fused_batch_launches(gpu, count):
+    """A fused batch takes each gridding stage in one launch, or two from four snapshots on, and
+    as many for the transforms of a shape."""
+    b = _Batch(gpu, [(256, 4.0, 2_000 + 100 * k, 3, 780 + k, None, 0.0) for k in range(count)], capi.PRECISION_FP32C)
+    gpu.set_timing(True)
+    try:
+        gpu.reset_timings()
+        gpu.image_batch(b.items, precision=capi.PRECISION_FP32C, flags=capi.BATCH_FUSED)
+        launches = {k: v[1] for k, v in gpu.timings().items()}
+    finally:
+        gpu.set_timing(False)
+        b.free()
+    chunks = 1 if count < 4 else 2
+    for k in ("batch_count", "batch_colscan", "batch_scatter", "batch_tiles", "batch_total", "fft_v_c2r", "fft_v_c2r_real"):
+        assert launches[k] == chunks, k
+    assert launches["fft_u"] == 2 * chunks

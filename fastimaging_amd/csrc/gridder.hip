@@ -615,8 +615,8 @@ __device__ uint32_t scan_tile_totals(const uint32_t* totals, int ntiles, uint32_
 // rest of the chip idle.  A tile of more than ch entries is summed in chunks of ch by
 // several workgroups: chunk 0 by the tile's own, chunks 1.. by extra workgroups.  Every
 // chunk of a split tile stores its FP64 sums in a slot, and merge workgroups add the
-// slots in chunk order.  ch = max(SPLIT_MIN, entries / ext_max), so at most ext_max
-// extra chunks, as many split tiles and 2 ext_max slots exist.  Below SPLIT_MIN entries
+// slots in chunk order.  ch = max(split_min, entries / ext_max), so at most ext_max
+// extra chunks, as many split tiles and 2 ext_max slots exist.  Below split_min entries
 // a tile's sums take less than a merge costs; SPLIT_EXTRA_MAX gives every CU two chunks.
 //
 // The plan and the slots lie in the unused end of the entry buffer, which is sized for
@@ -624,6 +624,19 @@ __device__ uint32_t scan_tile_totals(const uint32_t* totals, int ntiles, uint32_
 // taps; 1.2 to 1.6 are used): every kernel derives the same view from the entry count,
 // and where the end is short there are fewer chunks or none.
 constexpr uint32_t SPLIT_MIN = 1024;
+// A grid of few tiles leaves the chip idle whatever its tiles hold, and where the entries
+// crowd into a block or two, one wave sums them: smaller chunks there, but no more than a
+// heavy tile's merge can take.  3000 visibilities of a condensed array: 141 -> 91 us at 128 x
+// 128, 105 -> 82 us at 256 x 256; 100 k at 256 x 256 132 us at 1024, 141 at 256 entries.  The plan
+// costs 4 us where nothing is split, so not below SPLIT_FEW_VIS (128 x 128, 1000: 47 or 51 us).
+constexpr int SPLIT_FEW_TILES = 64;
+constexpr long long SPLIT_FEW_VIS = 2048;
+__host__ __device__ constexpr uint32_t split_min(int ntiles, long long n)
+{
+    return ntiles > SPLIT_FEW_TILES || n < SPLIT_FEW_VIS || n >= 64ll * SPLIT_MIN ? SPLIT_MIN
+        : n <= 64 * 256                                                         ? 256u
+                                                                                : uint32_t(n / 64);
+}
 constexpr uint32_t W_SPLIT_MIN = 256; // W-projection: an entry has up to 4096 taps in a tile
 constexpr size_t SPLIT_EXTRA_MAX = 512;
 constexpr size_t SPLIT_PLAN_BYTES = 16384;
@@ -636,7 +649,7 @@ struct Split {
     size_t room;       // bytes for slots
 };
 
-inline int split_extra_max(size_t n, uint32_t least = SPLIT_MIN) { return int(std::min(SPLIT_EXTRA_MAX, n / least)); }
+inline int split_extra_max(size_t n, uint32_t least) { return int(std::min(SPLIT_EXTRA_MAX, n / least)); }
 // Merge workgroups (four tile columns each).
 inline size_t merge_blocks(int ext_host, int tc) { return size_t(ext_host) * (tc / 4); }
 
@@ -778,7 +791,7 @@ __device__ __forceinline__ void bin_scatter_body(const GridGeom& g, const double
         const int chans = g.wproj ? 4 : 3;
         const Split sp = split_view(entries, cap, total, ext_host, g.tc, chans);
         if (sp.hdr)
-            split_plan(sp, totals, ntiles, total, ext_host, g.tc, chans, g.wproj ? W_SPLIT_MIN : SPLIT_MIN, wsum);
+            split_plan(sp, totals, ntiles, total, ext_host, g.tc, chans, g.wproj ? W_SPLIT_MIN : split_min(ntiles, g.n), wsum);
     }
 }
 
@@ -908,7 +921,7 @@ __device__ __forceinline__ void tiles_mfma_body(const GridGeom& g, Entry* entrie
     }
     uint32_t eb = min(offsets[t], cap), ee = min(offsets[t + 1], cap);
     uint32_t ch = 0xffffffffu;
-    if (ee - eb > SPLIT_MIN) { // light tiles do not wait for the plan
+    if (ee - eb > split_min(ntiles, g.n)) { // light tiles do not wait for the plan
         if (bid >= ext_host)
             sp = split_view(entries, cap, offsets[ntiles], ext_host, TC, 3);
         ch = sp.hdr ? sp.hdr[2] : ch;
@@ -3047,7 +3060,7 @@ void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const doubl
         const size_t hist_bytes = sizeof(uint32_t) * size_t(ntiles);
         HIP_CHECK(hipFuncSetAttribute((const void*)grid_bin_count_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, int(hist_bytes)));
         HIP_CHECK(hipFuncSetAttribute((const void*)grid_bin_scatter_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, int(hist_bytes)));
-        ext_host = wproj ? split_extra_max(n, W_SPLIT_MIN) : (mfma ? split_extra_max(n) : 0);
+        ext_host = wproj ? split_extra_max(n, W_SPLIT_MIN) : (mfma ? split_extra_max(n, split_min(int(ntiles), (long long)n)) : 0);
         launch(ctx, "grid_count", grid_bin_count_kernel, dim3(unsigned(nblk)), dim3(BWG), hist_bytes, g, d_uv, d_vis, d_w, counts,
             wpart);
         launch(ctx, "grid_colscan", bin_colscan_kernel, dim3(div_up(ntiles, 64)), dim3(1024), 0, counts, int(nblk), int(ntiles),
@@ -3198,7 +3211,7 @@ BatchPlan grid_batch_bin(stp_ctx* ctx, const std::vector<BatchGridItem>& items, 
         pool = al(pool + sizeof(double) * (2 * nblk + 2));
         p.entries = pool;
         pool = al(pool + sizeof(Entry) * cap64);
-        b.ext_host = twofloat ? 0 : split_extra_max(it.n);
+        b.ext_host = twofloat ? 0 : split_extra_max(it.n, split_min(int(ntiles), (long long)it.n));
         pre_m[k] = uint32_t(nm);
         nm += merge_blocks(b.ext_host, g.tc);
         pre_b[k] = uint32_t(nb);

@@ -43,6 +43,28 @@ def test_gpu_tile_forms(gpu, orc, N, n, s, os_, exact, halfplane, radius):
     assert abs(total - ototal) <= 1e-13 * ototal
 
 
+@pytest.mark.parametrize("N,n,radius", [
+    (128, 2_047, 8.0),    # too few to split, all in one tile
+    (128, 2_048, 8.0),    # chunks of 256
+    (256, 16_385, 8.0),   # one more than chunks of 256 take
+    (256, 65_535, 40.0),  # almost the full chunk
+    (256, 65_536, 40.0),
+    (512, 3_000, 8.0),    # more tiles: full chunks
+    (64, 4_000, 30.0),    # no room for slots beside the entries
+])
+@pytest.mark.parametrize("exact", [False, True])
+def test_gpu_tile_chunks(gpu, orc, N, n, radius, exact):
+    """Heavy tiles of grids of few tiles: on both sides of each line of the chunk size."""
+    uv, vis, w = scene(N, n, 3, radius, N + n)
+    args = (capi.KERNEL_GAUSSIANSINC, 3.0, 3, N, uv, vis, w)
+    kw = dict(kernel_exact=exact, oversampling=8, shift_uv=True, halfplane=True, generate_beam=True)
+    vg, sg, total = gpu.convolve_to_grid(*args, **kw)
+    ovg, osg, ototal, _ = orc.convolve_to_grid(*args, **kw)
+    assert peak_rel_err(vg, ovg) < 1e-12
+    assert peak_rel_err(sg, osg) < 1e-12
+    assert abs(total - ototal) <= 1e-13 * ototal
+
+
 @pytest.mark.parametrize("exact", [False, True])
 @pytest.mark.parametrize("bad", [np.nan, np.inf])
 def test_gpu_tile_values_not_finite(gpu, exact, bad):

@@ -1183,11 +1183,12 @@ stp_status stp_image_batch(stp_ctx* ctx, size_t n_items, const stp_batch_item* i
             for (size_t i : rest) {
                 const stp_batch_item& it = items[i];
                 const stp_imager_pars& q = it.img_pars;
-                snprintf(buf, sizeof(buf), "|%u,%u,%.17g,%.17g,%d,%u,%d,%u,%d,%d,%d,%u,%u,%u,%.17g,%d,%zu,%p,%p,%p,%p,%p", q.image_size,
+                snprintf(buf, sizeof(buf), "|%u,%u,%.17g,%.17g,%d,%u,%d,%u,%d,%d,%d,%u,%u,%u,%.17g,%d,%d,%d,%d,%zu,%p,%p,%p,%p,%p", q.image_size,
                     q.padded_image_size, q.cell_size, q.padding_factor, q.kernel_function, q.kernel_support, q.kernel_exact,
                     q.oversampling, q.generate_beam, q.gridding_correction, q.analytic_gcf, it.w_proj.num_wplanes,
                     it.w_proj.max_wpconv_support, it.w_proj.undersampling_opt, it.w_proj.kernel_trunc_perc,
-                    it.w_proj.wplanes_median, it.n_vis, (const void*)it.d_vis, (const void*)it.d_vis_weights,
+                    it.w_proj.wplanes_median, it.w_proj.hankel_opt, it.w_proj.hankel_proj_slice, it.w_proj.interp_type, it.n_vis,
+                    (const void*)it.d_vis, (const void*)it.d_vis_weights,
                     (const void*)it.d_uvw_lambda, it.d_image, it.d_beam);
                 sig += buf;
             }

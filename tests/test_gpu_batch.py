@@ -155,6 +155,24 @@ def test_batch_graph_cache_is_bounded(gpu):
         b.free()
 
 
+def test_batch_graph_w_kernels(gpu):
+    """Batches that differ in how their W-kernels are made alone are different graphs."""
+    b = _Batch(gpu, [(256, 20.0, 4_000, 6, 712, capi.wproj_pars(4, 8), 300.0)], capi.PRECISION_FP64)
+    try:
+        for kw in (dict(), dict(hankel_opt=True), dict(hankel_opt=True, interp_type=2),
+                   dict(hankel_opt=True, hankel_proj_slice=True, interp_type=2)):
+            b.items[0].w_proj = capi.wproj_pars(4, 8, **kw)
+            gpu.image_batch(b.items, precision=capi.PRECISION_FP64)
+            eager = b.images()[0]
+            for rep in range(2):
+                b.clear()
+                gpu.image_batch(b.items, precision=capi.PRECISION_FP64, flags=capi.BATCH_GRAPH)
+                got = b.images()[0]
+                assert peak_rel_err(got[0], eager[0]) <= 1e-12 and peak_rel_err(got[1], eager[1]) <= 1e-12, (kw, rep)
+    finally:
+        b.free()
+
+
 def test_autotune(gpu, orc, tmp_path):
     """Autotuning picks a tile width and an FFT split per shape, records them in the
     tune file, and the tuned configuration still matches the oracle."""

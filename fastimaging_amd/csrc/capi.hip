@@ -464,8 +464,9 @@ void read_diag(stp_ctx* ctx, const stp_imager_pars* p, const double* d_total, st
 }
 
 // Largest input and output (bytes, together) of a host call that go through page-locked
-// buffers of the context: one copy each way and one wait instead of three uploads, a wait for
-// the diagnostics and two downloads through the runtime's staging.  256^2 with beam, 2000
+// buffers of the context: one upload, two downloads (the diagnostics' three words, the images)
+// and one wait instead of three uploads, a wait for the diagnostics and two downloads through
+// the runtime's staging.  256^2 with beam, 2000
 // visibilities: 159 against 194 us; 512^2 with beam, 50000: 440 against 490 us; 1024^2
 // without beam, 100000 (13 MB): 700 against 765 us.  At 16 MB of images neither wins
 // reliably (1.1 or 2.3 ms, by how the caller's buffers were allocated).
@@ -729,7 +730,7 @@ stp_status stp_image_visibilities(stp_ctx* ctx, const stp_imager_pars* p, const 
         char* d_out = (char*)ws_get(ctx, "host_out", osz * isz * 2);
         const size_t in_bytes = sizeof(double) * 6 * n, out_bytes = osz * isz * (p->generate_beam ? 2 : 1);
         if (in_bytes + out_bytes <= HOST_STAGE_MAX) {
-            // small calls: page-locked buffers, one copy each way and one wait
+            // small calls: page-locked buffers and one wait
             unsigned long long* tri = (unsigned long long*)host_stage(ctx, "host_io", 32 + in_bytes + out_bytes);
             double* h_in = (double*)(tri + 4);
             char* h_out = (char*)(h_in + 6 * n);

@@ -314,15 +314,16 @@ struct UShape {
 // the LDS a row needs.  Lanes run over the rows first, so an access to a column is NR
 // elements long; neighbouring row blocks run on the same XCD and find the rest of their
 // cache lines in its L2.  Bound by the phases of a workgroup (loads, the vector unit at a
-// third of the time, stores), which overlap little while one image's rows fit the chip at
-// once.  N=4096 half plane with its half-length beam: 72 us FP32, 130 us FP64, against 87
+// third of the time, stores), which overlap little: one image's rows fit the chip about at
+// once, and from 4096 FP64 columns a CU holds one workgroup.  N=4096 half plane with its half-length beam: 72 us FP32, 130 us FP64, against 87
 // and 166 us for two passes of the four-step split (fft_u1, fft_u2), with a launch less per
 // grid; 8192 FP32 236 us against 247 us (every tile read).  Two FP32 rows per workgroup take 338 us at 8192
 // and two FP64 rows 144 us at 4096 (shorter runs); the whole complex row in LDS would
 // leave half as many rows per CU.
 template <typename T, int N>
 struct URow {
-    // 16 elements leave a wave 64 FP32 registers (128 FP64), so two workgroups fit a CU
+    // 16 elements leave a wave 64 FP32 registers (128 FP64), so two workgroups fit a CU's
+    // registers, and up to 2048 FP64 or 4096 FP32 columns its LDS too (above: 139 KB each)
     static constexpr int EPT = N == 8192 && sizeof(T) == 4 ? 32 : 16;
     static constexpr int TPR = N / EPT;                              // threads per row
     static constexpr int NR = TPR < 16 ? 64 / TPR : (N == 8192 && sizeof(T) == 8 ? 2 : 4);

@@ -48,9 +48,8 @@ struct GridGeom {
     long long n;
     int kfunc;
     double kparam, kwg, kws;
-    // W-projection: visibility k of the pass is perm[k] (|w| order) and lies in plane[k]
+    // W-projection: the inputs are in |w| order, visibility k lies in plane[k]
     int wproj = 0;
-    const uint32_t* perm = nullptr;
     const uint16_t* plane = nullptr;
     const int* psup = nullptr; // truncated support of each plane (null: s)
     int planes = 0;            // truncated planes, where the tile sums may take phases; they do
@@ -82,13 +81,12 @@ struct VisIn {
 __device__ __forceinline__ VisIn load_vis(const GridGeom& g, const double* uv, const double* vis, const double* wts, long long k)
 {
     VisIn r;
-    const long long i = g.perm ? (long long)g.perm[k] : k;
-    r.u = uv[i];
-    r.v = uv[g.n + i];
-    r.vr = vis[2 * i];
-    r.vi = vis[2 * i + 1];
-    r.w = wts[i];
-    r.wl = g.wproj ? uv[2 * g.n + i] : 0.0;
+    r.u = uv[k];
+    r.v = uv[g.n + k];
+    r.vr = vis[2 * k];
+    r.vi = vis[2 * k + 1];
+    r.w = wts[k];
+    r.wl = g.wproj ? uv[2 * g.n + k] : 0.0;
     return r;
 }
 
@@ -2914,7 +2912,6 @@ void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const doubl
             d_uv = uvw_s;
             d_vis = vis_s;
             d_w = wts_s;
-            g.perm = nullptr;  // position k of the pass is sorted position k
         }
         // 2. planes
         uint32_t* flag = (uint32_t*)ws_get(ctx, "w_flag", sizeof(uint32_t) * n);
@@ -2938,7 +2935,7 @@ void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const doubl
             (long long)n, plane_of);
         g.plane = plane_of;
         g.wproj = 1;
-        // 3. W-kernels: workarea (gridder.h:467-486), image-domain AA kernel, one FFT per plane
+        // 3. W-kernels: workarea (gridder.h:467-486), image-domain AA kernel, cosine sums per plane
         const int us = a.wproj.undersampling_opt > 0 ? (1 << (a.wproj.undersampling_opt - 1)) : 0;
         int workarea = 2;
         if (us > 0)
@@ -3005,7 +3002,7 @@ void grid_visibilities(stp_ctx* ctx, const GridderArgs& a, size_t n, const doubl
             launch(ctx, "w_kernel_extract", wk_hankel_extract_kernel<KT>, dim3(unsigned(csw * csw), unsigned(P)), dim3(256), 0,
                 h, (const cplx<double>*)kh, (const int*)psup, 0, wcache);
         } else {
-            STP_REQUIRE(arr >= 4 && (arr & (arr - 1)) == 0, "c2c size must be a power of two >= 4");
+            STP_REQUIRE(arr >= 4 && (arr & (arr - 1)) == 0, "W-kernel work array (workarea * oversampling) must be a power of two >= 4");
             const int half = workarea / 2, len = g.s + 1, npos = os * len;
             const size_t q2 = size_t(half) * half, t2 = size_t(half) * npos, c2 = size_t(npos) * npos;
             const int PB = int(w_group_planes(size_t(P), size_t(half), size_t(npos)));

@@ -641,7 +641,7 @@ def main():
         "config": {"workload": f"{args.workload}: N={N}, cell {wl['cell_arcsec']}\", {n} vis, "
                                f"{wl['n_sources']} sources, GaussianSinc s3 os9, beam, "
                                + ("source find 5/3 sigma BINMEDIAN 8-conn" if do_sf else "imaging only")
-                               + {"fp32c": ", FP32 taps with FP64 tile sums, FP32 grids and FFT",
+                               + {"fp32c": ", FP64 taps and tile sums, FP32 grids and FFT",
                                   "fp32tf": ", FP32 taps with two-float tile sums, FP32 grids and FFT",
                                   "fp64": ", FP64"}[head_name],
                    "image_size": N, "n_vis": n, "path": head_name},

@@ -1788,7 +1788,11 @@ __global__ __launch_bounds__(64) void wplane_bounds_kernel(const uint32_t* G, lo
     unsigned long long begin = 0;
     auto wv = [&](unsigned long long k) { return __longlong_as_double((long long)skey[k]); };
     for (int p = 0; p < P; p++) {
-        const unsigned long long plane_size = (unsigned long long)ceil(double(num_gvis - begin) / double(P - p));
+        // with many rejected visibilities the position `begin` passes the good count and the
+        // unsigned difference wraps (the reference's own arithmetic): a size past 64 bits, which
+        // only the last plane can have, is none, as the reference's conversion gives on x86
+        const double size = ceil(double(num_gvis - begin) / double(P - p));
+        const unsigned long long plane_size = size < 18446744073709551616.0 ? (unsigned long long)size : 0ull;
         unsigned long long k = begin, counter = 0;
         if (plane_size > 0 && begin < (unsigned long long)n) {
             const unsigned long long target = (unsigned long long)G[begin] + plane_size;

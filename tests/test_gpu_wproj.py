@@ -272,6 +272,18 @@ def test_gpu_wproj_kernel_shapes(gpu, orc, N, os_, support, us, trunc, planes):
     assert peak_rel_err(img, oimg) < TOL and peak_rel_err(beam, obeam) < TOL
 
 
+@pytest.mark.parametrize("planes,median", [(1, False), (2, False), (2, True), (3, False), (5, True), (6, False)])
+@pytest.mark.parametrize("scale", [1.25, 1.6])
+def test_gpu_wproj_many_rejected(gpu, orc, planes, median, scale):
+    """Most visibilities off the grid: a plane's first position passes the number of good ones, and
+    the last plane then counts none (average_w_planes, gridder.cpp:68-146)."""
+    snap = simdata.snapshot(128, 20.0, 4_000, 4, seed=770, field_frac=0.5, w_max=400.0)
+    snap["uvw"][:, :2] *= scale
+    wp = capi.wproj_pars(planes, 8, wplanes_median=median)
+    img, beam, oimg, obeam = _wcase(gpu, orc, snap, 128, 20.0, wp)
+    assert peak_rel_err(img, oimg) < TOL and peak_rel_err(beam, obeam) < TOL
+
+
 @pytest.mark.parametrize("n", [1, 64, 4_096, 4_097, 524_288, 524_289, (1 << 20) + 1])
 def test_gpu_wproj_order(gpu, orc, n):
     """The |w| order over the sort's block sizes and ways of adding up the counts, with many ties,

@@ -1171,14 +1171,19 @@ __device__ __forceinline__ ClipState clip_after(const SFState* st, int pass, uns
 // 278 us at 4096 x 4096, 517 either way at 5792 x 5792, 1083 against 1103 us at 8192 x 8192,
 // 3549 against 3872 us at 16384 x 16384.
 constexpr size_t CLIP_SELF = 8192;
+// Canonical blocks a workgroup of a clipping pass takes: one each up to this many blocks, so that
+// the pass of a small image is spread over the CUs; above, a wave each, since the steps repeat
+// by workgroup.  Source finding at 512 x 512 FP64 177 us, 200 with 16 blocks a workgroup
+// throughout (191 with the step in a launch of its own); 1024 x 1024 FP32 170 and 178 us.
+constexpr size_t CLIP_SPREAD = 256;
 
-// Clipping passes after the first (pass: 2, 3, ...): one wave per canonical block, reading
-// the kept candidates while the bound allows it.  SELF: every workgroup first takes the step
-// of the pass before from its partials (a kernel of one workgroup between the passes took
-// 4.5 us of 13 each); workgroup 0 stores the state.  The partials and the state
+// Clipping passes after the first (pass: 2, 3, ...): one wave per canonical block, PER blocks
+// a workgroup, reading the kept candidates while the bound allows it.  SELF: every workgroup
+// first takes the step of the pass before from its partials (a kernel of one workgroup between
+// the passes took 4.5 us of 13 each); workgroup 0 stores the state.  The partials and the state
 // alternate between two buffers, since the other workgroups still read the last ones.
 // Without SELF the step is taken (sf_clip_step).
-template <typename T, bool SELF>
+template <typename T, bool SELF, int PER>
 __global__ __launch_bounds__(CU_THREADS) void sf_clip_next_kernel(const T* x, size_t n, size_t nblk, SFState* st, int pass,
     int iters, double num_sigma, const double* fin, unsigned m, const uint32_t* removed_in, double* part, uint32_t* removed,
     T* cand, uint32_t* ltab)
@@ -1197,8 +1202,8 @@ __global__ __launch_bounds__(CU_THREADS) void sf_clip_next_kernel(const T* x, si
         cs = st->clip[(pass + 1) & 1];
     }
     __syncthreads();
-    const size_t blk = size_t(blockIdx.x) * (CU_THREADS / 64) + (threadIdx.x >> 6);
-    if (cs.done || blk >= nblk)
+    const size_t blk = size_t(blockIdx.x) * PER + (threadIdx.x >> 6);
+    if (cs.done || (PER < CU_THREADS / 64 && int(threadIdx.x >> 6) >= PER) || blk >= nblk)
         return;
     const double median = st->median;
     if (cs.compact)
@@ -2435,11 +2440,14 @@ void source_find_impl(stp_ctx* ctx, const T* x, int rows, int cols, const stp_so
                 else {
                     const uint32_t* before = removed + ((pass + 1) & 1) * nblk;
                     const bool self = nblk <= CLIP_SELF;
+                    const bool spread = nblk <= CLIP_SPREAD;
+                    constexpr int ALL = CU_THREADS / 64;
                     if (!self)
                         launch(ctx, "sf_clip_step", sf_clip_step, dim3(1), dim3(CU_THREADS), 0, st, pass - 1, fin, unsigned(mfin),
                             before, int(nblk), (unsigned long long)n, iters, 3.0);
-                    launch(ctx, "sf_clip_next", self ? sf_clip_next_kernel<T, true> : sf_clip_next_kernel<T, false>,
-                        dim3(div_up(nblk, CU_THREADS / 64)), dim3(CU_THREADS), 0, x, n, nblk, st, pass, iters, 3.0, fin,
+                    launch(ctx, "sf_clip_next",
+                        spread ? sf_clip_next_kernel<T, true, 1> : (self ? sf_clip_next_kernel<T, true, ALL> : sf_clip_next_kernel<T, false, ALL>),
+                        dim3(div_up(nblk, spread ? 1 : ALL)), dim3(CU_THREADS), 0, x, n, nblk, st, pass, iters, 3.0, fin,
                         unsigned(mfin), before, cp, rm, cand, ltab);
                 }
                 fin = canon_reduce_to_block(ctx, cp, nblk, cscr + (pass & 1) * canon_scratch_doubles(nblk), &mfin);

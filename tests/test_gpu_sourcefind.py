@@ -328,14 +328,18 @@ def test_gpu_tile_labelling(gpu, orc, rows, cols, analysis, conn4):
 
 
 @pytest.mark.parametrize("rows,cols,iters,steps", [
+    (2, 2, 3, 0),
+    (1024, 1024, 5, 0),  # the largest image with a workgroup for each canonical block
+    (1024, 1026, 5, 0),
     (5792, 5792, 5, 0),  # the largest image whose clipping passes take the steps themselves
     (5794, 5796, 1, 0),  # past it: a launch between two passes
     (5794, 5796, 2, 1),
     (5794, 5796, 5, 4),
 ])
 def test_gpu_clip_steps(gpu, orc, rows, cols, iters, steps):
-    """Sigma clipping on both sides of the image size from which a step is taken by one workgroup
-    instead of by every one of the next pass: bit for bit the oracle's RMS."""
+    """Sigma clipping on both sides of the image sizes from which a workgroup takes several canonical
+    blocks, and a step is taken by one workgroup instead of by every one of the next pass: bit
+    for bit the oracle's RMS."""
     img = np.asfortranarray(np.random.default_rng(rows + iters).standard_normal((cols, rows)).T)
     img[::97, ::89] *= 20.0
     pars = capi.sourcefind_pars(120.0, 110.0, sigma_clip_iters=iters, median_method=capi.MEDIAN_BINAPPROX)
